@@ -142,6 +142,12 @@ public:
     [[nodiscard]] T* get() const { return p_; }
     [[nodiscard]] std::size_t size() const { return n_; }
     T& operator[](std::size_t i) const { return p_[i]; }
+    // The buffer's address on the device.
+    [[nodiscard]] T* device() const {
+        void* d = nullptr;
+        hip_check(hipHostGetDevicePointer(&d, p_, 0), "hipHostGetDevicePointer");
+        return static_cast<T*>(d);
+    }
 
 private:
     T* p_ = nullptr;

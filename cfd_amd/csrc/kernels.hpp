@@ -1662,19 +1662,40 @@ __device__ __forceinline__ void finalize_step(const SysDev& S) {
     }
 }
 
-// One workgroup per system (ids: descriptor indices). With status_out, the system's status
-// after the step is also stored at status_out[id]: the last step of an iteration reports every
-// system's state to host-mapped memory this way, with no launch of its own.
+// A system's progress as one 64-bit word, so that a host that polls it never sees half a report:
+// the residual (FP32 bits) above, the number of finished iterations and the status below. The word
+// goes to host-mapped memory at the end of every iteration; the host reads it while later
+// iterations are queued, without an event (an event record between two graph launches costs 4 us).
+__device__ __forceinline__ unsigned long long report_word(const SolveState* st, int done) {
+    const unsigned low = (static_cast<unsigned>(done) << k_report_status_bits) | static_cast<unsigned>(st->status);
+    return (static_cast<unsigned long long>(__float_as_uint(static_cast<float>(st->res))) << 32) | low;
+}
+
+// Iterations finished when the step Op has run (st->it is already the next one after a residual
+// step that goes on, except in AMG-PCG, whose beta step counts).
+template <int Op>
+__device__ __forceinline__ int iterations_done(const SolveState* st) {
+    if (Op == FIN_AMG_INIT || Op == FIN_CG_INIT || Op == FIN_BICG_INIT) {
+        return 0;
+    }
+    if (Op == FIN_CG_RES_BETA || Op == FIN_BICG_RES) {
+        return st->status == ST_RUNNING ? st->it - 1 : st->it;
+    }
+    return st->it;
+}
+
+// One workgroup per system (ids: descriptor indices). With report, the system's report word after
+// the step is also stored at report[id]: the last step of an iteration tells the host every
+// system's state this way, with no launch of its own.
 template <int Op>
 __global__ void __launch_bounds__(k_fin_block) k_finalize(const SysDev* __restrict__ sys, const int* __restrict__ ids,
-                                                         int* __restrict__ status_out) {
+                                                         unsigned long long* __restrict__ report) {
     const int id = ids[blockIdx.x];
     finalize_step<Op>(sys[id]);
-    if (status_out != nullptr) {
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            status_out[id] = sys[id].st->status;
-        }
+    if (report != nullptr && threadIdx.x == 0) { // thread 0 wrote the state
+        const SolveState* st = sys[id].st;
+        __hip_atomic_store(report + id, report_word(st, iterations_done<Op>(st)), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 

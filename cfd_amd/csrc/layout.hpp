@@ -34,6 +34,11 @@ enum Status : int {
     ST_CONVERGED_PENDING = 4 // BiCGStab early exit: x += alpha ph still to apply
 };
 
+// Report word of a system's progress (report_word): status in the low bits, the number of finished
+// iterations above it, the FP32 residual in the upper half.
+constexpr int k_report_status_bits = 4;
+constexpr unsigned k_report_none = 15; // status of a word that no step has written yet
+
 struct SolveState {
     double tol;
     double rz;

@@ -1586,8 +1586,8 @@ struct SweepFactors {
     [[nodiscard]] double post(int j, int k) const { return pre[k - 1 - j]; }
 };
 
-// Iterations a runner keeps queued ahead of its convergence read-back (CFDG_QUEUE_DEPTH, 1 to
-// k_max_queue_depth; default 1).
+// How many iterations before the last queued one is reported a runner queues the next ones
+// (CFDG_QUEUE_DEPTH, 1 to k_max_queue_depth; default 1).
 constexpr int k_max_queue_depth = 7;
 
 int queue_depth() {
@@ -1727,8 +1727,8 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
 }
 
 template <int Op>
-void fin(const SysDev* d, const Tables& tb, hipStream_t s, int* status_out = nullptr) {
-    k_finalize<Op><<<tb.n_sys, k_fin_block, 0, s>>>(d, tb.ids.get(), status_out);
+void fin(const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report = nullptr) {
+    k_finalize<Op><<<tb.n_sys, k_fin_block, 0, s>>>(d, tb.ids.get(), report);
 }
 
 enum VecId { V_X = 0, V_R, V_P, V_Q, V_Z, V_R0, V_V, V_S, V_T, V_PH, V_SH };
@@ -1742,39 +1742,37 @@ struct Plan {
     SweepFactors sf = sweep_factors(1, 0.0); // all 1: plain damped Jacobi
 };
 
-void enqueue_init(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t s) {
+// The start of a solve: the initial residual and its convergence test. Its last step stores each
+// system's report word at report[id].
+void enqueue_init(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report) {
     const int g0 = tb.tn[0];
     const int2* b0 = tb.t[0].get();
     if (pl.method == CFDG_METHOD_BICGSTAB) {
         CFDG_LAUNCH(k_bicg_init<false>, g0, s, d, b0);
-        fin<FIN_BICG_INIT>(d, tb, s);
+        fin<FIN_BICG_INIT>(d, tb, s, report);
         return;
     }
     // CG start: r, z and beta = 0; p = z + 0 p_old (p_old = 0) is formed by the first
     // iteration's product (k_spmv_pz).
     if (!pl.amg) {
         CFDG_LAUNCH(k_cg_init<false>, g0, s, d, b0);
-        fin<FIN_CG_INIT>(d, tb, s);
+        fin<FIN_CG_INIT>(d, tb, s, report);
         return;
     }
     if (pl.fp32) {
         CFDG_LAUNCH(k_residual0<true>, g0, s, d, b0);
-        fin<FIN_AMG_INIT>(d, tb, s);
-        enqueue_vcycle<float, 2>(d, tb, pl.sweeps, s, !pl.bf16 && pair_sweeps(), pl.sf);
-        fin<FIN_BETA_FLEX>(d, tb, s);
     } else {
         CFDG_LAUNCH(k_residual0<false>, g0, s, d, b0);
-        fin<FIN_AMG_INIT>(d, tb, s);
-        enqueue_vcycle<double, 1>(d, tb, pl.sweeps, s, false, pl.sf);
-        fin<FIN_BETA>(d, tb, s);
     }
+    fin<FIN_AMG_INIT>(d, tb, s, report);
 }
 
-// One iteration; parity = iteration number mod 2 selects the search-direction buffers.
-// One iteration for every listed system; its last step stores each system's status at
-// status_out[id].
+// One iteration for every listed system; parity = iteration number mod 2 selects the
+// search-direction buffers. The AMG-PCG iteration begins with the V-cycle and ends with the
+// residual test, so that nothing is queued between a test that ends the solve and the report of
+// it; the last step stores each system's report word at report[id].
 void enqueue_iteration(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t s, int parity,
-                       int* status_out) {
+                       unsigned long long* report) {
     const int g0 = tb.tn[0];
     const int2* b0 = tb.t[0].get();
     if (pl.method == CFDG_METHOD_BICGSTAB) {
@@ -1787,10 +1785,17 @@ void enqueue_iteration(const Plan& pl, const SysDev* d, const Tables& tb, hipStr
         CFDG_LAUNCH((k_spmv_dot<true, false>), g0, s, d, b0, V_SH, V_T, V_T, SLOT_TT, V_S, SLOT_TS);
         fin<FIN_BICG_OMEGA>(d, tb, s);
         CFDG_LAUNCH(k_bicg_xr, g0, s, d, b0);
-        fin<FIN_BICG_RES>(d, tb, s, status_out);
+        fin<FIN_BICG_RES>(d, tb, s, report);
         return;
     }
     const int fz = final_index(pl.sweeps);
+    if (pl.amg && pl.fp32) {
+        enqueue_vcycle<float, 2>(d, tb, pl.sweeps, s, !pl.bf16 && pair_sweeps(), pl.sf);
+        fin<FIN_BETA_FLEX>(d, tb, s);
+    } else if (pl.amg) {
+        enqueue_vcycle<double, 1>(d, tb, pl.sweeps, s, false, pl.sf);
+        fin<FIN_BETA>(d, tb, s);
+    }
     probe_begin(PROBE_OUTER_SPMV, s);
     if (!pl.amg) {
         CFDG_LAUNCH((k_spmv_pz<double, false>), g0, s, d, b0, parity, 0, 0);
@@ -1803,34 +1808,84 @@ void enqueue_iteration(const Plan& pl, const SysDev* d, const Tables& tb, hipStr
     fin<FIN_ALPHA>(d, tb, s);
     if (!pl.amg) {
         CFDG_LAUNCH(k_update_xr<1>, g0, s, d, b0, parity);
-        fin<FIN_CG_RES_BETA>(d, tb, s, status_out);
+        fin<FIN_CG_RES_BETA>(d, tb, s, report);
         return;
     }
     if (pl.fp32) {
         CFDG_LAUNCH(k_update_xr<2>, g0, s, d, b0, parity);
-        fin<FIN_RES>(d, tb, s);
-        enqueue_vcycle<float, 2>(d, tb, pl.sweeps, s, !pl.bf16 && pair_sweeps(), pl.sf);
-        fin<FIN_BETA_FLEX>(d, tb, s, status_out);
     } else {
         CFDG_LAUNCH(k_update_xr<0>, g0, s, d, b0, parity);
-        fin<FIN_RES>(d, tb, s);
-        enqueue_vcycle<double, 1>(d, tb, pl.sweeps, s, false, pl.sf);
-        fin<FIN_BETA>(d, tb, s, status_out);
     }
+    fin<FIN_RES>(d, tb, s, report);
 }
+
+// A report word as the host reads it.
+struct Report {
+    int status;
+    int done;
+    float res;
+    explicit Report(unsigned long long w)
+        : status(static_cast<int>(w & ((1u << k_report_status_bits) - 1))),
+          done(static_cast<int>(static_cast<unsigned>(w) >> k_report_status_bits)) {
+        const unsigned bits = static_cast<unsigned>(w >> 32);
+        std::memcpy(&res, &bits, sizeof res);
+    }
+    [[nodiscard]] bool none() const { return status == static_cast<int>(k_report_none); }
+    [[nodiscard]] bool running() const { return none() || status == ST_RUNNING || status == ST_CONVERGED_PENDING; }
+};
+
+// Iterations a system still needs, from the residuals it has reported: the average reduction of
+// its last k_span iterations, continued to the tolerance. A surplus iteration is a row of launches
+// that do nothing, a missing one a wait of about one launch; they cost about the same, so the
+// estimate is rounded to nearest with a small bias to waiting.
+class Forecast {
+public:
+    void reset(double tol) {
+        tol_ = tol;
+        res_.clear();
+    }
+    void add(const Report& r) {
+        if (!r.none() && r.done >= static_cast<int>(res_.size())) {
+            res_.resize(static_cast<std::size_t>(r.done) + 1, r.res); // iterations the poll missed take this one's
+        }
+    }
+    // Number of the iteration at which the residual is expected to reach the tolerance.
+    [[nodiscard]] int last() const {
+        const int k = static_cast<int>(res_.size()) - 1;
+        if (k < 1) {
+            return k + k_unknown;
+        }
+        const int j = std::max(0, k - k_span);
+        const double now = res_[static_cast<std::size_t>(k)];
+        const double rate = std::log(now / static_cast<double>(res_[static_cast<std::size_t>(j)])) / (k - j);
+        const double need = std::log(tol_ / now);
+        if (!(rate < -1e-3) || !(need > -1e6)) { // stalled, growing, not finite, or no tolerance
+            return k + k_unknown;
+        }
+        return k + static_cast<int>(std::min(1000.0, std::max(1.0, std::floor(need / rate + 0.7))));
+    }
+
+private:
+    static constexpr int k_span = 3;
+    static constexpr int k_unknown = 4;
+    double tol_ = 0.0;
+    std::vector<float> res_;
+};
 
 } // namespace
 
 // Everything a set of systems needs to be solved together, built once and reused: launch
 // tables, device descriptors, and (unless kernels are being probed) HIP graphs of the solver's
-// start-up sequence and of one iteration. Iteration k of the graph pipeline writes every
-// system's status into pinned host memory slot k mod 2 from the device; the host waits for the
-// previous slot while the next iteration is already queued.
+// start-up sequence and of one, two and four iterations. Every iteration ends by writing each
+// system's report word into pinned host memory; the host polls the words and queues, one
+// iteration ahead of them, as many iterations as the residuals let it expect (Forecast): a graph
+// launch costs 8 us beyond its kernels, and an iteration queued past the end of the solve all its
+// launches.
 class Runner {
 public:
     Runner(const std::vector<System*>& systems, const BatchOptions& opt, hipStream_t s)
-        : sys_(systems), s_(s), running_(2 * systems.size()), init_host_(systems.size()),
-          out_host_(systems.size()) {
+        : sys_(systems), s_(s), report_(systems.size()), init_host_(systems.size()),
+          out_host_(systems.size()), forecast_(systems.size()) {
         require(!sys_.empty(), "solve_batch: no systems");
         const bool amg = opt.use_amg && opt.method == CFDG_METHOD_CG;
         const bool fp32 = amg && opt.precision != CFDG_PREC_FP64;
@@ -1863,17 +1918,15 @@ public:
             desc[i] = sys_[i]->descriptor(fp32, amg, bf16);
         }
         desc_.upload(desc.data(), desc.size(), s_);
-        d_init_.resize(sys_.size());
-        d_out_.resize(sys_.size());
-        void* dev = nullptr;
-        hip_check(hipHostGetDevicePointer(&dev, running_.get(), 0), "hipHostGetDevicePointer");
-        running_dev_ = static_cast<int*>(dev);
+        report_dev_ = report_.device();
+        init_dev_ = init_host_.device();
+        out_dev_ = out_host_.device();
         use_graphs_ = std::getenv("CFDG_NO_GRAPHS") == nullptr;
     }
     Runner(const Runner&) = delete;
     Runner& operator=(const Runner&) = delete;
     ~Runner() {
-        for (hipGraphExec_t g : {init_exec_, iter_exec_[0], iter_exec_[1]}) {
+        for (hipGraphExec_t g : {init_exec_, even_exec_, odd_exec_[0], odd_exec_[1], odd_exec_[2]}) {
             if (g != nullptr) {
                 (void)hipGraphExecDestroy(g);
             }
@@ -1927,53 +1980,63 @@ public:
         if (graphs && init_exec_ == nullptr) {
             capture_graphs();
         }
-        for (std::size_t i = 0; i < running_.size(); ++i) {
-            running_[i] = ST_RUNNING;
+        for (std::size_t i = 0; i < sys_.size(); ++i) {
+            report_[i] = k_report_none;
+            forecast_[i].reset(control[i].abs_tolerance);
         }
         hip_check(hipEventRecord(t0_.get(), s_), "event record");
-        hip_check(hipMemcpyAsync(d_init_.get(), init_host_.get(), sys_.size() * sizeof(SolveState),
-                                 hipMemcpyHostToDevice, s_),
-                  "H2D states");
-        k_init_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, d_init_.get());
+        k_init_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, init_dev_);
         if (graphs) {
             hip_check(hipGraphLaunch(init_exec_, s_), "graph launch");
         } else {
-            enqueue_init(pl_, d, tb_, s_);
+            enqueue_init(pl_, d, tb_, s_, report_dev_);
         }
         hip_check(hipGetLastError(), "init launch");
-        // Iterations are enqueued `depth` ahead of the convergence read-back (CFDG_QUEUE_DEPTH,
-        // 1 to 7; default 1); surplus iterations are no-ops on the device because every kernel
-        // tests the system's status first. Iteration k reports into status slot k & 1; with
-        // depth 2 or more the read after iteration j's event may see a later iteration's report
-        // in the same slot, which is only more recent (a status only ever leaves RUNNING).
-        const int depth = queue_depth();
-        for (int k = 1; k <= max_it + 1 + depth; ++k) {
-            const int slot = k & 1;
-            if (graphs) {
-                hip_check(hipGraphLaunch(iter_exec_[slot], s_), "graph launch");
-            } else {
-                enqueue_iteration(pl_, d, tb_, s_, slot, running_dev_ + slot * n_sys);
+        // One iteration past the limit: AMG-PCG finds the limit exceeded at its beginning.
+        const long long most = static_cast<long long>(max_it) + 1;
+        const int lead = graphs ? queue_depth() : queue_depth() + 1; // launches one by one take the host longer
+        long long queued = 0;
+        bool idle = false;
+        for (long long polls = 0;; ++polls) {
+            bool any = false;
+            long long known = most;
+            long long expected = 0;
+            for (std::size_t i = 0; i < sys_.size(); ++i) {
+                const Report r(__atomic_load_n(report_.get() + i, __ATOMIC_RELAXED));
+                if (r.running()) {
+                    any = true;
+                    forecast_[i].add(r);
+                    known = std::min<long long>(known, r.none() ? 0 : r.done);
+                    expected = std::max<long long>(expected, forecast_[i].last());
+                }
             }
-            hip_check(hipEventRecord(ev_[k % k_events].get(), s_), "event record");
-            hip_check(hipGetLastError(), "iteration launch");
-            if (k > depth) {
-                const int j = k - depth;
-                spin_wait(ev_[j % k_events].get(), "event sync");
-                if (!any_running(j & 1)) {
-                    break;
+            if (!any) {
+                break;
+            }
+            if (queued < most && queued - known <= lead && (queued < expected || queued == known)) {
+                queued += enqueue_iterations(graphs, queued, std::min(std::max(expected - queued, 1LL), most - queued));
+                polls = 0;
+                idle = false;
+            } else if ((polls & 0xffff) == 0xffff) {
+                if (idle) { // the words were read again after the queue had run empty
+                    if (known >= queued) {
+                        break; // every iteration allowed has been reported
+                    }
+                    hip_check(hipErrorUnknown, "solve: the device stopped reporting");
+                }
+                const hipError_t q = hipStreamQuery(s_); // a failed device never reports
+                idle = q == hipSuccess;
+                if (q != hipErrorNotReady) {
+                    hip_check(q, "solve");
                 }
             }
         }
         CFDG_LAUNCH(k_true_residual<false>, tb_.tn[0], s_, d, tb_.t[0].get());
         fin<FIN_TRUE>(d, tb_, s_);
-        k_gather_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, d_out_.get());
+        k_gather_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, out_dev_); // into pinned memory
+        hip_check(hipGetLastError(), "true residual launch");
         hip_check(hipEventRecord(t1_.get(), s_), "event record");
-        hip_check(hipMemcpyAsync(out_host_.get(), d_out_.get(), sys_.size() * sizeof(SolveState),
-                                 hipMemcpyDeviceToHost, s_),
-                  "D2H states");
-        hip_check(hipEventRecord(done_.get(), s_), "event record");
-        spin_wait(done_.get(), "solve sync");
-        hip_check(hipStreamSynchronize(s_), "solve sync");
+        spin_wait(t1_.get(), "solve sync");
         float ms = 0.0f;
         hip_check(hipEventElapsedTime(&ms, t0_.get(), t1_.get()), "event elapsed");
         stats.assign(sys_.size(), cfdg_solve_stats{});
@@ -2009,21 +2072,26 @@ public:
     }
 
 private:
-    // Statuses that iteration slot `slot` reported (host-mapped): is any system still going?
-    [[nodiscard]] bool any_running(int slot) const {
-        const std::size_t n = sys_.size();
-        for (std::size_t i = 0; i < n; ++i) {
-            const int st = running_[static_cast<std::size_t>(slot) * n + i];
-            if (st == ST_RUNNING || st == ST_CONVERGED_PENDING) {
-                return true;
-            }
+    // Queues up to `want` iterations after the `queued` ones (four, two or one with graphs, which
+    // start at an odd iteration unless they hold one); returns how many.
+    long long enqueue_iterations(bool graphs, long long queued, long long want) {
+        const bool odd = ((queued + 1) & 1) != 0;
+        if (!graphs) {
+            enqueue_iteration(pl_, desc_.get(), tb_, s_, odd ? 1 : 0, report_dev_);
+            hip_check(hipGetLastError(), "iteration launch");
+            return 1;
         }
-        return false;
+        if (!odd) {
+            hip_check(hipGraphLaunch(even_exec_, s_), "graph launch");
+            return 1;
+        }
+        const int k = want >= 4 ? 2 : want >= 2 ? 1 : 0;
+        hip_check(hipGraphLaunch(odd_exec_[k], s_), "graph launch");
+        return 1LL << k;
     }
 
     void capture_graphs() {
         const SysDev* d = desc_.get();
-        const int n_sys = static_cast<int>(sys_.size());
         auto capture = [&](auto&& enqueue) {
             hipGraph_t g = nullptr;
             hip_check(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal), "begin capture");
@@ -2034,12 +2102,16 @@ private:
             hip_check(hipGraphDestroy(g), "graph destroy");
             return e;
         };
-        init_exec_ = capture([&] { enqueue_init(pl_, d, tb_, s_); });
-        for (int slot = 0; slot < 2; ++slot) {
-            iter_exec_[slot] = capture([&] {
-                enqueue_iteration(pl_, d, tb_, s_, slot, running_dev_ + slot * n_sys);
-            });
+        auto iterations = [&](int first, int count) {
+            for (int k = first; k < first + count; ++k) {
+                enqueue_iteration(pl_, d, tb_, s_, k & 1, report_dev_);
+            }
+        };
+        for (int k = 0; k < 3; ++k) {
+            odd_exec_[k] = capture([&] { iterations(1, 1 << k); });
         }
+        even_exec_ = capture([&] { iterations(2, 1); });
+        init_exec_ = capture([&] { enqueue_init(pl_, d, tb_, s_, report_dev_); });
     }
 
 public:
@@ -2056,22 +2128,21 @@ private:
     Plan pl_{};
     Tables tb_;
     DevBuf<SysDev> desc_;
-    DevBuf<SolveState> d_init_;
-    DevBuf<SolveState> d_out_;
-    PinnedBuf<int> running_;     // per iteration slot (2) and system: status after the iteration
-    int* running_dev_ = nullptr;
+    PinnedBuf<unsigned long long> report_; // per system: report word of its latest finished step
     PinnedBuf<SolveState> init_host_;
     PinnedBuf<SolveState> out_host_;
-    static constexpr int k_events = k_max_queue_depth + 1; // one per queued iteration and the one waited on
-    Event ev_[k_events];
-    Event done_;
+    std::vector<Forecast> forecast_;
+    unsigned long long* report_dev_ = nullptr; // device addresses of the pinned buffers
+    SolveState* init_dev_ = nullptr;
+    SolveState* out_dev_ = nullptr;
     Event t0_;
     Event t1_;
     bool use_graphs_ = true;
     long long solves_ = 0;
     cfdg_precision precision_ = CFDG_PREC_FP64;
     hipGraphExec_t init_exec_ = nullptr;
-    hipGraphExec_t iter_exec_[2] = {nullptr, nullptr};
+    hipGraphExec_t even_exec_ = nullptr;                            // one even iteration
+    hipGraphExec_t odd_exec_[3] = {nullptr, nullptr, nullptr};      // 1, 2, 4 iterations from an odd one
 };
 
 System::~System() {
@@ -2100,8 +2171,8 @@ struct SlotMachinery {
     PinnedBuf<SysDev> desc_host;
     PinnedBuf<SolveState> init_host;
     PinnedBuf<SolveState> out_host;
-    PinnedBuf<int> status;      // two regions of k entries, one per iteration parity
-    int* status_dev = nullptr;
+    PinnedBuf<unsigned long long> status; // report words: two regions of k, one per iteration parity
+    unsigned long long* status_dev = nullptr;
     std::vector<System*> sys;   // per slot
     std::vector<int> phase;
     std::vector<Tables> single; // per slot: tables of the slot's system alone
@@ -2142,10 +2213,8 @@ SlotRunner::SlotRunner(int slots, const BatchOptions& opt, int sweeps, hipStream
     m.desc_host = PinnedBuf<SysDev>(k);
     m.init_host = PinnedBuf<SolveState>(k);
     m.out_host = PinnedBuf<SolveState>(k);
-    m.status = PinnedBuf<int>(2 * k);
-    void* dev = nullptr;
-    hip_check(hipHostGetDevicePointer(&dev, m.status.get(), 0), "hipHostGetDevicePointer");
-    m.status_dev = static_cast<int*>(dev);
+    m.status = PinnedBuf<unsigned long long>(2 * k);
+    m.status_dev = m.status.device();
     m.sys.assign(k, nullptr);
     m.phase.assign(k, SLOT_FREE);
     m.single = std::vector<Tables>(k);
@@ -2214,7 +2283,7 @@ int SlotRunner::start(System* x, const cfdg_solve_control& c) {
     st.status = ST_RUNNING;
     hip_check(hipMemcpyAsync(x->state(), &st, sizeof(SolveState), hipMemcpyHostToDevice, m.s),
               "slot state H2D");
-    enqueue_init(m.pl, m.desc.get(), m.single[ju], m.s);
+    enqueue_init(m.pl, m.desc.get(), m.single[ju], m.s, nullptr);
     hip_check(hipGetLastError(), "slot init launch");
     m.sys[ju] = x;
     m.epoch[ju] = m.solves_started++;
@@ -2258,13 +2327,12 @@ void SlotRunner::step(std::vector<Done>& done) {
         m.inflight.erase(m.inflight.begin());
         const int hp = static_cast<int>(h & 1);
         spin_wait(m.ev[hp].get(), "event sync");
-        const int* flags = m.status.get() + static_cast<std::size_t>(hp) * m.k;
+        const unsigned long long* flags = m.status.get() + static_cast<std::size_t>(hp) * m.k;
         for (const auto& [j, ep] : m.covered[hp]) {
             const std::size_t ju = static_cast<std::size_t>(j);
-            const int f = flags[ju];
+            const Report f(flags[ju]);
             // Flags of a slot's earlier solve say nothing about the one that occupies it now.
-            if (m.phase[ju] != SLOT_RUNNING || m.epoch[ju] != ep || f == ST_RUNNING ||
-                f == ST_CONVERGED_PENDING) {
+            if (m.phase[ju] != SLOT_RUNNING || m.epoch[ju] != ep || f.running()) {
                 continue;
             }
             const Tables& one = m.single[ju];
