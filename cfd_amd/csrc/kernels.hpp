@@ -10,10 +10,10 @@
 // Work mapping. A launch covers the rows of one level for a set of systems: block b processes
 // the 256-row block blocks[b].y of system blocks[b].x. A single solve is a set of one system.
 //
-// Reductions. Dot products never use atomics: each block writes one partial sum (wave
-// butterfly, then the four wave sums in order), and a finalize kernel with one workgroup per
-// system adds the partials in a fixed order. Results are reproducible run to run and do not
-// depend on which other systems share the launch.
+// Reductions. Dot products never use atomics: each group of rows (at most k_max_groups a system)
+// gets one partial sum (wave butterfly, then the four wave sums in order), and the kernel that needs
+// the dot product adds the partials in a fixed order in its prologue (take_step). Results are
+// reproducible run to run and do not depend on which other systems share the launch.
 //
 // Control. Each system carries a SolveState; kernels of a system whose status is non-zero
 // return at once, so the host may enqueue iterations ahead of the convergence test.
@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace cfdg {
 
@@ -243,68 +244,207 @@ __device__ __forceinline__ T csr_lane_sum(const gmem_t<const int>* __restrict__ 
 #endif
 constexpr int k_sym_group = CFDG_SYM_GROUP; // entries whose loads are issued together
 
-// One entry of a row in symmetric stencil storage: offset o, stored slot j of |o|. The value of
-// o >= 0 is in the row's own slot, of o < 0 in row + o's slot of -o (zero where row + o < 0); the
-// column is row + o clamped to the matrix, as in the per-slice stencil layout (whose missing
-// offsets hold zeros).
+// Element i of an array whose base is the same for the whole wavefront: the base stays in scalar
+// registers and the address is one 32-bit byte offset per lane (i sizeof(T) < 2^32), which all the
+// loads of a row share.
+template <class T>
+__device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, unsigned i) {
+    return *(const gmem_t<const T>*)((const gmem_t<const char>*)base + i * static_cast<unsigned>(sizeof(T)));
+}
+
+template <class T>
+__device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, unsigned i, T v) {
+    *(gmem_t<T>*)((gmem_t<char>*)base + i * static_cast<unsigned>(sizeof(T))) = v;
+}
+
+// What a row product multiplies a column with: (c) for any column; at(near, k, row) for column
+// row + o[k] of a stencil, near = near<N>(o) being the arrays' addresses moved by the stencil's
+// offsets (they stay in scalar registers; added to the row in the loop, they became a 64-bit vector
+// address per load).
+template <int N, class T>
+struct Moved {
+    const gmem_t<const T>* p[N];
+    __device__ __forceinline__ Moved(const gmem_t<const T>* base, const int (&o)[N]) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            p[k] = base + o[k];
+        }
+    }
+};
+
+template <class T>
+struct GatherX { // x_c
+    const gmem_t<const T>* x;
+    __device__ __forceinline__ T operator()(int c) const { return x[c]; }
+    template <int N>
+    struct Near {
+        Moved<N, T> x;
+    };
+    template <int N>
+    __device__ __forceinline__ Near<N> near(const int (&o)[N]) const {
+        return {Moved<N, T>(x, o)};
+    }
+    template <int N>
+    __device__ __forceinline__ T at(const Near<N>& a, int k, unsigned row) const {
+        return load_at<T>(a.x.p[k], row);
+    }
+};
+
+template <class T>
+struct GatherX1 { // (f wd_c) b_c: the first Jacobi iterate from zero, formed on the fly
+    const gmem_t<const T>* wd;
+    const gmem_t<const T>* b;
+    T f;
+    __device__ __forceinline__ T operator()(int c) const { return (f * wd[c]) * b[c]; }
+    template <int N>
+    struct Near {
+        Moved<N, T> wd;
+        Moved<N, T> b;
+    };
+    template <int N>
+    __device__ __forceinline__ Near<N> near(const int (&o)[N]) const {
+        return {Moved<N, T>(wd, o), Moved<N, T>(b, o)};
+    }
+    template <int N>
+    __device__ __forceinline__ T at(const Near<N>& a, int k, unsigned row) const {
+        return (f * load_at<T>(a.wd.p[k], row)) * load_at<T>(a.b.p[k], row);
+    }
+};
+
+template <class TZ>
+struct GatherPz { // z_c + beta p_c: the new search direction
+    const gmem_t<const TZ>* z;
+    const gmem_t<const double>* p;
+    double beta;
+    __device__ __forceinline__ double operator()(int c) const { return static_cast<double>(z[c]) + beta * p[c]; }
+    template <int N>
+    struct Near {
+        Moved<N, TZ> z;
+        Moved<N, double> p;
+    };
+    template <int N>
+    __device__ __forceinline__ Near<N> near(const int (&o)[N]) const {
+        return {Moved<N, TZ>(z, o), Moved<N, double>(p, o)};
+    }
+    template <int N>
+    __device__ __forceinline__ double at(const Near<N>& a, int k, unsigned row) const {
+        return static_cast<double>(load_at<TZ>(a.z.p[k], row)) + beta * load_at<double>(a.p.p[k], row);
+    }
+};
+
+struct GatherOne { // row sums of the matrix
+    __device__ __forceinline__ double operator()(int) const { return 1.0; }
+    template <int N>
+    struct Near {};
+    template <int N>
+    __device__ __forceinline__ Near<N> near(const int (&)[N]) const {
+        return {};
+    }
+    template <int N>
+    __device__ __forceinline__ double at(const Near<N>&, int, unsigned) const {
+        return 1.0;
+    }
+};
+
+// Entry of offset o of a row in symmetric stencil storage (stored slot j of |o|) where the row may
+// lie within the stencil's reach of the matrix's ends: the column is clamped to the matrix, as in
+// the per-slice stencil layout (whose missing offsets hold zeros), and the value is zero where
+// row + o < 0.
 template <class T, class F>
-__device__ __forceinline__ void sym_entry(const gmem_t<const T>* __restrict__ val, int stride, int last, int row, int o,
+__device__ __forceinline__ void sym_entry(const gmem_t<const T>* __restrict__ val, int pad, int last, int row, int o,
                                           int j, F load, T& a, T& x) {
     const int r = o < 0 ? row + o : row;
-    const int rr = max(r, 0);
-    const T v = val[(rr >> 6) * stride + j * k_wave + (rr & (k_wave - 1))];
+    const T v = load_at<T>(val + static_cast<long long>(j) * pad, static_cast<unsigned>(max(r, 0)));
     a = r < 0 ? T(0) : v;
     x = load(min(max(row + o, 0), last));
 }
 
-// Row sums (rows row0, and row0 + 64 when Rows == 2) of a stencil of N offsets known at compile
-// time: the table is read with constant indices (one batch of scalar loads, one wait) and every
-// entry's loads are issued before the sums, which run in offset order.
-template <int N, int Rows, class T, class F>
-__device__ __forceinline__ void sym_rows_fixed(const EllView& m, int row0, F load, T (&y)[2]) {
-    const auto tab = gm(m.soff); // offsets [0, N), stored slots [N, 2 N)
-    const auto val = gm(static_cast<const T*>(m.val));
-    const int stride = m.sym_w * k_wave;
-    const int last = m.n_rows - 1;
-    int o[N];
-    int j[N];
+// A symmetric stencil of N offsets, in scalar registers for a whole kernel (read from the table
+// inside a loop that stores, it came back by vector loads and a wait each time).
+template <int N, class T>
+struct SymStencil {
+    int o[N];                      // offsets, ascending and symmetric
+    const gmem_t<const T>* val[N]; // value of offset o[k] of row r at val[k][r]
+    int reach;
+    int last;
+    __device__ __forceinline__ explicit SymStencil(const EllView& m) {
+        const auto tab = gm(m.soff); // offsets [0, N), stored slots [N, 2 N)
+        const long long pad = static_cast<long long>(m.n_slices) * k_wave;
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-        o[k] = tab[k];
-        j[k] = tab[N + k];
+        for (int k = 0; k < N; ++k) {
+            o[k] = __builtin_amdgcn_readfirstlane(tab[k]);
+            const int j = __builtin_amdgcn_readfirstlane(tab[N + k]);
+            val[k] = gm(static_cast<const T*>(m.val)) + (j * pad + min(o[k], 0));
+        }
+        reach = o[N - 1];
+        last = m.n_rows - 1;
     }
+};
+
+// Row sums of Rows slices (s, s + ds) of a symmetric stencil: every entry's loads are issued before
+// the sums, which run in offset order. Away from the matrix's ends an entry is one value load and
+// the gather's loads, all from scalar bases with the lane's row as the only vector address; in the
+// first and last few slices, within the stencil's reach of the ends, every entry has clamped
+// addresses of its own. Rows past the end give the last row's sum.
+template <int Rows, int N, class T, class F, class Near>
+__device__ __forceinline__ void sym_rows_fixed(const SymStencil<N, T>& m, int s, int ds, int lane, const F& load,
+                                               const Near& near, T (&y)[2]) {
+    const int lo = s * k_wave;
+    const int hi = (s + (Rows - 1) * ds) * k_wave + k_wave - 1;
     T a[Rows][N];
     T x[Rows][N];
+    if (lo >= m.reach && hi + m.reach <= m.last) { // uniform over the wavefront
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
+        for (int k = 0; k < N; ++k) {
 #pragma unroll
-        for (int h = 0; h < Rows; ++h) {
-            sym_entry<T>(val, stride, last, row0 + h * k_wave, o[k], j[k], load, a[h][k], x[h][k]);
+            for (int h = 0; h < Rows; ++h) {
+                const unsigned row = static_cast<unsigned>((s + h * ds) * k_wave + lane);
+                a[h][k] = load_at<T>(m.val[k], row);
+                x[h][k] = load.at(near, k, row);
+            }
         }
+        asm volatile("; stencil inside"); // keeps the compiler from merging the two branches' loads
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+#pragma unroll
+            for (int h = 0; h < Rows; ++h) {
+                // Both arrays are read at the row whose column row + o[k] is clamped to the matrix,
+                // as in the per-slice stencil layout (whose missing offsets hold zeros). The value of
+                // an offset past the end is the row's own slot, a stored zero.
+                const int row = min((s + h * ds) * k_wave + lane, m.last);
+                const int c = min(max(row + m.o[k], 0), m.last);
+                const T v = load_at<T>(m.val[k], static_cast<unsigned>(m.o[k] < 0 ? c - m.o[k] : row));
+                a[h][k] = row + m.o[k] < 0 ? T(0) : v;
+                x[h][k] = load.at(near, k, static_cast<unsigned>(c - m.o[k]));
+            }
+        }
+        asm volatile("; stencil at an end");
     }
 #pragma unroll
     for (int h = 0; h < Rows; ++h) {
-        T s = T(0);
+        T t = T(0);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            s = madd(a[h][k], x[h][k], s);
+            t = madd(a[h][k], x[h][k], t);
         }
-        y[h] = s;
+        asm volatile("" : "+v"(t)); // summed here: not moved, loads and all, under the row's store
+        y[h] = t;
     }
 }
 
 // Any stencil size: the table read per entry, loads issued k_sym_group entries at a time.
 template <int Rows, class T, class F>
-__device__ __forceinline__ void sym_rows_any(const EllView& m, int row0, F load, T (&y)[2]) {
+__device__ __forceinline__ void sym_rows_any(const EllView& m, int s, int ds, int lane, F load, T (&y)[2]) {
     const int n = m.sym_n;
     const auto tab = gm(m.soff);
     const auto val = gm(static_cast<const T*>(m.val));
-    const int stride = m.sym_w * k_wave;
+    const int pad = m.n_slices * k_wave;
     const int last = m.n_rows - 1;
-    T s[Rows];
+    T t[Rows];
 #pragma unroll
     for (int h = 0; h < Rows; ++h) {
-        s[h] = T(0);
+        t[h] = T(0);
     }
     for (int k = 0; k < n; k += k_sym_group) {
         T a[Rows][k_sym_group];
@@ -316,7 +456,7 @@ __device__ __forceinline__ void sym_rows_any(const EllView& m, int row0, F load,
             const int j = tab[n + kk];
 #pragma unroll
             for (int h = 0; h < Rows; ++h) {
-                sym_entry<T>(val, stride, last, row0 + h * k_wave, o, j, load, a[h][g], x[h][g]);
+                sym_entry<T>(val, pad, last, min((s + h * ds) * k_wave + lane, last), o, j, load, a[h][g], x[h][g]);
             }
         }
 #pragma unroll
@@ -324,50 +464,42 @@ __device__ __forceinline__ void sym_rows_any(const EllView& m, int row0, F load,
             if (k + g < n) {
 #pragma unroll
                 for (int h = 0; h < Rows; ++h) {
-                    s[h] = madd(a[h][g], x[h][g], s[h]);
+                    t[h] = madd(a[h][g], x[h][g], t[h]);
                 }
             }
         }
     }
 #pragma unroll
     for (int h = 0; h < Rows; ++h) {
-        y[h] = s[h];
+        y[h] = t[h];
     }
 }
 
+// Row sums of slices s and (Rows == 2) s + ds in symmetric stencil storage (EllView::sym_w > 0),
+// entries in offset order; their loads are issued together. Rows past the end give the sums of the
+// last row.
 template <int Rows, class T, class F>
-__device__ __forceinline__ void sym_rows(const EllView& m, int row0, F load, T (&y)[2]) {
+__device__ __forceinline__ void sym_rows(const EllView& m, int s, int ds, int lane, F load, T (&y)[2]) {
+    s = __builtin_amdgcn_readfirstlane(s); // one slice per wavefront
     switch (m.sym_n) { // uniform: the stencils of 3-D, 2-D and 1-D box meshes unrolled
-    case 7:
-        sym_rows_fixed<7, Rows, T>(m, row0, load, y);
+    case 7: {
+        const SymStencil<7, T> st(m);
+        sym_rows_fixed<Rows>(st, s, ds, lane, load, load.near(st.o), y);
         return;
-    case 5:
-        sym_rows_fixed<5, Rows, T>(m, row0, load, y);
-        return;
-    case 3:
-        sym_rows_fixed<3, Rows, T>(m, row0, load, y);
-        return;
-    default:
-        sym_rows_any<Rows, T>(m, row0, load, y);
     }
-}
-
-// Row sum of a row in symmetric stencil storage (EllView::sym_w > 0), entries in offset order.
-template <class T, class F>
-__device__ __forceinline__ T ell_row_sym(const EllView& m, int slice, int lane, F load) {
-    T y[2];
-    sym_rows<1, T>(m, slice * k_wave + lane, load, y);
-    return y[0];
-}
-
-// ell_row_sym for the rows of slices s0 and s0 + 1 (lane's row in each), their loads issued
-// together: the same sums as two ell_row_sym calls.
-template <class T, class F>
-__device__ __forceinline__ void ell_row_sym_pair(const EllView& m, int s0, int lane, F load, T& ya, T& yb) {
-    T y[2];
-    sym_rows<2, T>(m, s0 * k_wave + lane, load, y);
-    ya = y[0];
-    yb = y[1];
+    case 5: {
+        const SymStencil<5, T> st(m);
+        sym_rows_fixed<Rows>(st, s, ds, lane, load, load.near(st.o), y);
+        return;
+    }
+    case 3: {
+        const SymStencil<3, T> st(m);
+        sym_rows_fixed<Rows>(st, s, ds, lane, load, load.near(st.o), y);
+        return;
+    }
+    default:
+        sym_rows_any<Rows, T>(m, s, ds, lane, load, y);
+    }
 }
 
 // Row sum of an ELL row with the x entry of column c produced by load(c), in storage order.
@@ -375,7 +507,9 @@ __device__ __forceinline__ void ell_row_sym_pair(const EllView& m, int s0, int l
 template <class T, class F>
 __device__ __forceinline__ T ell_row_f(const EllView& m, int slice, int lane, F load) {
     if (m.sym_w > 0) {
-        return ell_row_sym<T>(m, slice, lane, load);
+        T y[2];
+        sym_rows<1, T>(m, slice, 0, lane, load, y);
+        return y[0];
     }
     const int base = m.sp[slice];
     const int w = (m.sp[slice + 1] - base) / k_wave;
@@ -408,8 +542,7 @@ __device__ __forceinline__ T ell_row_f(const EllView& m, int slice, int lane, F 
 // Row sum of an ELL row: sum_k val_k * x[col_k] in storage order (any column / value format).
 template <class T>
 __device__ __forceinline__ T ell_row(const EllView& m, int slice, int lane, const T* __restrict__ x) {
-    const auto gx = gm(x);
-    return ell_row_f<T>(m, slice, lane, [&](int c) { return gx[c]; });
+    return ell_row_f<T>(m, slice, lane, GatherX<T>{gm(x)});
 }
 
 // Row sum with the first Jacobi iterate x1_j = wd_j * b_j formed on the fly (the reference's
@@ -417,7 +550,7 @@ __device__ __forceinline__ T ell_row(const EllView& m, int slice, int lane, cons
 template <class T>
 __device__ __forceinline__ T ell_row_x1(const EllView& m, int slice, int lane, const gmem_t<const T>* __restrict__ wd,
                                         const gmem_t<const T>* __restrict__ b, T f) {
-    return ell_row_f<T>(m, slice, lane, [&](int c) { return (f * wd[c]) * b[c]; });
+    return ell_row_f<T>(m, slice, lane, GatherX1<T>{wd, b, f});
 }
 
 // Row sums of two slices with equal widths and one column format, their loads issued together
@@ -495,36 +628,40 @@ __device__ __forceinline__ void ell_sum2(const C& ca, const C& cb, const gmem_t<
     }
 }
 
-// The lane's share of its rows in slices s0 and s0 + 1 of a sliced-ELL matrix (a slice past the
-// end gives 0; with tpr > 1 the caller adds the row groups): equal to ell_row_f on each slice,
+// The lane's share of its rows in slices s0 and s1 = s0 + ds of a sliced-ELL matrix (a slice past
+// the end gives 0; with tpr > 1 the caller adds the row groups): equal to ell_row_f on each slice,
 // bit for bit. Slices of different widths are summed one after the other. Stencil columns and
 // BF16 rows occur with one lane per row only.
 template <class T, class F>
-__device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int lane, F load, T& ya, T& yb) {
+__device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int ds, int lane, F load, T& ya, T& yb) {
+    const int s1 = s0 + ds;
     ya = T(0);
     yb = T(0);
     if (s0 >= m.n_slices) {
         return;
     }
-    if (s0 + 1 >= m.n_slices) {
+    if (s1 >= m.n_slices) {
         ya = ell_row_f<T>(m, s0, lane, load);
         return;
     }
     if (m.sym_w > 0) {
-        ell_row_sym_pair<T>(m, s0, lane, load, ya, yb);
+        T y[2];
+        sym_rows<2, T>(m, s0, ds, lane, load, y);
+        ya = y[0];
+        yb = y[1];
         return;
     }
     const int b0 = m.sp[s0];
-    const int b1 = m.sp[s0 + 1];
-    const int w = (b1 - b0) / k_wave;
-    if (w != (m.sp[s0 + 2] - b1) / k_wave) {
+    const int b1 = m.sp[s1];
+    const int w = (m.sp[s0 + 1] - b0) / k_wave;
+    if (w != (m.sp[s1 + 1] - b1) / k_wave) {
         ya = ell_row_f<T>(m, s0, lane, load);
-        yb = ell_row_f<T>(m, s0 + 1, lane, load);
+        yb = ell_row_f<T>(m, s1, lane, load);
         return;
     }
     const int lg = __builtin_ctz(m.tpr);
     const int r0 = s0 * (k_wave >> lg) + (lane >> lg);
-    const int r1 = r0 + (k_wave >> lg);
+    const int r1 = s1 * (k_wave >> lg) + (lane >> lg);
     auto pair = [&](const auto& c0, const auto& c1) {
         if constexpr (sizeof(T) == 4) {
             if (m.fmt == 1) {
@@ -548,7 +685,7 @@ __device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int lane,
         pair(ColStencil{gm(m.soff) + t0, r0, m.n_rows - 1}, ColStencil{gm(m.soff) + t1, r1, m.n_rows - 1});
     } else if (m.cbase != nullptr) {
         const auto dc = gm(reinterpret_cast<const unsigned short*>(m.dcol));
-        pair(ColBase{dc + b0 + lane, gm(m.cbase)[s0]}, ColBase{dc + b1 + lane, gm(m.cbase)[s0 + 1]});
+        pair(ColBase{dc + b0 + lane, gm(m.cbase)[s0]}, ColBase{dc + b1 + lane, gm(m.cbase)[s1]});
     } else if (m.dcol != nullptr) {
         pair(ColOff{gm(m.dcol) + b0 + lane, r0}, ColOff{gm(m.dcol) + b1 + lane, r1});
     } else {
@@ -608,8 +745,6 @@ __device__ __forceinline__ T mat_row_x1(const EllView& m, int row, int sub, cons
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup i runs on XCD i mod 8) and
 // every XCD has its own L2. This bijection hands each XCD a contiguous range of logical blocks,
 // so rows that share neighbours (and their x entries) meet in the same L2.
-constexpr int k_xcds = 8;
-
 __device__ __forceinline__ int xcd_block() {
     const int g = static_cast<int>(gridDim.x);
     const int b = static_cast<int>(blockIdx.x);
@@ -627,50 +762,51 @@ __device__ __forceinline__ int2 block_entry(const int2* __restrict__ blocks) {
     return make_int2(static_cast<int>(static_cast<unsigned>(e)), static_cast<int>(static_cast<unsigned>(e >> 32)));
 }
 
-// Outer vectors by id: 0 x, 1 r, 2 p, 3 q, 4 z, 5 r0, 6 v, 7 s, 8 t, 9 ph, 10 sh.
-__device__ __forceinline__ double* outer_vec(const SysDev& S, int id) {
-    switch (id) {
-    case 0: return S.x;
-    case 1: return S.r;
-    case 2: return S.p;
-    case 3: return S.q;
-    case 4: return S.z;
-    case 5: return S.r0;
-    case 6: return S.v;
-    case 7: return S.s;
-    case 8: return S.t;
-    case 9: return S.ph;
-    default: return S.sh;
-    }
-}
+// Forms of the level-0 operator that a kernel is built for. L0_ANY: the library's layouts, told
+// apart at run time. L0_SYM7: symmetric stencil storage of 7 offsets (every 3-D box's pressure
+// matrix), for launches whose systems all have it: the kernel holds that one path, in fewer
+// registers. L0_CSR: a caller's CSR arrays read in place (a64.sp = row offsets, a64.col, a64.val;
+// one lane per row, entries in CSR order), which gives the same sums: the sliced-ELL padding and
+// stencil gaps add exact zeros after or between the same products in the same order.
+enum L0Form : int { L0_ANY = 0, L0_SYM7 = 1, L0_CSR = 2 };
 
-// Level-0 FP64 row product of the calling lane's row. Csr = false: the library's sliced-ELL
-// layout (every lane of a live slice takes part). Csr = true: a caller's CSR arrays read in
-// place (a64.sp = row offsets, a64.col, a64.val; one lane per row, entries in CSR order), which
-// gives the same sums: the sliced-ELL padding and stencil gaps add exact zeros after or between
-// the same products in the same order. Rows past the end give 0.
-template <bool Csr>
-__device__ __forceinline__ bool a0_live(const EllView& m, int slice) {
-    return Csr || slice < m.n_slices;
-}
+// The level-0 operator and what it is multiplied with, as a kernel of that form keeps them.
+template <int Form, class T, class F>
+struct L0Op {
+    EllView m;
+    F load;
+    __device__ __forceinline__ L0Op(const EllView& v, const F& f) : m(v), load(f) {}
+};
 
-template <bool Csr, class F>
-__device__ __forceinline__ double a0_row_f(const EllView& m, int slice, int lane, int row, F load) {
-    if constexpr (Csr) {
-        if (row >= m.n_rows) {
-            return 0.0;
-        }
+template <class T, class F>
+struct L0Op<L0_SYM7, T, F> {
+    SymStencil<7, T> m;
+    F load;
+    typename F::template Near<7> near;
+    __device__ __forceinline__ L0Op(const EllView& v, const F& f) : m(v), load(f), near(f.near(m.o)) {}
+};
+
+// Row sums of the lane's rows of slices s and (Rows == 2) s + ds, their loads issued together. Rows
+// past the end give some row's sum, or 0.
+template <int Rows, int Form, class T, class F>
+__device__ __forceinline__ void l0_rows(const L0Op<Form, T, F>& op, int s, int ds, int lane, T (&y)[2]) {
+    const auto& m = op.m;
+    if constexpr (Form == L0_CSR) {
         const auto sp = gm(m.sp);
-        return csr_lane_sum<double>(gm(m.col), gm(static_cast<const double*>(m.val)), sp[row], sp[row + 1], 1, load);
+#pragma unroll
+        for (int h = 0; h < Rows; ++h) {
+            const int row = (s + h * ds) * k_wave + lane;
+            y[h] = row < m.n_rows ? csr_lane_sum<double>(gm(m.col), gm(static_cast<const double*>(m.val)), sp[row],
+                                                         sp[row + 1], 1, op.load)
+                                  : 0.0;
+        }
+    } else if constexpr (Form == L0_SYM7) {
+        sym_rows_fixed<Rows>(m, __builtin_amdgcn_readfirstlane(s), ds, lane, op.load, op.near, y);
+    } else if constexpr (Rows == 2) {
+        ell_row_pair<T>(m, s, ds, lane, op.load, y[0], y[1]);
     } else {
-        return ell_row_f<double>(m, slice, lane, load);
+        y[0] = s < m.n_slices ? ell_row_f<T>(m, s, lane, op.load) : T(0);
     }
-}
-
-template <bool Csr>
-__device__ __forceinline__ double a0_row(const EllView& m, int slice, int lane, int row, const double* __restrict__ x) {
-    const auto gx = gm(x);
-    return a0_row_f<Csr>(m, slice, lane, row, [&](int c) { return gx[c]; });
 }
 
 #define CFDG_BLOCK_PROLOGUE(sysarr, blocks)                                                     \
@@ -683,355 +819,736 @@ __device__ __forceinline__ double a0_row(const EllView& m, int slice, int lane, 
     (void)row;
 
 // ------------------------------------------------------------------------------------------
+// Scalar steps of the Krylov recurrences
+// ------------------------------------------------------------------------------------------
+
+// Steps between two kernels of an iteration. Each needs the sum of one or two partials of the
+// kernel before it. The kernel after it makes the step itself: every workgroup adds the at most
+// k_max_groups partials (a few kilobytes, L2-resident) in the same order and computes the same
+// scalars, and the system's first workgroup stores the new state. A launch of its own for the step
+// cost 4.6 to 8.9 us an iteration at 128^3 and 2.3 us in the smallest systems; in the kernel's
+// prologue it costs about 0.7 us. The state is kept in k_states copies, so that no workgroup reads
+// the copy that the first one writes: step Op reads copy state_in and writes state_out, and the
+// state goes round them once an iteration.
+enum FinOp : int {
+    FIN_RES = 0,          // AMG-PCG: |r|; converged?
+    FIN_BETA = 1,         // rz_new; beta = rz_new / rz (0 first); it++ / limit
+    FIN_BETA_FLEX = 2,    // rz_new, zq; beta = -zq / pq (0 first); it++ / limit
+    FIN_ALPHA = 3,        // pq; breakdown if 0; alpha = rz / pq
+    FIN_CG_RES_BETA = 4,  // Jacobi CG: residual test, then beta (0 first)
+    FIN_BICG_RES = 5,     // residual test, then rho and beta
+    FIN_BICG_ALPHA = 6,
+    FIN_BICG_S = 7,       // |s|: early exit?
+    FIN_BICG_OMEGA = 8,
+    FIN_TRUE = 9          // true residual (after the solve, copy 0 in place)
+};
+
+// Copies: AMG-PCG and Jacobi CG 2 -> (residual step) -> 0 -> (beta) -> 1 -> (alpha) -> 2, Jacobi CG
+// taking residual and beta in one step 2 -> 1 and reporting through copy 0; BiCGStab 3 ->
+// (residual, rho) -> 0 -> (alpha) -> 1 -> (s) -> 2 -> (omega) -> 3. Copy 0 is the solve's public state.
+__host__ __device__ constexpr int state_in(int op) {
+    return op == FIN_BETA || op == FIN_BETA_FLEX || op == FIN_BICG_ALPHA || op == FIN_TRUE ? 0
+           : op == FIN_ALPHA || op == FIN_BICG_S                                           ? 1
+           : op == FIN_BICG_RES                                                            ? 3
+                                                                                           : 2;
+}
+
+__host__ __device__ constexpr int state_out(int op) {
+    return op == FIN_BETA || op == FIN_BETA_FLEX || op == FIN_BICG_ALPHA || op == FIN_CG_RES_BETA ? 1
+           : op == FIN_ALPHA || op == FIN_BICG_S                                                  ? 2
+           : op == FIN_BICG_OMEGA                                                                 ? 3
+                                                                                                  : 0;
+}
+
+template <int Op>
+__host__ __device__ constexpr int step_slots() { // partials a step adds
+    return Op == FIN_BETA_FLEX || Op == FIN_CG_RES_BETA || Op == FIN_BICG_RES || Op == FIN_BICG_OMEGA ? 2 : 1;
+}
+
+template <int Op>
+__host__ __device__ constexpr int step_slot(int q) {
+    switch (Op) {
+    case FIN_RES: return SLOT_RR;
+    case FIN_BETA: return SLOT_RZ;
+    case FIN_BETA_FLEX: return q == 0 ? SLOT_RZ : SLOT_ZQ;
+    case FIN_ALPHA: return SLOT_PQ;
+    case FIN_CG_RES_BETA: return q == 0 ? SLOT_RR : SLOT_RZ;
+    case FIN_BICG_RES: return q == 0 ? SLOT_RR : SLOT_R0R;
+    case FIN_BICG_ALPHA: return SLOT_R0V;
+    case FIN_BICG_S: return SLOT_SS;
+    case FIN_BICG_OMEGA: return q == 0 ? SLOT_TT : SLOT_TS;
+    default: return SLOT_TRUE;
+    }
+}
+
+// Sums of the system's partials in slots slot(0) .. slot(N - 1), complete in every thread of a
+// k_block workgroup: thread t adds entries t, t + 256, ..., then the wavefront butterfly and the
+// four wavefronts in order. Every workgroup gets the same bits.
+template <int N, class Slot>
+__device__ __forceinline__ void reduce_slots(const SysDev& S, Slot slot, double (&out)[N]) {
+    __shared__ double red[N][k_slices_per_block];
+    const int n = S.n_groups;
+    double v[N][k_max_groups / k_block];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        const auto p = gm(static_cast<const double*>(S.partials)) + slot(q) * n;
+#pragma unroll
+        for (int k = 0; k < k_max_groups / k_block; ++k) { // every load before the first sum
+            const int i = static_cast<int>(threadIdx.x) + k * k_block;
+            v[q][k] = i < n ? p[i] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        double s = v[q][0];
+#pragma unroll
+        for (int k = 1; k < k_max_groups / k_block; ++k) {
+            s += v[q][k];
+        }
+        s = wave_sum(s);
+        if (threadIdx.x % k_wave == 0) {
+            red[q][threadIdx.x / k_wave] = s;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        double t = red[q][0];
+#pragma unroll
+        for (int w = 1; w < k_slices_per_block; ++w) {
+            t += red[q][w];
+        }
+        out[q] = t;
+    }
+}
+
+// A state in registers, loaded and stored field by field: copied as a SolveState, the compiler
+// keeps it in scratch memory (16 us a kernel).
+struct Scalars {
+    double tol, rz, pq, alpha, beta, res, bnorm, rho, omega;
+    int it, max_it, status;
+};
+
+__device__ __forceinline__ Scalars load_state(const SolveState* p) {
+    const auto g = gm(p);
+    Scalars s;
+    s.tol = g->tol;
+    s.rz = g->rz;
+    s.pq = g->pq;
+    s.alpha = g->alpha;
+    s.beta = g->beta;
+    s.res = g->res;
+    s.bnorm = g->bnorm;
+    s.rho = g->rho;
+    s.omega = g->omega;
+    s.it = g->it;
+    s.max_it = g->max_it;
+    s.status = g->status;
+    return s;
+}
+
+__device__ __forceinline__ void store_state(SolveState* p, const Scalars& s) {
+    const auto g = gm(p);
+    g->tol = s.tol;
+    g->rz = s.rz;
+    g->pq = s.pq;
+    g->alpha = s.alpha;
+    g->beta = s.beta;
+    g->res = s.res;
+    g->bnorm = s.bnorm;
+    g->rho = s.rho;
+    g->omega = s.omega;
+    g->it = s.it;
+    g->max_it = s.max_it;
+    g->status = s.status;
+}
+
+// The arithmetic of a step (krylov_kernels.inc:44-169, 240-301) on the sums v0, v1. A system that
+// ended keeps its state; an early exit of BiCGStab is complete after its x update.
+template <int Op>
+__device__ __forceinline__ void state_step(Scalars& st, double v0, double v1) {
+    if (Op == FIN_BICG_OMEGA && st.status == ST_CONVERGED_PENDING) {
+        st.status = ST_CONVERGED;
+    } else if (st.status == ST_RUNNING) {
+        if (Op == FIN_RES || Op == FIN_CG_RES_BETA || Op == FIN_BICG_RES) {
+            st.res = sqrt(v0);
+            st.status = st.res <= st.tol ? ST_CONVERGED : ST_RUNNING;
+        }
+        if (Op == FIN_BETA || Op == FIN_BETA_FLEX || (Op == FIN_CG_RES_BETA && st.status == ST_RUNNING)) {
+            const double rz_new = Op == FIN_CG_RES_BETA ? v1 : v0;
+            const double ratio = Op == FIN_BETA_FLEX ? -v1 / st.pq : rz_new / st.rz;
+            st.beta = st.it == 0 ? 0.0 : ratio;
+            st.rz = rz_new;
+            st.it += 1;
+            st.status = st.it > st.max_it ? ST_MAXIT : ST_RUNNING;
+        }
+        if (Op == FIN_ALPHA) {
+            st.pq = v0;
+            if (v0 == 0.0) {
+                st.status = ST_BREAKDOWN;
+            } else {
+                st.alpha = st.rz / v0;
+            }
+        }
+        if (Op == FIN_BICG_RES && st.status == ST_RUNNING) {
+            // rho_new = r0.r, the limit, the guards rho_new == 0 and omega == 0, beta
+            st.it += 1;
+            if (st.it > st.max_it) {
+                st.status = ST_MAXIT;
+            } else if (v1 == 0.0 || st.omega == 0.0) {
+                st.status = ST_BREAKDOWN;
+            } else {
+                st.beta = (v1 / st.rho) * (st.alpha / st.omega);
+                st.rho = v1;
+            }
+        }
+        if (Op == FIN_BICG_ALPHA) {
+            if (v0 == 0.0) {
+                st.status = ST_BREAKDOWN;
+            } else {
+                st.alpha = st.rho / v0;
+            }
+        }
+        if (Op == FIN_BICG_S) {
+            const double s_norm = sqrt(v0);
+            if (s_norm <= st.tol) {
+                st.res = s_norm;
+                st.status = ST_CONVERGED_PENDING;
+            }
+        }
+        if (Op == FIN_BICG_OMEGA) {
+            st.omega = v0 > 0.0 ? v1 / v0 : 0.0;
+        }
+    }
+}
+
+// A system's progress as one 64-bit word, so that a host that polls it never sees half a report:
+// the residual (FP32 bits) above, the number of finished iterations and the status below. The word
+// goes to host-mapped memory at every residual step; the host reads it while later iterations are
+// queued, without an event (an event record between two graph launches costs 4 us).
+__device__ __forceinline__ unsigned long long report_word(const Scalars& st, int done) {
+    const unsigned low = (static_cast<unsigned>(done) << k_report_status_bits) | static_cast<unsigned>(st.status);
+    return (static_cast<unsigned long long>(__float_as_uint(static_cast<float>(st.res))) << 32) | low;
+}
+
+// Iterations finished when residual step Op has run (Jacobi CG and BiCGStab count the next one
+// in the step when the solve goes on).
+template <int Op>
+__device__ __forceinline__ int iterations_done(const Scalars& st) {
+    return Op != FIN_RES && (st.status == ST_RUNNING || st.status == ST_BREAKDOWN) ? st.it - 1 : st.it;
+}
+
+template <int Op>
+__device__ __forceinline__ void store_report(const Scalars& st, unsigned long long* report, int id) {
+    if (report != nullptr) {
+        __hip_atomic_store(report + id, report_word(st, iterations_done<Op>(st)), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// Step Op in the prologue of a k_block kernel: the state after it in every thread, stored (and
+// reported, report may be null) by the system's first workgroup. Workgroups of a system that ended
+// skip the sums.
+template <int Op>
+__device__ __forceinline__ Scalars take_step(const SysDev& S, bool first, unsigned long long* report, int id) {
+    Scalars st = load_state(S.st + state_in(Op));
+    double v0 = 0.0;
+    double v1 = 0.0;
+    if (st.status == ST_RUNNING) { // uniform over the workgroup
+        double o[step_slots<Op>()];
+        reduce_slots<step_slots<Op>()>(S, [](int q) { return step_slot<Op>(q); }, o);
+        v0 = o[0];
+        v1 = o[step_slots<Op>() - 1];
+    }
+    state_step<Op>(st, v0, v1);
+    if (first && threadIdx.x == 0) {
+        store_state(S.st + state_out(Op), st);
+        store_report<Op>(st, report, id);
+    }
+    return st;
+}
+
+// Residual step Op (its result in the public copy 0), or the true residual, as a launch of its
+// own, one workgroup per system (ids: descriptor indices): at the end of a graph, where no kernel
+// of the next iteration makes the step yet, and in cycles whose first kernel cannot make it. The
+// step is the same one, bit for bit, so making it twice changes nothing.
+template <int Op>
+__global__ void __launch_bounds__(k_block) k_step(const SysDev* __restrict__ sys, const int* __restrict__ ids,
+                                                  unsigned long long* __restrict__ report) {
+    const int id = ids[blockIdx.x];
+    const SysDev& S = sys[id];
+    if (Op == FIN_TRUE) {
+        double t[1];
+        reduce_slots<1>(S, [](int) { return static_cast<int>(SLOT_TRUE); }, t);
+        if (threadIdx.x == 0) {
+            S.st[0].true_res = sqrt(t[0]);
+        }
+        return;
+    }
+    Scalars st = load_state(S.st + state_in(Op));
+    double o[step_slots<Op>()];
+    reduce_slots<step_slots<Op>()>(S, [](int q) { return step_slot<Op>(q); }, o);
+    if (threadIdx.x == 0) {
+        state_step<Op>(st, o[0], o[step_slots<Op>() - 1]);
+        store_state(S.st, st);
+        store_report<Op>(st, report, id);
+    }
+}
+
+// The start of a solve after its initial residual: |b| and BiCGStab's rho = alpha = omega = 1 into
+// the state that residual step Op reads, then that step.
+template <int Op>
+__global__ void __launch_bounds__(k_block) k_start(const SysDev* __restrict__ sys, const int* __restrict__ ids,
+                                                   unsigned long long* __restrict__ report) {
+    const int id = ids[blockIdx.x];
+    const SysDev& S = sys[id];
+    constexpr int n = step_slots<Op>() + 1;
+    double o[n];
+    reduce_slots<n>(S, [](int q) { return q + 1 == n ? static_cast<int>(SLOT_BB) : step_slot<Op>(q); }, o);
+    if (threadIdx.x == 0) {
+        Scalars st = load_state(S.st + state_in(Op));
+        st.bnorm = sqrt(o[n - 1]);
+        st.rho = 1.0;
+        st.alpha = 1.0;
+        st.omega = 1.0;
+        store_state(S.st + state_in(Op), st);
+        state_step<Op>(st, o[0], o[n - 2]);
+        store_state(S.st, st);
+        store_report<Op>(st, report, id);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// Level-0 kernels: groups of rows
+// ------------------------------------------------------------------------------------------
+
+// A level-0 kernel's workgroup serves the row groups [bk_.y, bk_.y + gpb) of its system, one after
+// the other. A group is S.chunks chunks of 256 rows and has one partial sum per dot product, so
+// that a step adds at most k_max_groups partials whatever the system's size (one chunk up to
+// 262,144 rows, 8 at 128^3); the grouping depends on the system's size only, so its sums do not
+// depend on which systems share the launch. gpb > 1 in large batches keeps the number of
+// workgroups, each of which makes the step, near 8192.
+//
+// A group's chunks are not neighbours: the groups fall into k_xcds segments (one XCD's workgroups of
+// a single system), a segment owns a contiguous range of chunks, and its groups take the chunks of
+// the range in turn. The workgroups of an XCD thus move through the rows as one window, as if every
+// chunk were a workgroup of its own. With a group's chunks side by side the workgroups read at a
+// distance of 2048 rows from each other, which keeps a few memory channels busy and the others idle:
+// 41.7 against 39.0 us for the outer product at 128^3 (two chunks of its rows at a time).
+#define CFDG_L0_PROLOGUE(sysarr, blocks)                                                          \
+    const int2 bk_ = block_entry(blocks);                                                         \
+    const SysDev& S = (sysarr)[bk_.x];                                                            \
+    const int wave_ = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / k_wave);     \
+    const int lane = static_cast<int>(threadIdx.x) % k_wave;                                      \
+    const bool first_ = bk_.y == 0;                                                               \
+    (void)first_;                                                                                 \
+    (void)lane;
+
+// Runs rows(H, slice, ds) over the slices of group g that the wavefront serves: slice and, where the
+// constant H is 2, slice + ds (its slice of the group's next chunk). Rows past the end are included.
+// Pair: two chunks at a time, so that two rows' loads are in flight in each lane (a system of more
+// than one chunk a group has about four wavefronts on a SIMD).
+template <bool Pair, class R>
+__device__ __forceinline__ void group_rows(const SysDev& S, int g, int wave, R rows) {
+    const int chunks = S.chunks;
+    const int seg = S.segment;
+    const int s = g / seg;
+    const int ds = min(seg, S.n_groups - s * seg) * k_slices_per_block; // a group's chunks are this far apart
+    int slice = (s * seg * chunks + (g - s * seg)) * k_slices_per_block + wave;
+    int c = 0;
+    if constexpr (Pair) {
+        for (; c + 1 < chunks; c += 2, slice += 2 * ds) {
+            rows(std::integral_constant<int, 2>{}, slice, ds);
+        }
+    }
+    for (; c < chunks; ++c, slice += ds) {
+        rows(std::integral_constant<int, 1>{}, slice, ds);
+    }
+}
+
+// The lane's rows of slices slice and (Rows == 2) slice + ds; load(h, r) requests what a row's result
+// needs of its own entries, before the row sums' loads (rows past the end: of the last row).
+template <int Rows, class F>
+__device__ __forceinline__ void own_rows(int slice, int ds, int lane, unsigned n, unsigned (&row)[2], F load) {
+#pragma unroll
+    for (int h = 0; h < Rows; ++h) {
+        row[h] = static_cast<unsigned>((slice + h * ds) * k_wave + lane);
+        load(h, min(row[h], n - 1));
+    }
+}
+
+// Runs rows(H, slice, ds, v) over the workgroup's groups (v[q] += the rows' terms, first row first)
+// and stores the sums of each group in partials slots slot(0) .. slot(N - 1).
+template <int N, bool Pair, class R, class Slot>
+__device__ __forceinline__ void for_groups(const SysDev& S, int first, int gpb, int wave, R rows, Slot slot) {
+    const int n = S.n_groups;
+    const int end = min(first + gpb, n);
+    for (int g = first; g < end; ++g) {
+        double v[N] = {};
+        group_rows<Pair>(S, g, wave, [&](auto H, int slice, int ds) { rows(H, slice, ds, v); });
+        double o[N];
+        block_sums<N>(v, o);
+        if (threadIdx.x == 0) {
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                S.partials[slot(q) * n + g] = o[q];
+            }
+        }
+        if (g + 1 < end) {
+            __syncthreads(); // block_sums' buffer is read by thread 0
+        }
+    }
+}
+
+// The same without dot products.
+template <bool Pair, class R>
+__device__ __forceinline__ void for_group_rows(const SysDev& S, int first, int gpb, int wave, R rows) {
+    const int end = min(first + gpb, S.n_groups);
+    for (int g = first; g < end; ++g) {
+        group_rows<Pair>(S, g, wave, rows);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // Outer Krylov kernels (level 0, FP64)
 // ------------------------------------------------------------------------------------------
 
 // r = b - A x, partials r.r and b.b; p = q = 0. For mixed precision also r32 = (float) r.
-template <bool Mixed>
-__global__ void __launch_bounds__(k_block) k_residual0(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    double rr = 0.0;
-    double bb = 0.0;
-    if (slice < S.a64.n_slices) {
-        const double ax = ell_row<double>(S.a64, slice, lane, S.x);
+template <bool Mixed, int Form>
+__global__ void __launch_bounds__(k_block) k_residual0(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
+    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2]) {
+        const int row = slice * k_wave + lane;
+        double y[2];
+        l0_rows<1>(A0, slice, 0, lane, y);
         if (row < S.n) {
             const double bi = gm(S.b)[row];
-            const double ri = bi - ax;
+            const double ri = bi - y[0];
             gm(S.r)[row] = ri;
             gm(S.p)[row] = 0.0;
             gm(S.q)[row] = 0.0;
             if (Mixed) {
                 gm(S.r32)[row] = static_cast<float>(ri);
             }
-            rr = ri * ri;
-            bb = bi * bi;
+            v[0] += ri * ri;
+            v[1] += bi * bi;
         }
-    }
-    double v[2] = {rr, bb};
-    double o[2];
-    block_sums<2>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-        S.partials[SLOT_BB * S.nblk0 + bk_.y] = o[1];
-    }
+    }, [](int q) { return q == 0 ? SLOT_RR : SLOT_BB; });
 }
 
 // Jacobi CG start: r = b - A x, z = dinv r, p = 0; partials r.r, r.z, b.b.
-template <bool Csr>
-__global__ void __launch_bounds__(k_block) k_cg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    double rr = 0.0;
-    double rz = 0.0;
-    double bb = 0.0;
-    if (a0_live<Csr>(S.a64, slice)) {
-        const double ax = a0_row<Csr>(S.a64, slice, lane, row, S.x);
+template <int Form>
+__global__ void __launch_bounds__(k_block) k_cg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
+    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[3]) {
+        const int row = slice * k_wave + lane;
+        double y[2];
+        l0_rows<1>(A0, slice, 0, lane, y);
         if (row < S.n) {
             const double bi = gm(S.b)[row];
-            const double ri = bi - ax;
+            const double ri = bi - y[0];
             const double zi = ri * gm(S.dinv)[row];
             gm(S.r)[row] = ri;
             gm(S.z)[row] = zi;
             gm(S.p)[row] = 0.0;
-            rr = ri * ri;
-            rz = ri * zi;
-            bb = bi * bi;
+            v[0] += ri * ri;
+            v[1] += ri * zi;
+            v[2] += bi * bi;
         }
-    }
-    double v[3] = {rr, rz, bb};
-    double o[3];
-    block_sums<3>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-        S.partials[SLOT_RZ * S.nblk0 + bk_.y] = o[1];
-        S.partials[SLOT_BB * S.nblk0 + bk_.y] = o[2];
-    }
+    }, [](int q) { return q == 0 ? SLOT_RR : q == 1 ? SLOT_RZ : SLOT_BB; });
 }
 
-// y = A x (level-0 FP64 operator) with the partial sum of w.y into `slot`; with Two, also the
-// partial of y.w2 into slot2. Used for q = A p (p.q), v = A ph (r0.v), t = A sh (t.t, t.s).
-template <bool Two, bool Csr>
-__global__ void __launch_bounds__(k_block) k_spmv_dot(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int which_x,
-                           int which_y, int which_w, int slot, int which_w2, int slot2) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    const double* x = outer_vec(S, which_x);
-    double* y = outer_vec(S, which_y);
-    const double* w = outer_vec(S, which_w);
-    double d1 = 0.0;
-    double d2 = 0.0;
-    if (a0_live<Csr>(S.a64, slice)) {
-        const double yi = a0_row<Csr>(S.a64, slice, lane, row, x);
-        if (row < S.n) {
-            y[row] = yi;
-            d1 = w[row] * yi;
-            if (Two) {
-                d2 = yi * outer_vec(S, which_w2)[row];
-            }
-        }
-    }
-    if (Two) {
-        double v[2] = {d1, d2};
-        double o[2];
-        block_sums<2>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[slot * S.nblk0 + bk_.y] = o[0];
-            S.partials[slot2 * S.nblk0 + bk_.y] = o[1];
-        }
-    } else {
-        double v[1] = {d1};
-        double o[1];
-        block_sums<1>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[slot * S.nblk0 + bk_.y] = o[0];
-        }
-    }
-}
-
-// x += alpha p; r -= alpha q; partial r.r. Jacobi CG also forms z = dinv r and r.z; the
-// mixed solver writes r32 = (float) r for the FP32 V-cycle.
 // Search directions alternate between two buffers: iteration k reads p_old = parity ? p : p2
 // and writes p_new = parity ? p2 : p (parity = k mod 2, iterations counted from 1).
 __device__ __forceinline__ double* p_old_of(const SysDev& S, int parity) { return (parity ^ S.flip) ? S.p : S.p2; }
 __device__ __forceinline__ double* p_new_of(const SysDev& S, int parity) { return (parity ^ S.flip) ? S.p2 : S.p; }
 
-// q = A p_new with p_new = z + beta p_old formed per gathered column (the reference's separate
-// p update, krylov_kernels.inc:293-296, folded into the next product; identical arithmetic),
-// p_new written for the own rows, and the partial p_new.q. z is the level-0 V-cycle output
-// v[z_buf] (which = 1, FP64 or FP32) or the Jacobi-preconditioned residual S.z (which = 0).
-template <class TZ, bool Csr>
-__global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int parity,
-                          int which, int z_buf) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    const EllView A0 = S.a64; // requested with the status (one wait)
-    if ((S.st->status != ST_RUNNING) | (A0.tpr <= 0)) {
-        return;
-    }
+// Step Op (beta), then q = A p_new with p_new = z + beta p_old formed per gathered column (the
+// reference's separate p update, krylov_kernels.inc:293-296, folded into the next product;
+// identical arithmetic), p_new written for the own rows, and the partial p_new.q. z is the level-0
+// V-cycle output v[z_buf] (which = 1, FP64 or FP32) or the Jacobi-preconditioned residual S.z
+// (which = 0).
+// At 128^3 (130 MB from memory in the mixed solve, whose matrix has left the Infinity Cache since the
+// last product) one chunk at a time takes 37.2 us and two 40.8: three arrays of loads a row fill the
+// wavefront's queue already. Before, with the step as a launch of its own: 36.4 + 8.9 us.
+template <class TZ, int Form, int Op>
+__global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int parity,
+                          int which, int z_buf, unsigned long long* __restrict__ report) {
+    CFDG_L0_PROLOGUE(sys, blocks)
     const auto z = gm(which == 0 ? reinterpret_cast<const TZ*>(S.z) : static_cast<const TZ*>(S.lv[0].v[z_buf]));
     const auto po = gm(static_cast<const double*>(p_old_of(S, parity)));
     const auto pn = gm(p_new_of(S, parity));
-    const double beta = S.st->beta;
-    double d = 0.0;
-    if (a0_live<Csr>(A0, slice)) {
-        const double qi = a0_row_f<Csr>(A0, slice, lane, row, [&](int c) {
-            return static_cast<double>(z[c]) + beta * po[c];
-        });
-        if (row < S.n) {
-            const double pi = static_cast<double>(z[row]) + beta * po[row];
-            pn[row] = pi;
-            gm(S.q)[row] = qi;
-            d = pi * qi;
+    const auto qv = gm(S.q);
+    const unsigned n = static_cast<unsigned>(S.n);
+    L0Op<Form, double, GatherPz<TZ>> A0(S.a64, {z, po, 0.0});
+    const Scalars st = take_step<Op>(S, first_, report, bk_.x);
+    if (st.status != ST_RUNNING) {
+        return;
+    }
+    A0.load.beta = st.beta;
+    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+        double y[2];
+        double pi[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { pi[h] = static_cast<double>(load_at<TZ>(z, r)) + st.beta * load_at<double>(po, r); });
+        l0_rows<H.value>(A0, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                store_at<double>(pn, row[h], pi[h]);
+                store_at<double>(qv, row[h], y[h]);
+                v[0] += pi[h] * y[h];
+            }
         }
-    }
-    double v[1] = {d};
-    double o[1];
-    block_sums<1>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_PQ * S.nblk0 + bk_.y] = o[0];
-    }
+    }, [](int) { return SLOT_PQ; });
 }
 
 // x = 0 for every system of a launch table (one launch for a whole batch).
-__global__ void __launch_bounds__(k_block) k_zero_x(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (row < S.n) {
-        gm(S.x)[row] = 0.0;
-    }
+__global__ void __launch_bounds__(k_block) k_zero_x(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    for_group_rows<false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int) {
+        const int row = slice * k_wave + lane;
+        if (row < S.n) {
+            gm(S.x)[row] = 0.0;
+        }
+    });
 }
 
+// Step FIN_ALPHA, then x += alpha p; r -= alpha q; partial r.r. Jacobi CG also forms z = dinv r and
+// r.z; the mixed solver writes r32 = (float) r for the FP32 V-cycle.
 template <int Mode> // 0 AMG FP64, 1 Jacobi CG, 2 mixed AMG
-__global__ void __launch_bounds__(k_block) k_update_xr(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int parity) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
+__global__ void __launch_bounds__(k_block) k_update_xr(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int parity) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto x = gm(S.x);
+    const auto r = gm(S.r);
+    const auto p = gm(static_cast<const double*>(p_new_of(S, parity)));
+    const auto qv = gm(static_cast<const double*>(S.q));
+    const auto z = gm(S.z);
+    const auto dinv = gm(S.dinv);
+    const auto r32 = gm(S.r32);
+    const int n = S.n;
+    const Scalars st = take_step<FIN_ALPHA>(S, first_, nullptr, 0);
+    if (st.status != ST_RUNNING) {
         return;
     }
-    const double alpha = S.st->alpha;
-    double rr = 0.0;
-    double rz = 0.0;
-    if (row < S.n) {
-        gm(S.x)[row] = gm(S.x)[row] + alpha * p_new_of(S, parity)[row];
-        const double ri = gm(S.r)[row] - alpha * gm(S.q)[row];
-        gm(S.r)[row] = ri;
-        rr = ri * ri;
-        if (Mode == 1) {
-            const double zi = ri * gm(S.dinv)[row];
-            gm(S.z)[row] = zi;
-            rz = ri * zi;
+    const double alpha = st.alpha;
+    constexpr int n_dots = Mode == 1 ? 2 : 1;
+    for_groups<n_dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[n_dots]) {
+        const int row = slice * k_wave + lane;
+        if (row < n) {
+            x[row] = x[row] + alpha * p[row];
+            const double ri = r[row] - alpha * qv[row];
+            r[row] = ri;
+            v[0] += ri * ri;
+            if constexpr (Mode == 1) {
+                const double zi = ri * dinv[row];
+                z[row] = zi;
+                v[1] += ri * zi;
+            }
+            if (Mode == 2) {
+                r32[row] = static_cast<float>(ri);
+            }
         }
-        if (Mode == 2) {
-            gm(S.r32)[row] = static_cast<float>(ri);
-        }
-    }
-    if (Mode == 1) {
-        double v[2] = {rr, rz};
-        double o[2];
-        block_sums<2>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-            S.partials[SLOT_RZ * S.nblk0 + bk_.y] = o[1];
-        }
-    } else {
-        double v[1] = {rr};
-        double o[1];
-        block_sums<1>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-        }
-    }
-}
-
-// p = z + beta p. which = 0: z is the Jacobi-preconditioned residual S.z (FP64); which = 1:
-// z is the level-0 V-cycle output v[z_buf] (FP64, or FP32 in the mixed solver).
-template <class TZ>
-__global__ void __launch_bounds__(k_block) k_p_update(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int which,
-                           int z_buf) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    const TZ* z = which == 0 ? reinterpret_cast<const TZ*>(S.z)
-                             : static_cast<const TZ*>(S.lv[0].v[z_buf]);
-    const double beta = S.st->beta;
-    if (row < S.n) {
-        gm(S.p)[row] = static_cast<double>(z[row]) + beta * gm(S.p)[row];
-    }
+    }, [](int q) { return q == 0 ? SLOT_RR : SLOT_RZ; });
 }
 
 // True residual |b - A x|^2 partials (always runs, after the solve).
-template <bool Csr>
-__global__ void __launch_bounds__(k_block) k_true_residual(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    double t = 0.0;
-    if (a0_live<Csr>(S.a64, slice)) {
-        const double ax = a0_row<Csr>(S.a64, slice, lane, row, S.x);
-        if (row < S.n) {
-            const double ri = gm(S.b)[row] - ax;
-            t = ri * ri;
+template <int Form>
+__global__ void __launch_bounds__(k_block) k_true_residual(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto b = gm(S.b);
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
+    const unsigned n = static_cast<unsigned>(S.n);
+    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+        double y[2];
+        double bi[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { bi[h] = load_at<double>(b, r); });
+        l0_rows<H.value>(A0, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                const double ri = bi[h] - y[h];
+                v[0] += ri * ri;
+            }
         }
-    }
-    double v[1] = {t};
-    double o[1];
-    block_sums<1>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_TRUE * S.nblk0 + bk_.y] = o[0];
-    }
+    }, [](int) { return SLOT_TRUE; });
 }
 
 // ------------------------------------------------------------------------------------------
-// BiCGStab kernels (krylov_kernels.inc:96-169)
+// BiCGStab kernels (krylov_kernels.inc:96-169): five launches an iteration
 // ------------------------------------------------------------------------------------------
 
 // r = b - A x; r0 = r; p = v = 0; partials r.r, b.b and r0.r.
-template <bool Csr>
-__global__ void __launch_bounds__(k_block) k_bicg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    double rr = 0.0;
-    double bb = 0.0;
-    if (a0_live<Csr>(S.a64, slice)) {
-        const double ax = a0_row<Csr>(S.a64, slice, lane, row, S.x);
+template <int Form>
+__global__ void __launch_bounds__(k_block) k_bicg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
+    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[3]) {
+        const int row = slice * k_wave + lane;
+        double y[2];
+        l0_rows<1>(A0, slice, 0, lane, y);
         if (row < S.n) {
             const double bi = gm(S.b)[row];
-            const double ri = bi - ax;
+            const double ri = bi - y[0];
             gm(S.r)[row] = ri;
-            S.r0[row] = ri;
+            gm(S.r0)[row] = ri;
             gm(S.p)[row] = 0.0;
             gm(S.v)[row] = 0.0;
-            rr = ri * ri;
-            bb = bi * bi;
+            v[0] += ri * ri;
+            v[1] += ri * ri;
+            v[2] += bi * bi;
         }
-    }
-    double v[2] = {rr, bb};
-    double o[2];
-    block_sums<2>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-        S.partials[SLOT_BB * S.nblk0 + bk_.y] = o[1];
-        S.partials[SLOT_R0R * S.nblk0 + bk_.y] = o[0];
-    }
+    }, [](int q) { return q == 0 ? SLOT_RR : q == 1 ? SLOT_R0R : SLOT_BB; });
 }
 
-// p = r + beta (p - omega v); ph = dinv p.
-__global__ void __launch_bounds__(k_block) k_bicg_p(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
+// Step FIN_BICG_RES (residual test, rho, beta), then p = r + beta (p - omega v); ph = dinv p.
+__global__ void __launch_bounds__(k_block) k_bicg_p(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb,
+                                                    unsigned long long* __restrict__ report) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto r = gm(static_cast<const double*>(S.r));
+    const auto vv = gm(static_cast<const double*>(S.v));
+    const auto dinv = gm(S.dinv);
+    const auto p = gm(S.p);
+    const auto ph = gm(S.ph);
+    const int n = S.n;
+    const Scalars st = take_step<FIN_BICG_RES>(S, first_, report, bk_.x);
+    if (st.status != ST_RUNNING) {
+        return;
+    }
+    const double beta = st.beta;
+    const double omega = st.omega;
+    for_group_rows<false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int) {
+        const int row = slice * k_wave + lane;
+        if (row < n) {
+            const double pi = r[row] + beta * (p[row] - omega * vv[row]);
+            p[row] = pi;
+            ph[row] = pi * dinv[row];
+        }
+    });
+}
+
+// v = A ph, partial r0.v.
+template <int Form>
+__global__ void __launch_bounds__(k_block) k_bicg_v(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto vv = gm(S.v);
+    const auto r0 = gm(static_cast<const double*>(S.r0));
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.ph))});
+    const unsigned n = static_cast<unsigned>(S.n);
     if (S.st->status != ST_RUNNING) {
         return;
     }
-    const double beta = S.st->beta;
-    const double omega = S.st->omega;
-    if (row < S.n) {
-        const double pi = gm(S.r)[row] + beta * (gm(S.p)[row] - omega * gm(S.v)[row]);
-        gm(S.p)[row] = pi;
-        gm(S.ph)[row] = pi * gm(S.dinv)[row];
-    }
+    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+        double y[2];
+        double ri[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { ri[h] = load_at<double>(r0, r); });
+        l0_rows<H.value>(A0, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                store_at<double>(vv, row[h], y[h]);
+                v[0] += ri[h] * y[h];
+            }
+        }
+    }, [](int) { return SLOT_R0V; });
 }
 
-// s = r - alpha v; sh = dinv s; partial s.s.
-__global__ void __launch_bounds__(k_block) k_bicg_s(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
+// Step FIN_BICG_ALPHA, then s = r - alpha v; sh = dinv s; partial s.s.
+__global__ void __launch_bounds__(k_block) k_bicg_s(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto r = gm(static_cast<const double*>(S.r));
+    const auto vv = gm(static_cast<const double*>(S.v));
+    const auto dinv = gm(S.dinv);
+    const auto sv = gm(S.s);
+    const auto sh = gm(S.sh);
+    const int n = S.n;
+    const Scalars st = take_step<FIN_BICG_ALPHA>(S, first_, nullptr, 0);
+    if (st.status != ST_RUNNING) {
         return;
     }
-    const double alpha = S.st->alpha;
-    double ss = 0.0;
-    if (row < S.n) {
-        const double si = gm(S.r)[row] - alpha * gm(S.v)[row];
-        S.s[row] = si;
-        gm(S.sh)[row] = si * gm(S.dinv)[row];
-        ss = si * si;
-    }
-    double v[1] = {ss};
-    double o[1];
-    block_sums<1>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_SS * S.nblk0 + bk_.y] = o[0];
-    }
+    const double alpha = st.alpha;
+    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[1]) {
+        const int row = slice * k_wave + lane;
+        if (row < n) {
+            const double si = r[row] - alpha * vv[row];
+            sv[row] = si;
+            sh[row] = si * dinv[row];
+            v[0] += si * si;
+        }
+    }, [](int) { return SLOT_SS; });
 }
 
-// Early exit of BiCGStab: x += alpha ph (status ST_CONVERGED_PENDING only).
-__global__ void __launch_bounds__(k_block) k_bicg_early_x(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_CONVERGED_PENDING) {
+// Step FIN_BICG_S, then t = A sh with the partials t.t and t.s, or on the early exit x += alpha ph.
+template <int Form>
+__global__ void __launch_bounds__(k_block) k_bicg_t(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto tv = gm(S.t);
+    const auto sv = gm(static_cast<const double*>(S.s));
+    const auto x = gm(S.x);
+    const auto ph = gm(static_cast<const double*>(S.ph));
+    const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.sh))});
+    const unsigned n = static_cast<unsigned>(S.n);
+    const Scalars st = take_step<FIN_BICG_S>(S, first_, nullptr, 0);
+    if (st.status == ST_CONVERGED_PENDING) {
+        for_group_rows<false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int) {
+            const int row = slice * k_wave + lane;
+            if (row < n) {
+                x[row] = x[row] + st.alpha * ph[row];
+            }
+        });
         return;
     }
-    if (row < S.n) {
-        gm(S.x)[row] = gm(S.x)[row] + S.st->alpha * gm(S.ph)[row];
+    if (st.status != ST_RUNNING) {
+        return;
     }
+    for_groups<2, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2]) {
+        double y[2];
+        double si[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { si[h] = load_at<double>(sv, r); });
+        l0_rows<H.value>(A0, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                store_at<double>(tv, row[h], y[h]);
+                v[0] += y[h] * y[h];
+                v[1] += y[h] * si[h];
+            }
+        }
+    }, [](int q) { return q == 0 ? SLOT_TT : SLOT_TS; });
 }
 
-// x += alpha ph + omega sh; r = s - omega t; partials r.r and r0.r.
-__global__ void __launch_bounds__(k_block) k_bicg_xr(const SysDev* __restrict__ sys, const int2* __restrict__ blocks) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
+// Step FIN_BICG_OMEGA, then x += alpha ph + omega sh; r = s - omega t; partials r.r and r0.r.
+__global__ void __launch_bounds__(k_block) k_bicg_xr(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const auto x = gm(S.x);
+    const auto r = gm(S.r);
+    const auto ph = gm(static_cast<const double*>(S.ph));
+    const auto sh = gm(static_cast<const double*>(S.sh));
+    const auto sv = gm(static_cast<const double*>(S.s));
+    const auto tv = gm(static_cast<const double*>(S.t));
+    const auto r0 = gm(static_cast<const double*>(S.r0));
+    const int n = S.n;
+    const Scalars st = take_step<FIN_BICG_OMEGA>(S, first_, nullptr, 0);
+    if (st.status != ST_RUNNING) {
         return;
     }
-    const double alpha = S.st->alpha;
-    const double omega = S.st->omega;
-    double rr = 0.0;
-    double r0r = 0.0;
-    if (row < S.n) {
-        gm(S.x)[row] = gm(S.x)[row] + (alpha * gm(S.ph)[row] + omega * gm(S.sh)[row]);
-        const double ri = S.s[row] - omega * S.t[row];
-        gm(S.r)[row] = ri;
-        rr = ri * ri;
-        r0r = S.r0[row] * ri;
-    }
-    double v[2] = {rr, r0r};
-    double o[2];
-    block_sums<2>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_RR * S.nblk0 + bk_.y] = o[0];
-        S.partials[SLOT_R0R * S.nblk0 + bk_.y] = o[1];
-    }
+    const double alpha = st.alpha;
+    const double omega = st.omega;
+    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2]) {
+        const int row = slice * k_wave + lane;
+        if (row < n) {
+            x[row] = x[row] + (alpha * ph[row] + omega * sh[row]);
+            const double ri = sv[row] - omega * tv[row];
+            r[row] = ri;
+            v[0] += ri * ri;
+            v[1] += r0[row] * ri;
+        }
+    }, [](int q) { return q == 0 ? SLOT_RR : SLOT_R0R; });
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1054,23 +1571,6 @@ __global__ void __launch_bounds__(k_block) k_bicg_xr(const SysDev* __restrict__ 
     const int row = bk_.y * (k_block / tpr) + static_cast<int>(threadIdx.x) / tpr;                \
     const int sub = static_cast<int>(threadIdx.x) & (tpr - 1);                                    \
     (void)sub;
-
-// First two Jacobi sweeps from x = 0: v[out] = x1 + (f2 wd) (b - A x1), x1 = (f1 wd) b
-// (sliced-ELL operators; the gathers of wd and b stay cache-resident for short rows). f1, f2:
-// the sweeps' factors on the level's damping (Chebyshev weights; 1 for plain damped Jacobi,
-// which leaves the arithmetic unchanged).
-template <class T>
-__global__ void __launch_bounds__(k_block) k_presmooth2(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int level, int out,
-                                                        T f1, T f2) {
-    CFDG_LEVEL_PROLOGUE(sys, blocks, level, a)
-    const auto b = gm(static_cast<const T*>(L.b));
-    const auto wd = gm(static_cast<const T*>(L.wd));
-    const T ax = mat_row_x1<T>(M, row, sub, wd, b, f1);
-    if (sub == 0 && row < L.n) {
-        const T x1 = (f1 * wd[row]) * b[row];
-        gm(static_cast<T*>(L.v[out]))[row] = x1 + (f2 * wd[row]) * (b[row] - ax);
-    }
-}
 
 // ------------------------------------------------------------------------------------------
 // V-cycle operations on one row (or one lane of a row's group), used by the level kernels below.
@@ -1191,126 +1691,174 @@ __global__ void __launch_bounds__(k_block) k_zero_level(const SysDev* __restrict
     gm(static_cast<T*>(L.v[out]))[row] = T(0);
 }
 
-// Jacobi sweep v[out] = v[in] + (f wd) (b - A v[in]). Dots (level 0 only, sliced ELL): 0 none;
-// 1 partial r.z with r = b (FP64 level 0, where b aliases r); 2 partials r.z and z.q with r, q
-// the FP64 outer vectors (mixed level 0).
-template <class T, int Dots>
+// Jacobi sweep v[out] = v[in] + (f wd) (b - A v[in]).
+template <class T>
 __global__ void __launch_bounds__(k_block) k_jacobi(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int level, int in, int out,
                                                     T f) {
     CFDG_LEVEL_PROLOGUE(sys, blocks, level, a)
-    const T z = op_jacobi<T>(L, M, row, sub, in, out, f);
-    double d1 = 0.0;
-    double d2 = 0.0;
-    if (Dots != 0 && sub == 0 && row < L.n) {
-        if (Dots == 1) {
-            d1 = static_cast<double>(gm(static_cast<const T*>(L.b))[row]) * static_cast<double>(z);
-        }
-        if (Dots == 2) {
-            const double zd = static_cast<double>(z);
-            d1 = gm(S.r)[row] * zd;
-            d2 = zd * gm(S.q)[row];
-        }
-    }
-    if (Dots == 1) {
-        double v[1] = {d1};
-        double o[1];
-        block_sums<1>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[SLOT_RZ * S.nblk0 + bk_.y] = o[0];
-        }
-    }
-    if (Dots == 2) {
-        double v[2] = {d1, d2};
-        double o[2];
-        block_sums<2>(v, o);
-        if (threadIdx.x == 0) {
-            S.partials[SLOT_RZ * S.nblk0 + bk_.y] = o[0];
-            S.partials[SLOT_ZQ * S.nblk0 + bk_.y] = o[1];
-        }
+    (void)op_jacobi<T>(L, M, row, sub, in, out, f);
+}
+
+// ------------------------------------------------------------------------------------------
+// Level-0 V-cycle kernels over row groups (the finest operator is sliced ELL, one lane per row)
+// ------------------------------------------------------------------------------------------
+
+// State of the cycle's first kernel: step FIN_RES made here (Step), or made by a launch before it.
+template <bool Step>
+__device__ __forceinline__ bool cycle_runs(const SysDev& S, bool first, unsigned long long* report, int id) {
+    if constexpr (Step) {
+        return take_step<FIN_RES>(S, first, report, id).status == ST_RUNNING;
+    } else {
+        return S.st->status == ST_RUNNING;
     }
 }
 
-// Level-0 FP32 post-sweep with two slices per wavefront (the finest operator is sliced ELL with
-// one lane per row): a workgroup of k_block_pair threads covers the same 256 rows as a k_block
-// one, wave w serving slices 4 y + 2 w and 4 y + 2 w + 1, so every table entry keeps its meaning.
-// Each row is computed as in k_jacobi and the block partials add the four slices' wavefront sums
-// in slice order: the results are bit-identical to k_jacobi's.
-constexpr int k_block_pair = k_block / 2;
+// v[out] = b - A x1 with x1 = (f wd) b, the single Jacobi sweep from zero, formed per gathered
+// column instead of stored (one pre-sweep per side).
+// 16.0 us at 128^3 in FP32 with the step (before: 17.4 and 5.2 for the step's launch).
+template <class T, int Form, bool Step>
+__global__ void __launch_bounds__(k_block) k_l0_residual_x1(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int out,
+                                                            T f, unsigned long long* __restrict__ report) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const LevelDev& L = S.lv[0];
+    const auto b = gm(static_cast<const T*>(L.b));
+    const auto t = gm(static_cast<T*>(L.v[out]));
+    const L0Op<Form, T, GatherX1<T>> M(L.a, {gm(static_cast<const T*>(L.wd)), b, f});
+    const unsigned n = static_cast<unsigned>(L.n);
+    if (!cycle_runs<Step>(S, first_, report, bk_.x) | (L.coarsest != 0)) {
+        return;
+    }
+    for_group_rows<true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds) {
+        T y[2];
+        T bi[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { bi[h] = load_at<T>(b, r); });
+        l0_rows<H.value>(M, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                store_at<T>(t, row[h], bi[h] - y[h]);
+            }
+        }
+    });
+}
 
-#define CFDG_PAIR_PROLOGUE(sysarr, blocks, level)                                                 \
-    const int2 bk_ = block_entry(blocks);                                                         \
-    const SysDev& S = (sysarr)[bk_.x];                                                            \
-    const LevelDev& L = S.lv[level];                                                              \
-    const EllView M = L.a;                                                                        \
-    if ((S.st->status != ST_RUNNING) | (L.coarsest != 0) | (M.tpr <= 0)) {                        \
-        return;                                                                                   \
-    }                                                                                             \
-    const int lane = static_cast<int>(threadIdx.x) % k_wave;                                      \
-    const int wave_ = static_cast<int>(threadIdx.x) / k_wave;                                     \
-    const int s0 = bk_.y * k_slices_per_block + 2 * wave_;                                        \
-    const int row0 = s0 * k_wave + lane;                                                          \
-    const int row1 = row0 + k_wave;
-
-// Jacobi sweep v[out] = v[in] + (f wd) (b - A v[in]) of level 0 with the partial dots of k_jacobi.
-template <class T, int Dots>
-__global__ void __launch_bounds__(k_block_pair) k_jacobi_pair(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int level, int in,
-                                                              int out, T f) {
-    CFDG_PAIR_PROLOGUE(sys, blocks, level)
-    const T* x = static_cast<const T*>(L.v[in]);
-    const auto gx = gm(x);
+// First two Jacobi sweeps from x = 0: v[out] = x1 + (f2 wd) (b - A x1), x1 = (f1 wd) b (the gathers
+// of wd and b stay cache-resident for short rows). f1, f2: the sweeps' factors on the level's
+// damping (Chebyshev weights; 1 for plain damped Jacobi, which leaves the arithmetic unchanged).
+template <class T, int Form, bool Step>
+__global__ void __launch_bounds__(k_block) k_l0_presmooth2(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int out,
+                                                           T f1, T f2, unsigned long long* __restrict__ report) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const LevelDev& L = S.lv[0];
     const auto b = gm(static_cast<const T*>(L.b));
     const auto wd = gm(static_cast<const T*>(L.wd));
-    T ya;
-    T yb;
-    ell_row_pair<T>(M, s0, lane, [&](int c) { return gx[c]; }, ya, yb);
-    const auto o = gm(static_cast<T*>(L.v[out]));
-    double d1[2] = {0.0, 0.0};
-    double d2[2] = {0.0, 0.0};
-    const int rows[2] = {row0, row1};
-    const T ys[2] = {ya, yb};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int row = rows[h];
-        if (row < L.n) {
-            const T z = gx[row] + (f * wd[row]) * (b[row] - ys[h]);
-            o[row] = z;
-            if (Dots == 1) {
-                d1[h] = static_cast<double>(b[row]) * static_cast<double>(z);
-            }
-            if (Dots == 2) {
-                const double zd = static_cast<double>(z);
-                d1[h] = gm(S.r)[row] * zd;
-                d2[h] = zd * gm(S.q)[row];
-            }
-        }
+    const auto x = gm(static_cast<T*>(L.v[out]));
+    const L0Op<Form, T, GatherX1<T>> M(L.a, {wd, b, f1});
+    const unsigned n = static_cast<unsigned>(L.n);
+    if (!cycle_runs<Step>(S, first_, report, bk_.x) | (L.coarsest != 0)) {
+        return;
     }
-    if (Dots != 0) {
-        __shared__ double red[2][k_slices_per_block];
+    for_group_rows<true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds) {
+        T y[2];
+        T bi[2];
+        T wi[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) {
+            bi[h] = load_at<T>(b, r);
+            wi[h] = load_at<T>(wd, r);
+        });
+        l0_rows<H.value>(M, slice, ds, lane, y);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const double w1 = wave_sum(d1[h]);
-            const double w2 = Dots == 2 ? wave_sum(d2[h]) : 0.0;
-            if (lane == 0) {
-                red[0][2 * wave_ + h] = w1;
-                red[1][2 * wave_ + h] = w2;
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                const T x1 = (f1 * wi[h]) * bi[h];
+                store_at<T>(x, row[h], x1 + (f2 * wi[h]) * (bi[h] - y[h]));
             }
         }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t1 = red[0][0];
-            double t2 = red[1][0];
-#pragma unroll
-            for (int w = 1; w < k_slices_per_block; ++w) {
-                t1 += red[0][w];
-                t2 += red[1][w];
-            }
-            S.partials[SLOT_RZ * S.nblk0 + bk_.y] = t1;
-            if (Dots == 2) {
-                S.partials[SLOT_ZQ * S.nblk0 + bk_.y] = t2;
-            }
-        }
-    }
+    });
 }
+
+// The last post-sweep v[out] = v[in] + (f wd) (b - A v[in]) with the dot products of its result:
+// Dots 1 partial r.z with r = b (FP64 level 0, where b aliases r); 2 partials r.z and z.q with r, q
+// the FP64 outer vectors (mixed level 0). Pair: two chunks' rows at a time (the same results bit
+// for bit; slower on BF16 rows).
+template <class T, int Form, int Dots, bool Pair>
+__global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int in, int out,
+                                                       T f) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    const LevelDev& L = S.lv[0];
+    const auto x = gm(static_cast<const T*>(L.v[in]));
+    const auto b = gm(static_cast<const T*>(L.b));
+    const auto wd = gm(static_cast<const T*>(L.wd));
+    const auto o = gm(static_cast<T*>(L.v[out]));
+    const auto r = gm(static_cast<const double*>(S.r));
+    const auto qv = gm(static_cast<const double*>(S.q));
+    const L0Op<Form, T, GatherX<T>> M(L.a, {x});
+    const unsigned n = static_cast<unsigned>(L.n);
+    if ((S.st->status != ST_RUNNING) | (L.coarsest != 0)) {
+        return;
+    }
+    for_groups<Dots, Pair>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[Dots]) {
+        T y[2];
+        T bi[2];
+        T wi[2];
+        T xi[2];
+        double ri[2];
+        double qi[2];
+        unsigned row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned i) {
+            bi[h] = load_at<T>(b, i);
+            wi[h] = load_at<T>(wd, i);
+            xi[h] = load_at<T>(x, i);
+            if constexpr (Dots == 2) {
+                ri[h] = load_at<double>(r, i);
+                qi[h] = load_at<double>(qv, i);
+            }
+        });
+        l0_rows<H.value>(M, slice, ds, lane, y);
+#pragma unroll
+        for (int h = 0; h < H.value; ++h) {
+            if (row[h] < n) {
+                const T z = xi[h] + (f * wi[h]) * (bi[h] - y[h]);
+                store_at<T>(o, row[h], z);
+                const double zd = static_cast<double>(z);
+                if constexpr (Dots == 1) {
+                    v[0] += static_cast<double>(bi[h]) * zd;
+                } else {
+                    v[0] += ri[h] * zd;
+                    v[1] += zd * qi[h];
+                }
+            }
+        }
+    }, [](int q) { return q == 0 ? SLOT_RZ : SLOT_ZQ; });
+}
+
+// Level-0 dot products from a finished V-cycle output v[buf] (used when no Jacobi sweep on
+// level 0 could carry them: one-level hierarchies and smoothing-free cycles).
+template <class T, int Dots>
+__global__ void __launch_bounds__(k_block) k_level0_dots(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int buf) {
+    CFDG_L0_PROLOGUE(sys, blocks)
+    if (S.st->status != ST_RUNNING) {
+        return;
+    }
+    const LevelDev& L = S.lv[0];
+    for_groups<Dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[Dots]) {
+        const int row = slice * k_wave + lane;
+        if (row < S.n) {
+            const double z = static_cast<double>(static_cast<const T*>(L.v[buf])[row]);
+            if constexpr (Dots == 1) {
+                v[0] += static_cast<double>(static_cast<const T*>(L.b)[row]) * z;
+            } else {
+                v[0] += S.r[row] * z;
+                v[1] += z * S.q[row];
+            }
+        }
+    }, [](int q) { return q == 0 ? SLOT_RZ : SLOT_ZQ; });
+}
+
+// Workgroup of the level kernels that serve two slices per wavefront.
+constexpr int k_block_pair = k_block / 2;
 
 // Rows of one table entry (the 256 / tpr rows a k_block workgroup covers) for a k_block_pair
 // workgroup: sliced ELL reads slices 4 y + 2 w and 4 y + 2 w + 1 together in wave w; CSR rows run
@@ -1326,7 +1874,7 @@ __device__ __forceinline__ void pair_rows(const EllView& m, int y, F load, E epi
         const int s0 = y * k_slices_per_block + 2 * (static_cast<int>(threadIdx.x) / k_wave);
         T ya;
         T yb;
-        ell_row_pair<T>(m, s0, lane, load, ya, yb);
+        ell_row_pair<T>(m, s0, 1, lane, load, ya, yb);
         if (tpr > 1) {
             ya = group_sum(ya, tpr);
             yb = group_sum(yb, tpr);
@@ -1366,7 +1914,7 @@ __global__ void __launch_bounds__(k_block_pair) k_prolong_pair(const SysDev* __r
     const LevelDev& N = S.lv[level + 1];
     const auto e = gm(static_cast<const T*>(N.v[coarse_buf]));
     const auto x = gm(static_cast<T*>(L.v[io]));
-    pair_rows<T>(L.p, bk_.y, [&](int c) { return e[c]; }, [&](int row, int sub, T t) {
+    pair_rows<T>(L.p, bk_.y, GatherX<T>{e}, [&](int row, int sub, T t) {
         if (sub == 0 && row < L.n) {
             if constexpr (X1) {
                 x[row] = (f * gm(static_cast<const T*>(L.wd))[row]) * gm(static_cast<const T*>(L.b))[row] + t;
@@ -1439,267 +1987,6 @@ __global__ void __launch_bounds__(k_block) k_coarse(const SysDev* __restrict__ s
 }
 
 // ------------------------------------------------------------------------------------------
-// Finalize kernels: one workgroup per system, partials added in a fixed order.
-// ------------------------------------------------------------------------------------------
-constexpr int k_fin_block = 1024;
-
-__device__ __forceinline__ double reduce_slot(const SysDev& S, int slot) {
-    __shared__ double red[k_fin_block / k_wave];
-    const double* p = S.partials + static_cast<long long>(slot) * S.nblk0;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < S.nblk0; i += k_fin_block) {
-        s += p[i];
-    }
-    s = wave_sum(s);
-    if (threadIdx.x % k_wave == 0) {
-        red[threadIdx.x / k_wave] = s;
-    }
-    __syncthreads();
-    double t = red[0];
-#pragma unroll
-    for (int w = 1; w < k_fin_block / k_wave; ++w) {
-        t += red[w];
-    }
-    __syncthreads();
-    return t;
-}
-
-enum FinOp : int {
-    FIN_AMG_INIT = 0,   // res0, |b|; converged before iterating?
-    FIN_ALPHA = 1,      // pq; breakdown if 0; alpha = rz / pq
-    FIN_RES = 2,        // res; converged?
-    FIN_BETA = 3,       // rz_new; beta = rz_new / rz (0 first); it++ / limit
-    FIN_BETA_FLEX = 4,  // rz_new, zq; beta = -zq / pq (0 first); it++ / limit
-    FIN_CG_INIT = 5,    // Jacobi CG start: res0, |b|, rz; beta = 0; it = 1
-    FIN_CG_RES_BETA = 6,// Jacobi CG: res check then beta
-    FIN_TRUE = 7,       // true residual
-    FIN_BICG_INIT = 8,
-    FIN_BICG_ALPHA = 10,
-    FIN_BICG_S = 11,
-    FIN_BICG_OMEGA = 12,
-    FIN_BICG_RES = 13
-};
-
-// Start of a BiCGStab iteration (krylov_kernels.inc:96-169): rho_new = r0.r (kept in rz), the
-// iteration limit, the breakdown guards rho_new == 0 and omega == 0, and beta. Run by thread 0 of
-// the finalize that ends the previous step (the start-up or the previous iteration's residual),
-// so an iteration needs no launch of its own for it.
-__device__ __forceinline__ void bicg_rho(SolveState* st) {
-    const double rho_new = st->rz;
-    if (st->it > st->max_it) {
-        st->status = ST_MAXIT;
-    } else if (rho_new == 0.0 || st->omega == 0.0) {
-        st->status = ST_BREAKDOWN;
-    } else {
-        st->beta = (rho_new / st->rho) * (st->alpha / st->omega);
-        st->rho = rho_new;
-    }
-}
-
-template <int Op>
-__device__ __forceinline__ void finalize_step(const SysDev& S) {
-    SolveState* st = S.st;
-    const int status = st->status;
-    if (Op == FIN_TRUE) {
-        const double t = reduce_slot(S, SLOT_TRUE);
-        if (threadIdx.x == 0) {
-            st->true_res = sqrt(t);
-        }
-        return;
-    }
-    if (status != ST_RUNNING && !(Op == FIN_BICG_OMEGA && status == ST_CONVERGED_PENDING)) {
-        return;
-    }
-    if (Op == FIN_AMG_INIT || Op == FIN_CG_INIT || Op == FIN_BICG_INIT) {
-        const double rr = reduce_slot(S, SLOT_RR);
-        const double bb = reduce_slot(S, SLOT_BB);
-        double rz = 0.0;
-        if (Op == FIN_CG_INIT) {
-            rz = reduce_slot(S, SLOT_RZ);
-        }
-        double r0r = 0.0;
-        if (Op == FIN_BICG_INIT) {
-            r0r = reduce_slot(S, SLOT_R0R);
-        }
-        if (threadIdx.x == 0) {
-            const double res = sqrt(rr);
-            st->res = res;
-            st->bnorm = sqrt(bb);
-            st->it = 0;
-            if (res <= st->tol) {
-                st->status = ST_CONVERGED;
-            } else if (Op == FIN_CG_INIT) {
-                st->rz = rz;
-                st->beta = 0.0;
-                st->it = 1;
-                if (st->it > st->max_it) {
-                    st->status = ST_MAXIT;
-                }
-            } else if (Op == FIN_BICG_INIT) {
-                st->rho = 1.0;
-                st->alpha = 1.0;
-                st->omega = 1.0;
-                st->rz = r0r; // rho_new of the first iteration
-                st->it = 1;
-                bicg_rho(st);
-            }
-        }
-        return;
-    }
-    if (Op == FIN_ALPHA) {
-        const double pq = reduce_slot(S, SLOT_PQ);
-        if (threadIdx.x == 0) {
-            st->pq = pq;
-            if (pq == 0.0) {
-                st->status = ST_BREAKDOWN;
-            } else {
-                st->alpha = st->rz / pq;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_RES) {
-        const double rr = reduce_slot(S, SLOT_RR);
-        if (threadIdx.x == 0) {
-            const double res = sqrt(rr);
-            st->res = res;
-            if (res <= st->tol) {
-                st->status = ST_CONVERGED;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_BETA || Op == FIN_BETA_FLEX) {
-        const double rz_new = reduce_slot(S, SLOT_RZ);
-        double zq = 0.0;
-        if (Op == FIN_BETA_FLEX) {
-            zq = reduce_slot(S, SLOT_ZQ);
-        }
-        if (threadIdx.x == 0) {
-            if (st->it == 0) {
-                st->beta = 0.0;
-            } else if (Op == FIN_BETA) {
-                st->beta = rz_new / st->rz;
-            } else {
-                st->beta = -zq / st->pq;
-            }
-            st->rz = rz_new;
-            st->it += 1;
-            if (st->it > st->max_it) {
-                st->status = ST_MAXIT;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_CG_RES_BETA) {
-        const double rr = reduce_slot(S, SLOT_RR);
-        const double rz_new = reduce_slot(S, SLOT_RZ);
-        if (threadIdx.x == 0) {
-            const double res = sqrt(rr);
-            st->res = res;
-            if (res <= st->tol) {
-                st->status = ST_CONVERGED;
-            } else {
-                st->beta = rz_new / st->rz;
-                st->rz = rz_new;
-                st->it += 1;
-                if (st->it > st->max_it) {
-                    st->status = ST_MAXIT;
-                }
-            }
-        }
-        return;
-    }
-    if (Op == FIN_BICG_ALPHA) {
-        const double r0v = reduce_slot(S, SLOT_R0V);
-        if (threadIdx.x == 0) {
-            if (r0v == 0.0) {
-                st->status = ST_BREAKDOWN;
-            } else {
-                st->alpha = st->rho / r0v;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_BICG_S) {
-        const double ss = reduce_slot(S, SLOT_SS);
-        if (threadIdx.x == 0) {
-            const double s_norm = sqrt(ss);
-            if (s_norm <= st->tol) {
-                st->res = s_norm;
-                st->status = ST_CONVERGED_PENDING;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_BICG_OMEGA) {
-        const double tt = reduce_slot(S, SLOT_TT);
-        const double ts = reduce_slot(S, SLOT_TS);
-        if (threadIdx.x == 0) {
-            if (status == ST_CONVERGED_PENDING) {
-                st->status = ST_CONVERGED;
-            } else {
-                st->omega = tt > 0.0 ? ts / tt : 0.0;
-            }
-        }
-        return;
-    }
-    if (Op == FIN_BICG_RES) {
-        const double rr = reduce_slot(S, SLOT_RR);
-        const double r0r = reduce_slot(S, SLOT_R0R);
-        if (threadIdx.x == 0) {
-            const double res = sqrt(rr);
-            st->res = res;
-            if (res <= st->tol) {
-                st->status = ST_CONVERGED;
-            } else {
-                st->rz = r0r;
-                st->it += 1;
-                bicg_rho(st);
-            }
-        }
-        return;
-    }
-}
-
-// A system's progress as one 64-bit word, so that a host that polls it never sees half a report:
-// the residual (FP32 bits) above, the number of finished iterations and the status below. The word
-// goes to host-mapped memory at the end of every iteration; the host reads it while later
-// iterations are queued, without an event (an event record between two graph launches costs 4 us).
-__device__ __forceinline__ unsigned long long report_word(const SolveState* st, int done) {
-    const unsigned low = (static_cast<unsigned>(done) << k_report_status_bits) | static_cast<unsigned>(st->status);
-    return (static_cast<unsigned long long>(__float_as_uint(static_cast<float>(st->res))) << 32) | low;
-}
-
-// Iterations finished when the step Op has run (st->it is already the next one after a residual
-// step that goes on, except in AMG-PCG, whose beta step counts).
-template <int Op>
-__device__ __forceinline__ int iterations_done(const SolveState* st) {
-    if (Op == FIN_AMG_INIT || Op == FIN_CG_INIT || Op == FIN_BICG_INIT) {
-        return 0;
-    }
-    if (Op == FIN_CG_RES_BETA || Op == FIN_BICG_RES) {
-        return st->status == ST_RUNNING ? st->it - 1 : st->it;
-    }
-    return st->it;
-}
-
-// One workgroup per system (ids: descriptor indices). With report, the system's report word after
-// the step is also stored at report[id]: the last step of an iteration tells the host every
-// system's state this way, with no launch of its own.
-template <int Op>
-__global__ void __launch_bounds__(k_fin_block) k_finalize(const SysDev* __restrict__ sys, const int* __restrict__ ids,
-                                                         unsigned long long* __restrict__ report) {
-    const int id = ids[blockIdx.x];
-    finalize_step<Op>(sys[id]);
-    if (report != nullptr && threadIdx.x == 0) { // thread 0 wrote the state
-        const SolveState* st = sys[id].st;
-        __hip_atomic_store(report + id, report_word(st, iterations_done<Op>(st)), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-}
-
-// ------------------------------------------------------------------------------------------
 // Normalised residual (ldu_matrix.cpp:65-103): res = sum_c |b_c - (Ax)_c| and
 // norm = sum_c |(Ax)_c - (A xref)_c| + |b_c - (A xref)_c|, with A xref = rowsum(A) * mean(x).
 // Three passes with fixed-order sums: block sums of x, their total, then per row the two terms
@@ -1727,7 +2014,7 @@ __global__ void __launch_bounds__(k_block) k_nr_rows(EllView a, int n, const dou
     double t[3] = {0.0, 0.0, 0.0};
     if (slice < a.n_slices) {
         const double ax = ell_row<double>(a, slice, lane, x);
-        const double rs = ell_row_f<double>(a, slice, lane, [](int) { return 1.0; });
+        const double rs = ell_row_f<double>(a, slice, lane, GatherOne{});
         if (row < n) {
             const double bi = b[row];
             const double ax_ref = rs * mean;
@@ -1745,6 +2032,8 @@ __global__ void __launch_bounds__(k_block) k_nr_rows(EllView a, int n, const dou
         part[2 * nblk + blockIdx.x] = o[2];
     }
 }
+
+constexpr int k_fin_block = 1024;
 
 // out[q] = sum over i < nblk of part[q nblk + i], q < count, in a fixed order (one workgroup).
 __global__ void __launch_bounds__(k_fin_block) k_nr_reduce(const double* __restrict__ part, int nblk, int count,

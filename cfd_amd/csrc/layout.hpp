@@ -39,6 +39,19 @@ enum Status : int {
 constexpr int k_report_status_bits = 4;
 constexpr unsigned k_report_none = 15; // status of a word that no step has written yet
 
+constexpr int k_states = 4;        // copies of a system's state (kernels.hpp, take_step)
+constexpr int k_max_groups = 1024; // row groups (partial sums per dot product) of a system
+
+// 256-row chunks of a system's row groups, and the number of groups.
+constexpr int group_chunks(int n) { return ((n + k_block - 1) / k_block + k_max_groups - 1) / k_max_groups; }
+constexpr int group_count(int n) {
+    return ((n + k_block - 1) / k_block + group_chunks(n) - 1) / group_chunks(n);
+}
+
+// Groups of a segment (kernels.hpp: the groups of a segment take its chunks in turn).
+constexpr int k_xcds = 8;
+constexpr int group_segment(int n) { return (group_count(n) + k_xcds - 1) / k_xcds; }
+
 struct SolveState {
     double tol;
     double rz;
@@ -73,10 +86,11 @@ struct SolveState {
 // slices; tpr == 1 only).
 // Symmetric stencil storage (sym_w > 0; square, exactly symmetric, tpr == 1): one stencil of
 // sym_n offsets for all rows, soff = [offsets ascending | stored slot of each], and only the
-// entries with offset >= 0 stored: sym_w slots per row, slice s holding rows 64 s .. 64 s + 63
-// at val[s sym_w 64 + j 64 + lane] for the j-th offset >= 0. An entry with offset o < 0 is read
-// from row + o's stored slot of -o (a_ij = a_ji); a row's entries are summed in offset order,
-// the order (and result) of the per-slice stencil layout.
+// entries with offset >= 0 stored: sym_w slots per row, one array of n_slices * 64 rows for each
+// offset, row r's j-th offset >= 0 at val[j n_slices 64 + r]. An entry with offset o < 0 is read
+// from row + o's stored slot of -o (a_ij = a_ji), so that every entry of a row is at a distance
+// from the row that is the same for all rows; a row's entries are summed in offset order, the order
+// (and result) of the per-slice stencil layout.
 struct EllView {
     int n_rows;
     int tpr;
@@ -111,9 +125,11 @@ struct LevelDev {
 };
 
 struct SysDev {
-    SolveState* st;
-    double* partials; // k_slots * nblk0
-    int nblk0;        // 256-row blocks of level 0
+    SolveState* st;   // k_states copies; st[0] is the solve's result
+    double* partials; // k_slots * n_groups
+    int n_groups;     // group_count(n)
+    int chunks;       // group_chunks(n)
+    int segment;      // group_segment(n)
     int n;
     int n_levels;
     int flip;               // XOR on the launch's iteration parity: 0 unless the system joined

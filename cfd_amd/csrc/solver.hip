@@ -335,37 +335,6 @@ double mixed_weight(double h, double w_ref) {
 }
 
 
-// Level-0 dot products from a finished V-cycle output v[buf] (used when no Jacobi sweep on
-// level 0 could carry them: one-level hierarchies and smoothing-free cycles).
-template <class T, int Dots>
-__global__ void __launch_bounds__(k_block) k_level0_dots(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int buf) {
-    CFDG_BLOCK_PROLOGUE(sys, blocks)
-    if (S.st->status != ST_RUNNING) {
-        return;
-    }
-    const LevelDev& L = S.lv[0];
-    double d1 = 0.0;
-    double d2 = 0.0;
-    if (row < S.n) {
-        const double z = static_cast<double>(static_cast<const T*>(L.v[buf])[row]);
-        if (Dots == 1) {
-            d1 = static_cast<double>(static_cast<const T*>(L.b)[row]) * z;
-        } else {
-            d1 = S.r[row] * z;
-            d2 = z * S.q[row];
-        }
-    }
-    double v[2] = {d1, d2};
-    double o[2];
-    block_sums<2>(v, o);
-    if (threadIdx.x == 0) {
-        S.partials[SLOT_RZ * S.nblk0 + bk_.y] = o[0];
-        if (Dots == 2) {
-            S.partials[SLOT_ZQ * S.nblk0 + bk_.y] = o[1];
-        }
-    }
-}
-
 __global__ void k_gather_states(const SysDev* __restrict__ sys, int n_sys, SolveState* __restrict__ out) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < n_sys) {
@@ -376,7 +345,9 @@ __global__ void k_gather_states(const SysDev* __restrict__ sys, int n_sys, Solve
 __global__ void k_init_states(const SysDev* __restrict__ sys, int n_sys, const SolveState* __restrict__ init) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < n_sys) {
-        *sys[s].st = init[s];
+        for (int k = 0; k < k_states; ++k) {
+            sys[s].st[k] = init[s];
+        }
     }
 }
 
@@ -590,7 +561,7 @@ void System::build_symmetric_layout(const cfdg_ldu_pattern& pt, const std::vecto
     sym_w_ = 0;
     sym_n_ = 0;
     sym_active_ = false;
-    if (std::getenv("CFDG_NO_SYM") != nullptr) {
+    if (std::getenv("CFDG_NO_SYM") != nullptr || n_ >= (1 << 29)) { // 32-bit byte offsets in the kernels
         return;
     }
     // The stencil: the distinct column offsets of all rows (at most k_max_offsets).
@@ -642,8 +613,8 @@ void System::build_symmetric_layout(const cfdg_ldu_pattern& pt, const std::vecto
         const int a = off[static_cast<std::size_t>(k)] < 0 ? -off[static_cast<std::size_t>(k)] : off[static_cast<std::size_t>(k)];
         tab[static_cast<std::size_t>(n_off + k)] = static_cast<int>(std::lower_bound(up.begin(), up.end(), a) - up.begin());
     }
-    const std::size_t per_slice = static_cast<std::size_t>(w) * k_wave;
-    const std::size_t slots = static_cast<std::size_t>(ceil_div(n_, k_wave)) * per_slice;
+    const std::size_t pad = static_cast<std::size_t>(ceil_div(n_, k_wave)) * k_wave;
+    const std::size_t slots = static_cast<std::size_t>(w) * pad;
     std::vector<int> src(slots, -1);
 #pragma omp parallel for schedule(static)
     for (int i = 0; i < n_; ++i) {
@@ -651,8 +622,7 @@ void System::build_symmetric_layout(const cfdg_ldu_pattern& pt, const std::vecto
             const int o = pt.col[k] - i;
             if (o >= 0) {
                 const std::size_t j = static_cast<std::size_t>(std::lower_bound(up.begin(), up.end(), o) - up.begin());
-                src[static_cast<std::size_t>(i / k_wave) * per_slice + j * k_wave + static_cast<std::size_t>(i % k_wave)] =
-                    csr_src[static_cast<std::size_t>(k)];
+                src[j * pad + static_cast<std::size_t>(i)] = csr_src[static_cast<std::size_t>(k)];
             }
         }
     }
@@ -706,10 +676,10 @@ void System::init_vectors() {
     }
     r32_.resize(n);
     wd0_32_.resize(n);
-    const int nblk0 = ceil_div(n_, k_block);
+    const int nblk0 = ceil_div(n_, k_block); // the normalised residual's blocks, at least the row groups
     partials_.resize(static_cast<std::size_t>(k_slots) * static_cast<std::size_t>(nblk0));
     partials_.zero(stream_.get());
-    state_.resize(1);
+    state_.resize(k_states);
     state_.zero(stream_.get());
     hip_check(hipStreamSynchronize(stream_.get()), "init sync");
 }
@@ -869,7 +839,7 @@ std::size_t estimate_footprint(const cfdg_ldu_pattern& pt, const cfdg_amg_view* 
     std::size_t b = layout_slots(pt.n, pt.row_ptr) * (4 + 2 + 8 + 4 + 2 + 4);
     b += n * (15 * 8 + 3 * 4 + 2 * 4) + (n + 2 * static_cast<std::size_t>(pt.n_faces)) * 8;
     b += n * 5 * (4 + 8 + 4); // symmetric stencil storage (box stencils store 3 to 5 slots per row)
-    b += static_cast<std::size_t>(k_slots) * nblk0 * 8 + sizeof(SolveState) + 64 * 1024;
+    b += static_cast<std::size_t>(k_slots) * nblk0 * 8 + k_states * sizeof(SolveState) + 64 * 1024;
     if (amg != nullptr && amg->levels != nullptr) {
         for (int l = 0; l < amg->n_levels; ++l) {
             const cfdg_amg_level_view& v = amg->levels[l];
@@ -1252,7 +1222,9 @@ SysDev System::descriptor(bool fp32, bool use_amg, bool bf16) {
     SysDev d{};
     d.st = state_.get();
     d.partials = partials_.get();
-    d.nblk0 = ceil_div(n_, k_block);
+    d.n_groups = group_count(n_);
+    d.chunks = group_chunks(n_);
+    d.segment = group_segment(n_);
     d.n = n_;
     d.a64 = a0_view(false);
     d.b = b_.get();
@@ -1344,8 +1316,11 @@ struct IdsRef {
 struct Tables {
     int n_sys = 0;
     int l_max = 1;
-    IdsRef ids;                    // descriptor index of each system (finalize workgroups)
-    std::vector<TableRef> t;       // per level: 256-row blocks of systems having the level
+    int gpb = 1;                   // row groups per workgroup of the level-0 tables
+    bool sym7 = false;             // every system's finest operator is in L0_SYM7 form
+    IdsRef ids;                    // descriptor index of each system (workgroups of k_step)
+    std::vector<TableRef> t;       // level 0: every gpb-th row group; below: 256-row blocks of the
+                                   // systems having the level
     std::vector<int> tn;
     std::vector<TableRef> c;       // per level: 4-row blocks of systems whose coarsest it is
     std::vector<int> cn;
@@ -1382,6 +1357,16 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
             tb.l_max = std::max(tb.l_max, x->n_levels(fp32));
         }
     }
+    // Row groups per workgroup: one up to 8192 groups in all, so that a single system's few groups
+    // spread over the chip; above, the workgroups of a large batch stay near 8192, each making its
+    // kernel's step once for several groups.
+    long long groups = 0;
+    tb.sym7 = true;
+    for (System* x : sys) {
+        groups += group_count(x->n());
+        tb.sym7 = tb.sym7 && x->symmetric_offsets() == 7;
+    }
+    tb.gpb = static_cast<int>(std::min(16LL, std::max(1LL, (groups + 8191) / 8192)));
     const std::size_t L = static_cast<std::size_t>(tb.l_max);
     // Host image: ids (two per int2), then the tables; offsets recorded per table.
     std::vector<int2> img((ids.size() + 1) / 2, make_int2(0, 0));
@@ -1402,8 +1387,9 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
                 continue;
             }
             const int rows = (use_amg && l > 0) ? x->level_rows(l) : x->n();
-            const int nb = ceil_div(rows, k_block);
-            for (int b = 0; b < nb; ++b) {
+            const int nb = l == 0 ? group_count(rows) : ceil_div(rows, k_block);
+            const int step = l == 0 ? tb.gpb : 1;
+            for (int b = 0; b < nb; b += step) {
                 img.push_back(make_int2(id, b));
             }
             if (use_amg && l == nl - 1) {
@@ -1412,7 +1398,7 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
                     c.push_back(make_int2(id, b));
                 }
                 if (l == 0) {
-                    for (int b = 0; b < nb; ++b) {
+                    for (int b = 0; b < nb; b += step) {
                         single.push_back(make_int2(id, b));
                     }
                 }
@@ -1550,6 +1536,16 @@ void probe_end(int kind, hipStream_t s) {
         }                                                                                         \
     } while (0)
 
+// Calls f(form) with the form (L0Form) that the level-0 kernels of a launch are built for.
+template <class F>
+void with_form(bool sym7, F f) {
+    if (sym7) {
+        f(std::integral_constant<int, L0_SYM7>{});
+    } else {
+        f(std::integral_constant<int, L0_ANY>{});
+    }
+}
+
 // One of two kernels of the same arithmetic: the pair variant (k_block_pair threads, two slices
 // per wavefront) or the one-slice kernel.
 #define CFDG_LAUNCH_EITHER(pair, kpair, kone, grid, stream, ...)                                  \
@@ -1614,11 +1610,30 @@ SweepFactors sweep_factors(int k, double ratio) {
     return f;
 }
 
+template <int Op>
+void run_step(const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report) {
+    k_step<Op><<<tb.n_sys, k_block, 0, s>>>(d, tb.ids.get(), report);
+}
+
+template <int Op>
+void run_start(const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report) {
+    k_start<Op><<<tb.n_sys, k_block, 0, s>>>(d, tb.ids.get(), report);
+}
+
 template <class T, int Dots>
-void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s, bool pair, const SweepFactors& sf) {
+void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s, bool pair, const SweepFactors& sf,
+                    unsigned long long* report, bool sym7) {
     const int fin = final_index(sweeps);
     const T f1 = static_cast<T>(sf.pre[0]);
     const int L = tb.l_max;
+    // The residual step is made by the cycle's first kernel where that is a level-0 sweep for every
+    // system; else (one-level hierarchies, cycles without smoothing) by a launch of its own.
+    const int g0 = tb.tn[0];
+    const int2* b0 = tb.t[0].get();
+    const bool step = sweeps > 0 && tb.cn[0] == 0 && (sweeps == 1 ? tb.x1[0] : tb.a_ell[0]) != 0;
+    if (!step) {
+        run_step<FIN_RES>(d, tb, s, report);
+    }
     CFDG_LAUNCH(k_coarse<T>, tb.cn[0], s, d, tb.c[0].get(), 0, fin);
     std::vector<int> cur(static_cast<std::size_t>(L), 0);
     // Where the first sweep from zero of level l is stored as v[x1_slot(l)] = wd b (-1: not
@@ -1646,7 +1661,7 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
         const int x1_next = l + 2 < L ? x1_slot(l + 1) : -1;
         int c = 0;
         if (sweeps == 0) {
-            CFDG_LAUNCH(k_zero_level<T>, g, s, d, blk, l, 0);
+            CFDG_LAUNCH(k_zero_level<T>, l == 0 ? ga : g, s, d, l == 0 ? ba : blk, l, 0);
         } else if (sweeps == 1) {
             // x1 = wd b is formed inside the residual (or stored, for many long rows) and
             // inside the prolongation; bitwise the same as a stored sweep
@@ -1656,11 +1671,19 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
                 CFDG_LAUNCH(k_coarse<T>, tb.cn[li + 1], s, d, tb.c[li + 1].get(), l + 1, fin);
                 continue;
             }
-            if (tb.x1[li] != 0) {
+            if (tb.x1[li] != 0 && l == 0) {
+                if (step) {
+                    with_form(sym7, [&](auto form) {
+                        CFDG_LAUNCH((k_l0_residual_x1<T, form.value, true>), g0, s, d, b0, tb.gpb, 1, f1, report);
+                    });
+                } else {
+                    CFDG_LAUNCH((k_l0_residual_x1<T, L0_ANY, false>), g0, s, d, b0, tb.gpb, 1, f1, nullptr);
+                }
+            } else if (tb.x1[li] != 0) {
                 CFDG_LAUNCH(k_residual_x1<T>, ga, s, d, ba, l, 1, f1);
             } else {
                 if (l == 0) {
-                    CFDG_LAUNCH(k_jacobi_zero<T>, g, s, d, blk, l, 0, f1);
+                    CFDG_LAUNCH(k_jacobi_zero<T>, ga, s, d, ba, l, 0, f1);
                 }
                 CFDG_LAUNCH(k_residual<T>, ga, s, d, ba, l, 0, 1);
             }
@@ -1669,17 +1692,21 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
             continue;
         } else {
             const T f2 = static_cast<T>(sf.pre[1]);
-            if (tb.a_ell[li] != 0) {
-                CFDG_LAUNCH(k_presmooth2<T>, ga, s, d, ba, l, 0, f1, f2);
+            if (tb.a_ell[li] != 0 && step) { // level 0 only
+                with_form(sym7, [&](auto form) {
+                    CFDG_LAUNCH((k_l0_presmooth2<T, form.value, true>), g0, s, d, b0, tb.gpb, 0, f1, f2, report);
+                });
+            } else if (tb.a_ell[li] != 0) {
+                CFDG_LAUNCH((k_l0_presmooth2<T, L0_ANY, false>), g0, s, d, b0, tb.gpb, 0, f1, f2, nullptr);
             } else { // long rows: form x1 = wd b once instead of gathering it per entry
                 if (l == 0) {
-                    CFDG_LAUNCH(k_jacobi_zero<T>, g, s, d, blk, l, 2, f1);
+                    CFDG_LAUNCH(k_jacobi_zero<T>, ga, s, d, ba, l, 2, f1);
                 }
-                CFDG_LAUNCH((k_jacobi<T, 0>), ga, s, d, ba, l, 2, 0, f2);
+                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, 2, 0, f2);
             }
             for (int k = 2; k < sweeps; ++k) {
                 const int o = c == 0 ? 2 : 0;
-                CFDG_LAUNCH((k_jacobi<T, 0>), ga, s, d, ba, l, c, o, static_cast<T>(sf.pre[k]));
+                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, c, o, static_cast<T>(sf.pre[k]));
                 c = o;
             }
         }
@@ -1708,30 +1735,27 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
             if (l == 0 && last) {
                 probe_begin(PROBE_L0_SWEEP, s);
                 if (pair) {
-                    CFDG_LAUNCH_PAIR((k_jacobi_pair<T, Dots>), ga, s, d, ba, l, c, o, fk);
+                    with_form(sym7, [&](auto form) {
+                        CFDG_LAUNCH((k_l0_jacobi<T, form.value, Dots, true>), g0, s, d, b0, tb.gpb, c, o, fk);
+                    });
                 } else {
-                    CFDG_LAUNCH((k_jacobi<T, Dots>), ga, s, d, ba, l, c, o, fk);
+                    with_form(sym7, [&](auto form) {
+                        CFDG_LAUNCH((k_l0_jacobi<T, form.value, Dots, false>), g0, s, d, b0, tb.gpb, c, o, fk);
+                    });
                 }
                 probe_end(PROBE_L0_SWEEP, s);
             } else {
-                CFDG_LAUNCH((k_jacobi<T, 0>), ga, s, d, ba, l, c, o, fk);
+                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, c, o, fk);
             }
             c = o;
         }
     }
     if (sweeps == 0 && L > 1) {
-        CFDG_LAUNCH((k_level0_dots<T, Dots>), tb.tn[0], s, d, tb.t[0].get(), fin);
+        CFDG_LAUNCH((k_level0_dots<T, Dots>), g0, s, d, b0, tb.gpb, fin);
     } else {
-        CFDG_LAUNCH((k_level0_dots<T, Dots>), tb.t0_single_n, s, d, tb.t0_single.get(), fin);
+        CFDG_LAUNCH((k_level0_dots<T, Dots>), tb.t0_single_n, s, d, tb.t0_single.get(), tb.gpb, fin);
     }
 }
-
-template <int Op>
-void fin(const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report = nullptr) {
-    k_finalize<Op><<<tb.n_sys, k_fin_block, 0, s>>>(d, tb.ids.get(), report);
-}
-
-enum VecId { V_X = 0, V_R, V_P, V_Q, V_Z, V_R0, V_V, V_S, V_T, V_PH, V_SH };
 
 struct Plan {
     cfdg_method method;
@@ -1748,75 +1772,86 @@ void enqueue_init(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t
     const int g0 = tb.tn[0];
     const int2* b0 = tb.t[0].get();
     if (pl.method == CFDG_METHOD_BICGSTAB) {
-        CFDG_LAUNCH(k_bicg_init<false>, g0, s, d, b0);
-        fin<FIN_BICG_INIT>(d, tb, s, report);
+        with_form(tb.sym7, [&](auto form) { CFDG_LAUNCH((k_bicg_init<form.value>), g0, s, d, b0, tb.gpb); });
+        run_start<FIN_BICG_RES>(d, tb, s, report);
         return;
     }
-    // CG start: r, z and beta = 0; p = z + 0 p_old (p_old = 0) is formed by the first
-    // iteration's product (k_spmv_pz).
+    // CG start: r, z; p = z + 0 p_old (p_old = 0) is formed by the first iteration's product
+    // (k_spmv_pz).
     if (!pl.amg) {
-        CFDG_LAUNCH(k_cg_init<false>, g0, s, d, b0);
-        fin<FIN_CG_INIT>(d, tb, s, report);
+        with_form(tb.sym7, [&](auto form) { CFDG_LAUNCH((k_cg_init<form.value>), g0, s, d, b0, tb.gpb); });
+        run_start<FIN_CG_RES_BETA>(d, tb, s, report);
         return;
     }
     if (pl.fp32) {
-        CFDG_LAUNCH(k_residual0<true>, g0, s, d, b0);
+        with_form(tb.sym7, [&](auto form) {
+            CFDG_LAUNCH((k_residual0<true, form.value>), g0, s, d, b0, tb.gpb);
+        });
     } else {
-        CFDG_LAUNCH(k_residual0<false>, g0, s, d, b0);
+        with_form(tb.sym7, [&](auto form) {
+            CFDG_LAUNCH((k_residual0<false, form.value>), g0, s, d, b0, tb.gpb);
+        });
     }
-    fin<FIN_AMG_INIT>(d, tb, s, report);
+    run_start<FIN_RES>(d, tb, s, report);
 }
 
 // One iteration for every listed system; parity = iteration number mod 2 selects the
-// search-direction buffers. The AMG-PCG iteration begins with the V-cycle and ends with the
-// residual test, so that nothing is queued between a test that ends the solve and the report of
-// it; the last step stores each system's report word at report[id].
+// search-direction buffers. It begins with the residual step of the iteration before it, which
+// stores each system's report word at report[id] (report may be null), and leaves its own to the
+// next iteration or enqueue_check.
 void enqueue_iteration(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t s, int parity,
                        unsigned long long* report) {
     const int g0 = tb.tn[0];
     const int2* b0 = tb.t[0].get();
+    const int gpb = tb.gpb;
     if (pl.method == CFDG_METHOD_BICGSTAB) {
-        CFDG_LAUNCH(k_bicg_p, g0, s, d, b0); // rho and beta: ended the previous finalize (bicg_rho)
-        CFDG_LAUNCH((k_spmv_dot<false, false>), g0, s, d, b0, V_PH, V_V, V_R0, SLOT_R0V, 0, 0);
-        fin<FIN_BICG_ALPHA>(d, tb, s);
-        CFDG_LAUNCH(k_bicg_s, g0, s, d, b0);
-        fin<FIN_BICG_S>(d, tb, s);
-        CFDG_LAUNCH(k_bicg_early_x, g0, s, d, b0);
-        CFDG_LAUNCH((k_spmv_dot<true, false>), g0, s, d, b0, V_SH, V_T, V_T, SLOT_TT, V_S, SLOT_TS);
-        fin<FIN_BICG_OMEGA>(d, tb, s);
-        CFDG_LAUNCH(k_bicg_xr, g0, s, d, b0);
-        fin<FIN_BICG_RES>(d, tb, s, report);
+        CFDG_LAUNCH(k_bicg_p, g0, s, d, b0, gpb, report);
+        with_form(tb.sym7, [&](auto form) { CFDG_LAUNCH((k_bicg_v<form.value>), g0, s, d, b0, gpb); });
+        CFDG_LAUNCH(k_bicg_s, g0, s, d, b0, gpb);
+        with_form(tb.sym7, [&](auto form) { CFDG_LAUNCH((k_bicg_t<form.value>), g0, s, d, b0, gpb); });
+        CFDG_LAUNCH(k_bicg_xr, g0, s, d, b0, gpb);
         return;
     }
     const int fz = final_index(pl.sweeps);
     if (pl.amg && pl.fp32) {
-        enqueue_vcycle<float, 2>(d, tb, pl.sweeps, s, !pl.bf16 && pair_sweeps(), pl.sf);
-        fin<FIN_BETA_FLEX>(d, tb, s);
+        // BF16 cycles keep the full layout of the finest operator
+        enqueue_vcycle<float, 2>(d, tb, pl.sweeps, s, !pl.bf16 && pair_sweeps(), pl.sf, report, tb.sym7 && !pl.bf16);
     } else if (pl.amg) {
-        enqueue_vcycle<double, 1>(d, tb, pl.sweeps, s, false, pl.sf);
-        fin<FIN_BETA>(d, tb, s);
+        enqueue_vcycle<double, 1>(d, tb, pl.sweeps, s, false, pl.sf, report, tb.sym7);
     }
     probe_begin(PROBE_OUTER_SPMV, s);
     if (!pl.amg) {
-        CFDG_LAUNCH((k_spmv_pz<double, false>), g0, s, d, b0, parity, 0, 0);
+        with_form(tb.sym7, [&](auto form) {
+            CFDG_LAUNCH((k_spmv_pz<double, form.value, FIN_CG_RES_BETA>), g0, s, d, b0, gpb, parity, 0, 0, report);
+        });
     } else if (pl.fp32) {
-        CFDG_LAUNCH((k_spmv_pz<float, false>), g0, s, d, b0, parity, 1, fz);
+        with_form(tb.sym7, [&](auto form) {
+            CFDG_LAUNCH((k_spmv_pz<float, form.value, FIN_BETA_FLEX>), g0, s, d, b0, gpb, parity, 1, fz, nullptr);
+        });
     } else {
-        CFDG_LAUNCH((k_spmv_pz<double, false>), g0, s, d, b0, parity, 1, fz);
+        with_form(tb.sym7, [&](auto form) {
+            CFDG_LAUNCH((k_spmv_pz<double, form.value, FIN_BETA>), g0, s, d, b0, gpb, parity, 1, fz, nullptr);
+        });
     }
     probe_end(PROBE_OUTER_SPMV, s);
-    fin<FIN_ALPHA>(d, tb, s);
     if (!pl.amg) {
-        CFDG_LAUNCH(k_update_xr<1>, g0, s, d, b0, parity);
-        fin<FIN_CG_RES_BETA>(d, tb, s, report);
-        return;
-    }
-    if (pl.fp32) {
-        CFDG_LAUNCH(k_update_xr<2>, g0, s, d, b0, parity);
+        CFDG_LAUNCH(k_update_xr<1>, g0, s, d, b0, gpb, parity);
+    } else if (pl.fp32) {
+        CFDG_LAUNCH(k_update_xr<2>, g0, s, d, b0, gpb, parity);
     } else {
-        CFDG_LAUNCH(k_update_xr<0>, g0, s, d, b0, parity);
+        CFDG_LAUNCH(k_update_xr<0>, g0, s, d, b0, gpb, parity);
     }
-    fin<FIN_RES>(d, tb, s, report);
+}
+
+// The residual step of the last queued iteration, into the public state and report[id].
+void enqueue_check(const Plan& pl, const SysDev* d, const Tables& tb, hipStream_t s, unsigned long long* report) {
+    if (pl.method == CFDG_METHOD_BICGSTAB) {
+        run_step<FIN_BICG_RES>(d, tb, s, report);
+    } else if (!pl.amg) {
+        run_step<FIN_CG_RES_BETA>(d, tb, s, report);
+    } else {
+        run_step<FIN_RES>(d, tb, s, report);
+    }
 }
 
 // A report word as the host reads it.
@@ -2031,8 +2066,8 @@ public:
                 }
             }
         }
-        CFDG_LAUNCH(k_true_residual<false>, tb_.tn[0], s_, d, tb_.t[0].get());
-        fin<FIN_TRUE>(d, tb_, s_);
+        with_form(tb_.sym7, [&](auto form) { CFDG_LAUNCH((k_true_residual<form.value>), tb_.tn[0], s_, d, tb_.t[0].get(), tb_.gpb); });
+        run_step<FIN_TRUE>(d, tb_, s_, nullptr);
         k_gather_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, out_dev_); // into pinned memory
         hip_check(hipGetLastError(), "true residual launch");
         hip_check(hipEventRecord(t1_.get(), s_), "event record");
@@ -2078,6 +2113,7 @@ private:
         const bool odd = ((queued + 1) & 1) != 0;
         if (!graphs) {
             enqueue_iteration(pl_, desc_.get(), tb_, s_, odd ? 1 : 0, report_dev_);
+            enqueue_check(pl_, desc_.get(), tb_, s_, report_dev_);
             hip_check(hipGetLastError(), "iteration launch");
             return 1;
         }
@@ -2106,6 +2142,7 @@ private:
             for (int k = first; k < first + count; ++k) {
                 enqueue_iteration(pl_, d, tb_, s_, k & 1, report_dev_);
             }
+            enqueue_check(pl_, d, tb_, s_, report_dev_);
         };
         for (int k = 0; k < 3; ++k) {
             odd_exec_[k] = capture([&] { iterations(1, 1 << k); });
@@ -2117,7 +2154,7 @@ private:
 public:
     // x = 0 for every system, one launch on the runner's stream (ordered before its next solve).
     void zero_x() {
-        CFDG_LAUNCH(k_zero_x, tb_.tn[0], s_, desc_.get(), tb_.t[0].get());
+        CFDG_LAUNCH(k_zero_x, tb_.tn[0], s_, desc_.get(), tb_.t[0].get(), tb_.gpb);
     }
 
 private:
@@ -2169,7 +2206,7 @@ struct SlotMachinery {
     hipStream_t s = nullptr;
     DevBuf<SysDev> desc;
     PinnedBuf<SysDev> desc_host;
-    PinnedBuf<SolveState> init_host;
+    PinnedBuf<SolveState> init_host; // k_states copies per slot
     PinnedBuf<SolveState> out_host;
     PinnedBuf<unsigned long long> status; // report words: two regions of k, one per iteration parity
     unsigned long long* status_dev = nullptr;
@@ -2211,7 +2248,7 @@ SlotRunner::SlotRunner(int slots, const BatchOptions& opt, int sweeps, hipStream
     const std::size_t k = static_cast<std::size_t>(slots);
     m.desc.resize(k);
     m.desc_host = PinnedBuf<SysDev>(k);
-    m.init_host = PinnedBuf<SolveState>(k);
+    m.init_host = PinnedBuf<SolveState>(k_states * k);
     m.out_host = PinnedBuf<SolveState>(k);
     m.status = PinnedBuf<unsigned long long>(2 * k);
     m.status_dev = m.status.device();
@@ -2276,12 +2313,14 @@ int SlotRunner::start(System* x, const cfdg_solve_control& c) {
         m.single_of[ju] = x->uid();
         m.single_gen[ju] = x->generation();
     }
-    SolveState& st = m.init_host[ju];
-    std::memset(&st, 0, sizeof(st));
-    st.tol = c.abs_tolerance;
-    st.max_it = c.max_iterations;
-    st.status = ST_RUNNING;
-    hip_check(hipMemcpyAsync(x->state(), &st, sizeof(SolveState), hipMemcpyHostToDevice, m.s),
+    SolveState* st = m.init_host.get() + k_states * ju;
+    std::memset(st, 0, k_states * sizeof(SolveState));
+    for (int q = 0; q < k_states; ++q) {
+        st[q].tol = c.abs_tolerance;
+        st[q].max_it = c.max_iterations;
+        st[q].status = ST_RUNNING;
+    }
+    hip_check(hipMemcpyAsync(x->state(), st, k_states * sizeof(SolveState), hipMemcpyHostToDevice, m.s),
               "slot state H2D");
     enqueue_init(m.pl, m.desc.get(), m.single[ju], m.s, nullptr);
     hip_check(hipGetLastError(), "slot init launch");
@@ -2310,7 +2349,8 @@ void SlotRunner::step(std::vector<Done>& done) {
         }
         const Tables& tb = m.merged[m.cur];
         const int parity = static_cast<int>(m.g & 1);
-        enqueue_iteration(m.pl, d, tb, m.s, parity, m.status_dev + static_cast<std::size_t>(parity) * m.k);
+        enqueue_iteration(m.pl, d, tb, m.s, parity, nullptr);
+        enqueue_check(m.pl, d, tb, m.s, m.status_dev + static_cast<std::size_t>(parity) * m.k);
         hip_check(hipEventRecord(m.ev[parity].get(), m.s), "event record");
         hip_check(hipGetLastError(), "slot iteration launch");
         m.covered[parity].clear();
@@ -2336,8 +2376,8 @@ void SlotRunner::step(std::vector<Done>& done) {
                 continue;
             }
             const Tables& one = m.single[ju];
-            CFDG_LAUNCH(k_true_residual<false>, one.tn[0], m.s, d, one.t[0].get());
-            fin<FIN_TRUE>(d, one, m.s);
+            with_form(one.sym7, [&](auto form) { CFDG_LAUNCH((k_true_residual<form.value>), one.tn[0], m.s, d, one.t[0].get(), one.gpb); });
+            run_step<FIN_TRUE>(d, one, m.s, nullptr);
             hip_check(hipMemcpyAsync(m.out_host.get() + j, m.sys[ju]->state(), sizeof(SolveState),
                                      hipMemcpyDeviceToHost, m.s),
                       "slot state D2H");
@@ -2830,9 +2870,9 @@ constexpr int k_na_vectors = 12; // r p p2 q z dinv r0 v s t ph sh
 constexpr std::size_t k_na_max_blocks = static_cast<std::size_t>(k_na_max_rows) / k_block;
 static_assert(k_na_max_rows % k_block == 0, "whole blocks");
 // Byte offsets of the scratch regions.
-constexpr std::size_t k_na_state = 0;   // SolveState
-constexpr std::size_t k_na_flag = 256;  // int: 1 when the CSR check failed
-constexpr std::size_t k_na_ids = 512;   // int: system id 0 (finalize launches)
+constexpr std::size_t k_na_state = 0;   // k_states SolveState
+constexpr std::size_t k_na_flag = 512;  // int: 1 when the CSR check failed
+constexpr std::size_t k_na_ids = 768;   // int: system id 0 (step launches)
 constexpr std::size_t k_na_desc = 1024; // SysDev
 constexpr std::size_t k_na_blocks = round_up(k_na_desc + sizeof(SysDev), 256);
 constexpr std::size_t k_na_partials = round_up(k_na_blocks + k_na_max_blocks * sizeof(int2), 256);
@@ -2841,7 +2881,7 @@ constexpr std::size_t k_na_vecs =
 constexpr std::size_t k_na_bytes =
     k_na_vecs + static_cast<std::size_t>(k_na_vectors) * static_cast<std::size_t>(k_na_max_rows) * sizeof(double);
 static_assert(k_na_bytes <= CFDG_NOALLOC_SCRATCH_BYTES, "scratch size stated in cfdgpu.h");
-static_assert(sizeof(SolveState) <= k_na_flag - k_na_state, "state region");
+static_assert(k_states * sizeof(SolveState) <= k_na_flag - k_na_state, "state region");
 
 // Checks a caller's CSR matrix in place: row offsets from 0 to nnz and non-decreasing, columns
 // in [0, n). Any violation stores 1 at *bad (every writer stores the same value). Thread i
@@ -2915,8 +2955,8 @@ unsigned char* na_scratch(int dev) {
 }
 
 template <int Op>
-void na_fin(const SysDev* d, const int* ids) {
-    k_finalize<Op><<<1, k_fin_block, 0, nullptr>>>(d, ids, nullptr);
+void na_step(const SysDev* d, const int* ids) {
+    k_step<Op><<<1, k_block, 0, nullptr>>>(d, ids, nullptr);
 }
 
 int na_status(const SolveState* st) {
@@ -2974,7 +3014,10 @@ extern "C" cfdg_status cfdg_solve_csr_noalloc(const cfdg_csr* a, const double* b
         SysDev d{};
         d.st = st;
         d.partials = partials;
-        d.nblk0 = nblk;
+        d.n_groups = group_count(n);
+        d.chunks = group_chunks(n);
+        d.segment = group_segment(n);
+        const int groups = d.n_groups;
         d.n = n;
         d.n_levels = 0;
         d.flip = 0;
@@ -2999,12 +3042,14 @@ extern "C" cfdg_status cfdg_solve_csr_noalloc(const cfdg_csr* a, const double* b
         d.t = vec(9);
         d.ph = vec(10);
         d.sh = vec(11);
-        SolveState s0{};
-        s0.tol = control->abs_tolerance;
-        s0.max_it = control->max_iterations;
-        s0.status = ST_RUNNING;
+        SolveState s0[k_states] = {};
+        for (SolveState& q : s0) {
+            q.tol = control->abs_tolerance;
+            q.max_it = control->max_iterations;
+            q.status = ST_RUNNING;
+        }
         hip_check(hipMemcpy(desc, &d, sizeof(SysDev), hipMemcpyHostToDevice), "H2D descriptor");
-        hip_check(hipMemcpy(st, &s0, sizeof(SolveState), hipMemcpyHostToDevice), "H2D state");
+        hip_check(hipMemcpy(st, s0, sizeof s0, hipMemcpyHostToDevice), "H2D state");
         k_na_setup<<<nblk, k_block, 0, nullptr>>>(n, a->row_ptr, a->col, a->val, nblk, blocks, ids, dinv);
         hip_check(hipGetLastError(), "k_na_setup launch");
 
@@ -3012,31 +3057,27 @@ extern "C" cfdg_status cfdg_solve_csr_noalloc(const cfdg_csr* a, const double* b
         // the status after each iteration (surplus iterations would be no-ops on the device).
         const int max_it = control->max_iterations;
         if (method == CFDG_METHOD_CG) {
-            k_cg_init<true><<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-            na_fin<FIN_CG_INIT>(desc, ids);
+            k_cg_init<L0_CSR><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+            k_start<FIN_CG_RES_BETA><<<1, k_block, 0, nullptr>>>(desc, ids, nullptr);
         } else {
-            k_bicg_init<true><<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-            na_fin<FIN_BICG_INIT>(desc, ids);
+            k_bicg_init<L0_CSR><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+            k_start<FIN_BICG_RES><<<1, k_block, 0, nullptr>>>(desc, ids, nullptr);
         }
         hip_check(hipGetLastError(), "init launch");
         for (int k = 1; k <= max_it + 2; ++k) {
             const int parity = k & 1;
             if (method == CFDG_METHOD_CG) {
-                k_spmv_pz<double, true><<<nblk, k_block, 0, nullptr>>>(desc, blocks, parity, 0, 0);
-                na_fin<FIN_ALPHA>(desc, ids);
-                k_update_xr<1><<<nblk, k_block, 0, nullptr>>>(desc, blocks, parity);
-                na_fin<FIN_CG_RES_BETA>(desc, ids);
+                k_spmv_pz<double, L0_CSR, FIN_CG_RES_BETA><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1, parity, 0, 0,
+                                                                                         nullptr);
+                k_update_xr<1><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1, parity);
+                na_step<FIN_CG_RES_BETA>(desc, ids);
             } else {
-                k_bicg_p<<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-                k_spmv_dot<false, true><<<nblk, k_block, 0, nullptr>>>(desc, blocks, V_PH, V_V, V_R0, SLOT_R0V, 0, 0);
-                na_fin<FIN_BICG_ALPHA>(desc, ids);
-                k_bicg_s<<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-                na_fin<FIN_BICG_S>(desc, ids);
-                k_bicg_early_x<<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-                k_spmv_dot<true, true><<<nblk, k_block, 0, nullptr>>>(desc, blocks, V_SH, V_T, V_T, SLOT_TT, V_S, SLOT_TS);
-                na_fin<FIN_BICG_OMEGA>(desc, ids);
-                k_bicg_xr<<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-                na_fin<FIN_BICG_RES>(desc, ids);
+                k_bicg_p<<<groups, k_block, 0, nullptr>>>(desc, blocks, 1, nullptr);
+                k_bicg_v<L0_CSR><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+                k_bicg_s<<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+                k_bicg_t<L0_CSR><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+                k_bicg_xr<<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+                na_step<FIN_BICG_RES>(desc, ids);
             }
             hip_check(hipGetLastError(), "iteration launch");
             const int status = na_status(st);
@@ -3044,8 +3085,8 @@ extern "C" cfdg_status cfdg_solve_csr_noalloc(const cfdg_csr* a, const double* b
                 break;
             }
         }
-        k_true_residual<true><<<nblk, k_block, 0, nullptr>>>(desc, blocks);
-        na_fin<FIN_TRUE>(desc, ids);
+        k_true_residual<L0_CSR><<<groups, k_block, 0, nullptr>>>(desc, blocks, 1);
+        na_step<FIN_TRUE>(desc, ids);
         hip_check(hipGetLastError(), "true residual launch");
         SolveState out{};
         hip_check(hipMemcpy(&out, st, sizeof(SolveState), hipMemcpyDeviceToHost), "D2H state");

@@ -108,6 +108,8 @@ public:
     // (0: the hierarchy's own weight).
     [[nodiscard]] double smoother_ratio() const { return mixed_ratio_; }
     [[nodiscard]] hipStream_t stream() const { return stream_.get(); }
+    // Offsets of the finest operator's stencil while it is in symmetric storage, else 0.
+    [[nodiscard]] int symmetric_offsets() const { return sym_active_ ? sym_n_ : 0; }
     [[nodiscard]] SolveState* state() const { return state_.get(); }
     [[nodiscard]] int level_rows(int l) const { return levels_[static_cast<std::size_t>(l)].n; }
     // Lanes per row of level l's operator (which 0), prolongation (1) or restriction (2).
