@@ -1219,11 +1219,10 @@ public:
             k_fv_pressure_cells<<<blocks(), k_fv_block, 0, s>>>(m, phih_.get(), gface_.get(), pin, pout);
         });
         have_pressure_ = true;
+        std::vector<HostCopy> backs;
         const auto back = [&](const DevBuf<double>& buf, double* dst, long long n) {
             if (dst != nullptr && n > 0) {
-                hip_check(hipMemcpyAsync(dst, buf.get(), static_cast<std::size_t>(n) * sizeof(double),
-                                         hipMemcpyDeviceToHost, stream_.get()),
-                          "DeviceFv D2H");
+                backs.push_back({buf.get(), dst, static_cast<std::size_t>(n) * sizeof(double)});
             }
         };
         if (out != nullptr) {
@@ -1236,7 +1235,7 @@ public:
             back(hbya_, out->hbya, 3 * c);
             back(rau_, out->rau, c);
         }
-        hip_check(hipStreamSynchronize(stream_.get()), "DeviceFv sync");
+        d2h_copies(backs.data(), static_cast<int>(backs.size()), stream_.get());
     }
 
     // The last pressure equation on the device (all null before the first one).
@@ -1356,12 +1355,8 @@ private:
     }
 
     void get(const DevBuf<double>& buf, double* data, long long n) {
-        if (n > 0) {
-            hip_check(hipMemcpyAsync(data, buf.get(), static_cast<std::size_t>(n) * sizeof(double),
-                                     hipMemcpyDeviceToHost, stream_.get()),
-                      "DeviceFv D2H");
-        }
-        hip_check(hipStreamSynchronize(stream_.get()), "DeviceFv sync");
+        const HostCopy c{buf.get(), data, static_cast<std::size_t>(n) * sizeof(double)};
+        d2h_copies(&c, 1, stream_.get());
     }
 
     int nc_ = 0;

@@ -794,10 +794,8 @@ void System::set_x(const double* x) {
 
 void System::get_x(double* x) {
     require(x != nullptr, "get_x: null x");
-    hip_check(hipMemcpyAsync(x, x_.get(), static_cast<std::size_t>(n_) * sizeof(double),
-                             hipMemcpyDeviceToHost, stream_.get()),
-              "D2H x");
-    hip_check(hipStreamSynchronize(stream_.get()), "D2H sync");
+    const HostCopy c{x_.get(), x, static_cast<std::size_t>(n_) * sizeof(double)};
+    d2h_copies(&c, 1, stream_.get());
 }
 
 void System::copy_rhs_from(const double* dev, hipStream_t s) {
