@@ -86,26 +86,45 @@ __device__ __forceinline__ gmem_t<T>* gm(T* p) {
     return (gmem_t<T>*)p;
 }
 
-// Column index of slot k: 32-bit columns (ColAbs), row + 16-bit offset (ColOff, square
-// matrices), the slice's base column + unsigned 16-bit offset (ColBase, transfer operators) or
-// row + the slice's stencil offset of round k (ColStencil, square matrices, one lane per row).
-// The format is chosen once per matrix (a uniform branch), never per slot: a per-lane pointer
-// test would turn every column load into a divergent branch with its own wait.
+// Element i of an array whose base is the same for the whole wavefront: the base stays in scalar
+// registers and the address is one 32-bit byte offset per lane (i sizeof(T) < 2^32), which all the
+// loads of a row share.
+template <class T>
+__device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, unsigned i) {
+    return *(const gmem_t<const T>*)((const gmem_t<const char>*)base + i * static_cast<unsigned>(sizeof(T)));
+}
+
+template <class T>
+__device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, unsigned i, T v) {
+    *(gmem_t<T>*)((gmem_t<char>*)base + i * static_cast<unsigned>(sizeof(T))) = v;
+}
+
+// Column index of the lane's entry in the 64 slots from k on (uniform over the wavefront): 32-bit
+// columns (ColAbs), row + 16-bit offset (ColOff, square matrices), the slice's base column + unsigned
+// 16-bit offset (ColBase, transfer operators) or row + the slice's stencil offset of round k
+// (ColStencil, square matrices, one lane per row). The format is chosen once per matrix (a uniform
+// branch), never per slot: a per-lane pointer test would turn every column load into a divergent
+// branch with its own wait.
 struct ColAbs {
     const gmem_t<const int>* __restrict__ col;
-    __device__ __forceinline__ int operator()(int k) const { return col[k]; }
+    unsigned lane;
+    __device__ __forceinline__ int operator()(int k) const { return load_at<int>(col + k, lane); }
 };
 
 struct ColOff {
     const gmem_t<const short>* __restrict__ dcol;
+    unsigned lane;
     int row;
-    __device__ __forceinline__ int operator()(int k) const { return row + static_cast<int>(dcol[k]); }
+    __device__ __forceinline__ int operator()(int k) const { return row + static_cast<int>(load_at<short>(dcol + k, lane)); }
 };
 
 struct ColBase {
     const gmem_t<const unsigned short>* __restrict__ dcol;
+    unsigned lane;
     int base;
-    __device__ __forceinline__ int operator()(int k) const { return base + static_cast<int>(dcol[k]); }
+    __device__ __forceinline__ int operator()(int k) const {
+        return base + static_cast<int>(load_at<unsigned short>(dcol + k, lane));
+    }
 };
 
 // Stencil column: the slice's offset table (uniform over the wavefront) added to the row,
@@ -118,26 +137,29 @@ struct ColStencil {
 };
 
 template <class T, class V>
-__device__ __forceinline__ T value_at(const gmem_t<const V>* __restrict__ val, int i) {
+__device__ __forceinline__ T value_at(const gmem_t<const V>* __restrict__ val, unsigned lane) {
     if constexpr (sizeof(V) == 2) {
-        return bf16_to_float(val[i]);
+        return bf16_to_float(load_at<V>(val, lane));
     } else {
-        return val[i];
+        return load_at<V>(val, lane);
     }
 }
 
-#ifndef CFDG_ELL_GROUP
-#define CFDG_ELL_GROUP 4
-#endif
-constexpr int k_ell_group = CFDG_ELL_GROUP;
+// Entries of a sliced-ELL row whose loads are issued together. FP32: 6 (level 1 of a 16-system batch,
+// 4 / 6 / 8 entries: sweep 16.3 / 14.6 / 17.3 us, level-0 prolongation 13.5 / 12.1 / 15.6; 128^3 within
+// 4%, 4 and 6 alike). FP64: 4 (128^3: level-1 sweep 20.8 / 21.7 / 24.7, restriction 33.8 / 34.9 / 36.3).
+template <class T>
+constexpr int ell_group() {
+    return sizeof(T) == 4 ? 6 : 4;
+}
 
 // Storage-order row sum of sliced-ELL slots with values val (type V) converted to T. Loads are
-// issued k_ell_group entries at a time, the tail (w mod k_ell_group, uniform over the slice's
+// issued ell_group entries at a time, the tail (w mod k_ell_group, uniform over the slice's
 // wavefront) as one more group with its unused loads repeating a valid slot; only real entries
 // are summed.
 template <class T, class V, class C, class F>
-__device__ __forceinline__ T ell_sum(const C& ci, const gmem_t<const V>* __restrict__ val, int w, F load) {
-    constexpr int G = k_ell_group;
+__device__ __forceinline__ T ell_sum(const C& ci, const gmem_t<const V>* __restrict__ val, unsigned lane, int w, F load) {
+    constexpr int G = ell_group<T>();
     T s = T(0);
     int k = 0;
     for (; k + G <= w; k += G) {
@@ -150,7 +172,7 @@ __device__ __forceinline__ T ell_sum(const C& ci, const gmem_t<const V>* __restr
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            a[g] = value_at<T, V>(val, (k + g) * k_wave);
+            a[g] = value_at<T, V>(val + (k + g) * k_wave, lane);
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -172,7 +194,7 @@ __device__ __forceinline__ T ell_sum(const C& ci, const gmem_t<const V>* __restr
         }
 #pragma unroll
         for (int g = 0; g < G - 1; ++g) {
-            a[g] = value_at<T, V>(val, (g < rem ? k + g : k) * k_wave);
+            a[g] = value_at<T, V>(val + (g < rem ? k + g : k) * k_wave, lane);
         }
 #pragma unroll
         for (int g = 0; g < G - 1; ++g) {
@@ -239,23 +261,7 @@ __device__ __forceinline__ T csr_lane_sum(const gmem_t<const int>* __restrict__ 
     return s;
 }
 
-#ifndef CFDG_SYM_GROUP
-#define CFDG_SYM_GROUP 8
-#endif
-constexpr int k_sym_group = CFDG_SYM_GROUP; // entries whose loads are issued together
-
-// Element i of an array whose base is the same for the whole wavefront: the base stays in scalar
-// registers and the address is one 32-bit byte offset per lane (i sizeof(T) < 2^32), which all the
-// loads of a row share.
-template <class T>
-__device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, unsigned i) {
-    return *(const gmem_t<const T>*)((const gmem_t<const char>*)base + i * static_cast<unsigned>(sizeof(T)));
-}
-
-template <class T>
-__device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, unsigned i, T v) {
-    *(gmem_t<T>*)((gmem_t<char>*)base + i * static_cast<unsigned>(sizeof(T))) = v;
-}
+constexpr int k_sym_group = 8; // entries whose loads are issued together
 
 // What a row product multiplies a column with: (c) for any column; at(near, k, row) for column
 // row + o[k] of a stencil, near = near<N>(o) being the arrays' addresses moved by the stencil's
@@ -511,32 +517,34 @@ __device__ __forceinline__ T ell_row_f(const EllView& m, int slice, int lane, F 
         sym_rows<1, T>(m, slice, 0, lane, load, y);
         return y[0];
     }
-    const int base = m.sp[slice];
-    const int w = (m.sp[slice + 1] - base) / k_wave;
+    slice = __builtin_amdgcn_readfirstlane(slice); // one slice per wavefront: its streams have scalar bases
+    const unsigned ul = static_cast<unsigned>(lane);
+    const auto sp = gm(m.sp);
+    const int base = __builtin_amdgcn_readfirstlane(sp[slice]);
+    const int w = (__builtin_amdgcn_readfirstlane(sp[slice + 1]) - base) / k_wave;
     const int lg = __builtin_ctz(m.tpr); // lanes per row = 2^lg
     const int row = slice * (k_wave >> lg) + (lane >> lg);
     auto sum = [&](const auto& ci) -> T {
         if constexpr (sizeof(T) == 4) {
             if (m.fmt == 1) {
-                const auto val = gm(static_cast<const unsigned short*>(m.val)) + base + lane;
-                const T s = ell_sum<T, unsigned short>(ci, val, w, load);
+                const auto val = gm(static_cast<const unsigned short*>(m.val)) + base;
+                const T s = ell_sum<T, unsigned short>(ci, val, ul, w, load);
                 const T dx = row < m.n_rows ? gm(m.diag)[row] * load(row) : T(0);
                 return madd(gm(m.rscale)[row], s, dx);
             }
         }
-        return ell_sum<T, T>(ci, gm(static_cast<const T*>(m.val)) + base + lane, w, load);
+        return ell_sum<T, T>(ci, gm(static_cast<const T*>(m.val)) + base, ul, w, load);
     };
     if (m.soff != nullptr) {
-        const int tab = __builtin_amdgcn_readfirstlane(base / k_wave); // uniform: one slice per wavefront
-        return sum(ColStencil{gm(m.soff) + tab, row, m.n_rows - 1});
+        return sum(ColStencil{gm(m.soff) + base / k_wave, row, m.n_rows - 1});
     }
     if (m.cbase != nullptr) {
-        return sum(ColBase{gm(reinterpret_cast<const unsigned short*>(m.dcol)) + base + lane, gm(m.cbase)[slice]});
+        return sum(ColBase{gm(reinterpret_cast<const unsigned short*>(m.dcol)) + base, ul, gm(m.cbase)[slice]});
     }
     if (m.dcol != nullptr) {
-        return sum(ColOff{gm(m.dcol) + base + lane, row});
+        return sum(ColOff{gm(m.dcol) + base, ul, row});
     }
-    return sum(ColAbs{gm(m.col) + base + lane});
+    return sum(ColAbs{gm(m.col) + base, ul});
 }
 
 // Row sum of an ELL row: sum_k val_k * x[col_k] in storage order (any column / value format).
@@ -554,12 +562,13 @@ __device__ __forceinline__ T ell_row_x1(const EllView& m, int slice, int lane, c
 }
 
 // Row sums of two slices with equal widths and one column format, their loads issued together
-// (k_ell_group entries of each slice, then the sums in storage order per row): twice the loads in
+// (ell_group entries of each slice, then the sums in storage order per row): twice the loads in
 // flight per wavefront, the same arithmetic as two ell_sum calls.
 template <class T, class V, class C, class F>
 __device__ __forceinline__ void ell_sum2(const C& ca, const C& cb, const gmem_t<const V>* __restrict__ va,
-                                         const gmem_t<const V>* __restrict__ vb, int w, F load, T& sa, T& sb) {
-    constexpr int G = k_ell_group;
+                                         const gmem_t<const V>* __restrict__ vb, unsigned lane, int w, F load, T& sa,
+                                         T& sb) {
+    constexpr int G = ell_group<T>();
     sa = T(0);
     sb = T(0);
     int k = 0;
@@ -577,8 +586,8 @@ __device__ __forceinline__ void ell_sum2(const C& ca, const C& cb, const gmem_t<
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            a0[g] = value_at<T, V>(va, (k + g) * k_wave);
-            a1[g] = value_at<T, V>(vb, (k + g) * k_wave);
+            a0[g] = value_at<T, V>(va + (k + g) * k_wave, lane);
+            a1[g] = value_at<T, V>(vb + (k + g) * k_wave, lane);
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -608,8 +617,8 @@ __device__ __forceinline__ void ell_sum2(const C& ca, const C& cb, const gmem_t<
 #pragma unroll
         for (int g = 0; g < G - 1; ++g) {
             const int kk = g < rem ? k + g : k;
-            a0[g] = value_at<T, V>(va, kk * k_wave);
-            a1[g] = value_at<T, V>(vb, kk * k_wave);
+            a0[g] = value_at<T, V>(va + kk * k_wave, lane);
+            a1[g] = value_at<T, V>(vb + kk * k_wave, lane);
         }
 #pragma unroll
         for (int g = 0; g < G - 1; ++g) {
@@ -651,10 +660,13 @@ __device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int ds, i
         yb = y[1];
         return;
     }
-    const int b0 = m.sp[s0];
-    const int b1 = m.sp[s1];
-    const int w = (m.sp[s0 + 1] - b0) / k_wave;
-    if (w != (m.sp[s1 + 1] - b1) / k_wave) {
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    const unsigned ul = static_cast<unsigned>(lane);
+    const auto sp = gm(m.sp);
+    const int b0 = __builtin_amdgcn_readfirstlane(sp[s0]);
+    const int b1 = __builtin_amdgcn_readfirstlane(sp[s0 + ds]);
+    const int w = (__builtin_amdgcn_readfirstlane(sp[s0 + 1]) - b0) / k_wave;
+    if (w != (__builtin_amdgcn_readfirstlane(sp[s0 + ds + 1]) - b1) / k_wave) {
         ya = ell_row_f<T>(m, s0, lane, load);
         yb = ell_row_f<T>(m, s1, lane, load);
         return;
@@ -668,7 +680,7 @@ __device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int ds, i
                 const auto val = gm(static_cast<const unsigned short*>(m.val));
                 T sa;
                 T sb;
-                ell_sum2<T, unsigned short>(c0, c1, val + b0 + lane, val + b1 + lane, w, load, sa, sb);
+                ell_sum2<T, unsigned short>(c0, c1, val + b0, val + b1, ul, w, load, sa, sb);
                 const T dxa = r0 < m.n_rows ? gm(m.diag)[r0] * load(r0) : T(0);
                 const T dxb = r1 < m.n_rows ? gm(m.diag)[r1] * load(r1) : T(0);
                 ya = madd(gm(m.rscale)[r0], sa, dxa);
@@ -677,19 +689,17 @@ __device__ __forceinline__ void ell_row_pair(const EllView& m, int s0, int ds, i
             }
         }
         const auto val = gm(static_cast<const T*>(m.val));
-        ell_sum2<T, T>(c0, c1, val + b0 + lane, val + b1 + lane, w, load, ya, yb);
+        ell_sum2<T, T>(c0, c1, val + b0, val + b1, ul, w, load, ya, yb);
     };
     if (m.soff != nullptr) {
-        const int t0 = __builtin_amdgcn_readfirstlane(b0 / k_wave);
-        const int t1 = __builtin_amdgcn_readfirstlane(b1 / k_wave);
-        pair(ColStencil{gm(m.soff) + t0, r0, m.n_rows - 1}, ColStencil{gm(m.soff) + t1, r1, m.n_rows - 1});
+        pair(ColStencil{gm(m.soff) + b0 / k_wave, r0, m.n_rows - 1}, ColStencil{gm(m.soff) + b1 / k_wave, r1, m.n_rows - 1});
     } else if (m.cbase != nullptr) {
         const auto dc = gm(reinterpret_cast<const unsigned short*>(m.dcol));
-        pair(ColBase{dc + b0 + lane, gm(m.cbase)[s0]}, ColBase{dc + b1 + lane, gm(m.cbase)[s1]});
+        pair(ColBase{dc + b0, ul, gm(m.cbase)[s0]}, ColBase{dc + b1, ul, gm(m.cbase)[s0 + ds]});
     } else if (m.dcol != nullptr) {
-        pair(ColOff{gm(m.dcol) + b0 + lane, r0}, ColOff{gm(m.dcol) + b1 + lane, r1});
+        pair(ColOff{gm(m.dcol) + b0, ul, r0}, ColOff{gm(m.dcol) + b1, ul, r1});
     } else {
-        pair(ColAbs{gm(m.col) + b0 + lane}, ColAbs{gm(m.col) + b1 + lane});
+        pair(ColAbs{gm(m.col) + b0, ul}, ColAbs{gm(m.col) + b1, ul});
     }
 }
 
@@ -1649,15 +1659,32 @@ __device__ __forceinline__ void op_prolong(const LevelDev& L, const LevelDev& N,
 }
 
 // Coarsest level, row i: v[out]_i = sum_j Cinv_ij b_j in FP64 by one wavefront (lane-strided
-// partial sums, then the wavefront butterfly).
+// partial sums, then the wavefront butterfly). A row's time is its loads' latency: 8 entries a lane
+// are requested before the first is added (all of a row of 512). Order 507 (128^3's tail): 6.6 us one
+// entry at a time, 4.6 so; 2.1 MB.
 template <class T>
 __device__ __forceinline__ void op_coarse_row(const LevelDev& L, int i, int lane, int out) {
-    const int n = L.n;
-    const double* m = L.cinv + static_cast<long long>(i) * n;
+    constexpr int G = 8;
+    const unsigned n = static_cast<unsigned>(L.n);
+    const auto m = gm(L.cinv) + static_cast<long long>(i) * L.n;
     const auto b = gm(static_cast<const T*>(L.b));
     double s = 0.0;
-    for (int j = lane; j < n; j += k_wave) {
-        s += m[j] * static_cast<double>(b[j]);
+    for (unsigned j0 = static_cast<unsigned>(lane); j0 < n; j0 += G * k_wave) {
+        double a[G];
+        T x[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const unsigned j = j0 + static_cast<unsigned>(g * k_wave);
+            const unsigned c = min(j, n - 1);
+            a[g] = load_at<double>(m, c);
+            x[g] = load_at<T>(b, c);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (j0 + static_cast<unsigned>(g * k_wave) < n) {
+                s += a[g] * static_cast<double>(x[g]);
+            }
+        }
     }
     s = wave_sum(s);
     if (lane == 0) {
@@ -1977,7 +2004,7 @@ __global__ void __launch_bounds__(k_block) k_coarse(const SysDev* __restrict__ s
     const int2 bk = block_entry(blocks);
     const SysDev& S = sys[bk.x];
     const LevelDev& L = S.lv[level]; // fields requested with the status (one wait)
-    const int wave = threadIdx.x / k_wave;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / k_wave);
     const int lane = threadIdx.x % k_wave;
     const int i = bk.y * k_slices_per_block + wave;
     if ((S.st->status != ST_RUNNING) | (L.coarsest == 0) | (i >= L.n)) {
