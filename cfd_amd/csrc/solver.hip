@@ -1116,11 +1116,12 @@ void System::set_amg(const cfdg_amg_view& v, bool fuse_wanted) {
     // Dense tail of the FP32 cycle: a level below the finest that is not the coarsest is solved
     // exactly with its dense inverse (computed on the matrix cores) instead of being smoothed and
     // restricted further: the levels under it are launch-bound, and one dense product replaces
-    // their launches. The first level with at most kTailOrder rows takes it, or one with at most
+    // their launches. The first level with at most tail_order rows takes it, or one with at most
     // kDenseWideMaxOrder rows whose inverse holds at most a tenth as many entries as the finest
     // operator: in a batch the launches are shared by all members while every member reads its
     // own inverse, so the larger tails pay off only against a large finest level (CFDG_DENSE_TAIL=0:
     // off).
+    const int tail_order = fuse_wanted ? kTailOrderKept : kTailOrder;
     int tail = 0;
     const char* tenv = std::getenv("CFDG_DENSE_TAIL");
     if (!(tenv != nullptr && std::string(tenv) == "0")) {
@@ -1130,7 +1131,7 @@ void System::set_amg(const cfdg_amg_view& v, bool fuse_wanted) {
         for (int l = 1; l + 1 < L; ++l) {
             const int nl = rows[static_cast<std::size_t>(l)];
             const long long cells = static_cast<long long>(nl) * nl;
-            if (nl > kDenseWideMaxOrder || (nl > kTailOrder && 10 * cells > nnz0)) {
+            if (nl > kDenseWideMaxOrder || (nl > tail_order && 10 * cells > nnz0)) {
                 continue;
             }
             const cfdg_csr& a = v.levels[l].a;
@@ -2019,16 +2020,17 @@ public:
         }
         hip_check(hipEventRecord(t0_.get(), s_), "event record");
         k_init_states<<<ceil_div(n_sys, 64), 64, 0, s_>>>(d, n_sys, init_dev_);
-        if (graphs) {
-            hip_check(hipGraphLaunch(init_exec_, s_), "graph launch");
-        } else {
-            enqueue_init(pl_, d, tb_, s_, report_dev_);
-        }
-        hip_check(hipGetLastError(), "init launch");
         // One iteration past the limit: AMG-PCG finds the limit exceeded at its beginning.
         const long long most = static_cast<long long>(max_it) + 1;
         const int lead = graphs ? queue_depth() : queue_depth() + 1; // launches one by one take the host longer
         long long queued = 0;
+        if (graphs) {
+            hip_check(hipGraphLaunch(init_exec_, s_), "graph launch");
+            queued = std::min(most, static_cast<long long>(k_start_iterations));
+        } else {
+            enqueue_init(pl_, d, tb_, s_, report_dev_);
+        }
+        hip_check(hipGetLastError(), "init launch");
         bool idle = false;
         for (long long polls = 0;; ++polls) {
             bool any = false;
@@ -2146,7 +2148,10 @@ private:
             odd_exec_[k] = capture([&] { iterations(1, 1 << k); });
         }
         even_exec_ = capture([&] { iterations(2, 1); });
-        init_exec_ = capture([&] { enqueue_init(pl_, d, tb_, s_, report_dev_); });
+        init_exec_ = capture([&] {
+            enqueue_init(pl_, d, tb_, s_, report_dev_);
+            iterations(1, k_start_iterations);
+        });
     }
 
 public:
@@ -2175,6 +2180,9 @@ private:
     bool use_graphs_ = true;
     long long solves_ = 0;
     cfdg_precision precision_ = CFDG_PREC_FP64;
+    // The start and the first two iterations (no-ops of a solve that starts converged): one launch
+    // less, and the first residuals tell how many more to queue.
+    static constexpr int k_start_iterations = 2;
     hipGraphExec_t init_exec_ = nullptr;
     hipGraphExec_t even_exec_ = nullptr;                            // one even iteration
     hipGraphExec_t odd_exec_[3] = {nullptr, nullptr, nullptr};      // 1, 2, 4 iterations from an odd one
