@@ -32,10 +32,10 @@ sys.path.insert(0, str(ROOT))
 METRIC = "pressure solves/s @1e-8 rel-res, mixed vs FP64 AMG-PCG; HBM GB/s; p99 ms"
 HBM_PEAK_GBS = 8000.0
 # Kernel names as rocprofv3 reports them (profiles/ and profiles/traffic.json are keyed by these).
-K_SPMV_MIXED = "k_spmv_pz<float, false>"
-K_SPMV_FP64 = "k_spmv_pz<double, false>"
-K_SWEEP_MIXED = "k_jacobi_pair<float, 2>"
-K_SWEEP_FP64 = "k_jacobi<double, 1>"
+K_SPMV_MIXED = "k_spmv_pz<float, 1, 2>"
+K_SPMV_FP64 = "k_spmv_pz<double, 1, 1>"
+K_SWEEP_MIXED = "k_l0_jacobi<float, 1, 2, true>"
+K_SWEEP_FP64 = "k_l0_jacobi<double, 1, 1, false>"
 
 
 def _traffic() -> dict:

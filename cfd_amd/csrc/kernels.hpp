@@ -1280,9 +1280,12 @@ __device__ __forceinline__ double* p_new_of(const SysDev& S, int parity) { retur
 // identical arithmetic), p_new written for the own rows, and the partial p_new.q. z is the level-0
 // V-cycle output v[z_buf] (which = 1, FP64 or FP32) or the Jacobi-preconditioned residual S.z
 // (which = 0).
-// At 128^3 (130 MB from memory in the mixed solve, whose matrix has left the Infinity Cache since the
+// At 128^3 (170 MB from memory in the mixed solve, whose matrix has left the Infinity Cache since the
 // last product) one chunk at a time takes 37.2 us and two 40.8: three arrays of loads a row fill the
-// wavefront's queue already. Before, with the step as a launch of its own: 36.4 + 8.9 us.
+// wavefront's queue already. Before, with the step as a launch of its own: 36.4 + 8.9 us and 130 MB:
+// the groups of an XCD drift apart, and the plane below has left its L2 when it is read again (24
+// bytes a row). Non-temporal stores of p and q don't bring it back (a mixed solve 3.21 -> 3.24 ms, FP64 6.33
+// -> 6.40 ms).
 template <class TZ, int Form, int Op>
 __global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb, int parity,
                           int which, int z_buf, unsigned long long* __restrict__ report) {
