@@ -1358,8 +1358,8 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
     }
     // Row groups per workgroup: one up to 8192 groups in all, so that a single system's few groups
     // spread over the chip; above, the workgroups of a large batch stay near 8192, each making its
-    // kernel's step once for several groups. The line at 2048: 16 systems of 4 k to 500 k cells 2.53
-    // instead of 2.60 ms, 64 such systems (8.0 M cells) 13.86 instead of 13.13 ms; at 4096: 2.58 and
+    // kernel's step once for several groups. The line at 2048: 16 systems of 4 k to 300 k cells 2.53
+    // instead of 2.60 ms, 64 of 4 k to 500 k (8.0 M cells) 13.86 instead of 13.13 ms; at 4096: 2.58 and
     // 13.39 ms; at 16384 both as here.
     long long groups = 0;
     tb.sym7 = true;
@@ -2013,9 +2013,6 @@ public:
         // Graphs from the second solve of a runner on: one-shot solves skip the capture cost.
         const bool graphs = use_graphs_ && probe == nullptr && solves_ > 0;
         ++solves_;
-        if (graphs && init_exec_ == nullptr) {
-            capture_graphs();
-        }
         for (std::size_t i = 0; i < sys_.size(); ++i) {
             report_[i] = k_report_none;
             forecast_[i].reset(control[i].abs_tolerance);
@@ -2027,7 +2024,10 @@ public:
         const int lead = graphs ? queue_depth() : queue_depth() + 1; // launches one by one take the host longer
         long long queued = 0;
         if (graphs) {
-            hip_check(hipGraphLaunch(init_exec_, s_), "graph launch");
+            launch(init_exec_, [&] {
+                enqueue_init(pl_, d, tb_, s_, report_dev_);
+                enqueue_steps(1, k_start_iterations);
+            });
             queued = std::min(most, static_cast<long long>(k_start_iterations));
         } else {
             enqueue_init(pl_, d, tb_, s_, report_dev_);
@@ -2120,40 +2120,38 @@ private:
             return 1;
         }
         if (!odd) {
-            hip_check(hipGraphLaunch(even_exec_, s_), "graph launch");
+            launch(even_exec_, [&] { enqueue_steps(2, 1); });
             return 1;
         }
         const int k = want >= 4 ? 2 : want >= 2 ? 1 : 0;
-        hip_check(hipGraphLaunch(odd_exec_[k], s_), "graph launch");
+        launch(odd_exec_[k], [&] { enqueue_steps(1, 1 << k); });
         return 1LL << k;
     }
 
-    void capture_graphs() {
-        const SysDev* d = desc_.get();
-        auto capture = [&](auto&& enqueue) {
+    // `count` iterations from iteration `first` on and the residual test of the last.
+    void enqueue_steps(int first, int count) {
+        for (int k = first; k < first + count; ++k) {
+            enqueue_iteration(pl_, desc_.get(), tb_, s_, k & 1, report_dev_);
+        }
+        enqueue_check(pl_, desc_.get(), tb_, s_, report_dev_);
+    }
+
+    // Launches the graph of what `enqueue` queues, captured at its first use: a solve captures no
+    // graph that it does not need, and all but the first while the device works on those before it.
+    // Second FP64 solves of 40 systems of 4 k to 500 k cells: 1.65 ms on average; with the five graphs
+    // captured first 1.98 ms.
+    template <class F>
+    void launch(hipGraphExec_t& exec, F&& enqueue) {
+        if (exec == nullptr) {
             hipGraph_t g = nullptr;
             hip_check(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal), "begin capture");
             enqueue();
             hip_check(hipStreamEndCapture(s_, &g), "end capture");
-            hipGraphExec_t e = nullptr;
-            hip_check(hipGraphInstantiate(&e, g, nullptr, nullptr, 0), "graph instantiate");
+            const hipError_t made = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
             hip_check(hipGraphDestroy(g), "graph destroy");
-            return e;
-        };
-        auto iterations = [&](int first, int count) {
-            for (int k = first; k < first + count; ++k) {
-                enqueue_iteration(pl_, d, tb_, s_, k & 1, report_dev_);
-            }
-            enqueue_check(pl_, d, tb_, s_, report_dev_);
-        };
-        for (int k = 0; k < 3; ++k) {
-            odd_exec_[k] = capture([&] { iterations(1, 1 << k); });
+            hip_check(made, "graph instantiate");
         }
-        even_exec_ = capture([&] { iterations(2, 1); });
-        init_exec_ = capture([&] {
-            enqueue_init(pl_, d, tb_, s_, report_dev_);
-            iterations(1, k_start_iterations);
-        });
+        hip_check(hipGraphLaunch(exec, s_), "graph launch");
     }
 
 public:
