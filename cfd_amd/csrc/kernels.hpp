@@ -90,13 +90,31 @@ __device__ __forceinline__ gmem_t<T>* gm(T* p) {
 // registers and the address is one 32-bit byte offset per lane (i sizeof(T) < 2^32), which all the
 // loads of a row share.
 template <class T>
-__device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, unsigned i) {
+__host__ __device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, unsigned i) {
     return *(const gmem_t<const T>*)((const gmem_t<const char>*)base + i * static_cast<unsigned>(sizeof(T)));
 }
 
 template <class T>
-__device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, unsigned i, T v) {
+__host__ __device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, unsigned i, T v) {
     *(gmem_t<T>*)((gmem_t<char>*)base + i * static_cast<unsigned>(sizeof(T))) = v;
+}
+
+// A lane's row in a slice of 64, for arrays of any length: the slice's first row, the same for the
+// whole wavefront, moves the scalar base, and only the lane's place in the slice is a vector offset.
+struct LaneRow {
+    long long start;
+    unsigned lane;
+    int left; // rows from start to the end of the matrix; at most 0 past it
+};
+
+template <class T>
+__host__ __device__ __forceinline__ T load_at(const gmem_t<const T>* __restrict__ base, const LaneRow& r) {
+    return load_at<T>(base + r.start, r.lane);
+}
+
+template <class T>
+__host__ __device__ __forceinline__ void store_at(gmem_t<T>* __restrict__ base, const LaneRow& r, T v) {
+    store_at<T>(base + r.start, r.lane, v);
 }
 
 // Column index of the lane's entry in the 64 slots from k on (uniform over the wavefront): 32-bit
@@ -1176,14 +1194,43 @@ __device__ __forceinline__ void group_rows(const SysDev& S, int g, int wave, R r
     }
 }
 
+// How a level-0 kernel names a lane's row. Symmetric storage has fewer than 2^29 rows (System builds
+// it for no more), so that its row number alone is the offset that a row's own loads and its stencil's
+// share; the other forms take systems of any size.
+template <int Form>
+using RowOf = std::conditional_t<Form == L0_SYM7, unsigned, LaneRow>;
+
+__host__ __device__ __forceinline__ void set_row(unsigned& r, int slice, int lane, int) {
+    r = static_cast<unsigned>(slice) * k_wave + static_cast<unsigned>(lane);
+}
+__host__ __device__ __forceinline__ void set_row(LaneRow& r, int slice, int lane, int n) {
+    r.start = static_cast<long long>(slice) * k_wave;
+    r.lane = static_cast<unsigned>(lane);
+    r.left = static_cast<int>(n - r.start);
+}
+__host__ __device__ __forceinline__ bool inside(unsigned r, int n) { return r < static_cast<unsigned>(n); }
+__host__ __device__ __forceinline__ bool inside(const LaneRow& r, int) { return static_cast<int>(r.lane) < r.left; }
+
+// The row, or some row of the matrix for one past its end.
+__host__ __device__ __forceinline__ unsigned in_matrix(unsigned r, int n) {
+    const unsigned last = static_cast<unsigned>(n) - 1;
+    return r < last ? r : last;
+}
+__host__ __device__ __forceinline__ LaneRow in_matrix(const LaneRow& r, int) {
+    LaneRow c = r;
+    c.start = r.left > 0 ? r.start : 0;
+    c.lane = static_cast<int>(r.lane) < r.left ? r.lane : 0;
+    return c;
+}
+
 // The lane's rows of slices slice and (Rows == 2) slice + ds; load(h, r) requests what a row's result
-// needs of its own entries, before the row sums' loads (rows past the end: of the last row).
-template <int Rows, class F>
-__device__ __forceinline__ void own_rows(int slice, int ds, int lane, unsigned n, unsigned (&row)[2], F load) {
+// needs of its own entries, before the row sums' loads (rows past the end: of some other row).
+template <int Rows, class Row, class F>
+__host__ __device__ __forceinline__ void own_rows(int slice, int ds, int lane, int n, Row (&row)[2], F load) {
 #pragma unroll
     for (int h = 0; h < Rows; ++h) {
-        row[h] = static_cast<unsigned>((slice + h * ds) * k_wave + lane);
-        load(h, min(row[h], n - 1));
+        set_row(row[h], slice + h * ds, lane, n);
+        load(h, in_matrix(row[h], n));
     }
 }
 
@@ -1294,7 +1341,7 @@ __global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ 
     const auto po = gm(static_cast<const double*>(p_old_of(S, parity)));
     const auto pn = gm(p_new_of(S, parity));
     const auto qv = gm(S.q);
-    const unsigned n = static_cast<unsigned>(S.n);
+    const int n = S.n;
     L0Op<Form, double, GatherPz<TZ>> A0(S.a64, {z, po, 0.0});
     const Scalars st = take_step<Op>(S, first_, report, bk_.x);
     if (st.status != ST_RUNNING) {
@@ -1304,12 +1351,12 @@ __global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ 
     for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
         double y[2];
         double pi[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { pi[h] = static_cast<double>(load_at<TZ>(z, r)) + st.beta * load_at<double>(po, r); });
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) { pi[h] = static_cast<double>(load_at<TZ>(z, r)) + st.beta * load_at<double>(po, r); });
         l0_rows<H.value>(A0, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 store_at<double>(pn, row[h], pi[h]);
                 store_at<double>(qv, row[h], y[h]);
                 v[0] += pi[h] * y[h];
@@ -1373,16 +1420,16 @@ __global__ void __launch_bounds__(k_block) k_true_residual(const SysDev* __restr
     CFDG_L0_PROLOGUE(sys, blocks)
     const auto b = gm(S.b);
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
-    const unsigned n = static_cast<unsigned>(S.n);
+    const int n = S.n;
     for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
         double y[2];
         double bi[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { bi[h] = load_at<double>(b, r); });
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) { bi[h] = load_at<double>(b, r); });
         l0_rows<H.value>(A0, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 const double ri = bi[h] - y[h];
                 v[0] += ri * ri;
             }
@@ -1450,19 +1497,19 @@ __global__ void __launch_bounds__(k_block) k_bicg_v(const SysDev* __restrict__ s
     const auto vv = gm(S.v);
     const auto r0 = gm(static_cast<const double*>(S.r0));
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.ph))});
-    const unsigned n = static_cast<unsigned>(S.n);
+    const int n = S.n;
     if (S.st->status != ST_RUNNING) {
         return;
     }
     for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
         double y[2];
         double ri[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { ri[h] = load_at<double>(r0, r); });
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) { ri[h] = load_at<double>(r0, r); });
         l0_rows<H.value>(A0, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 store_at<double>(vv, row[h], y[h]);
                 v[0] += ri[h] * y[h];
             }
@@ -1504,7 +1551,7 @@ __global__ void __launch_bounds__(k_block) k_bicg_t(const SysDev* __restrict__ s
     const auto x = gm(S.x);
     const auto ph = gm(static_cast<const double*>(S.ph));
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.sh))});
-    const unsigned n = static_cast<unsigned>(S.n);
+    const int n = S.n;
     const Scalars st = take_step<FIN_BICG_S>(S, first_, nullptr, 0);
     if (st.status == ST_CONVERGED_PENDING) {
         for_group_rows<false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int) {
@@ -1521,12 +1568,12 @@ __global__ void __launch_bounds__(k_block) k_bicg_t(const SysDev* __restrict__ s
     for_groups<2, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2]) {
         double y[2];
         double si[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { si[h] = load_at<double>(sv, r); });
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) { si[h] = load_at<double>(sv, r); });
         l0_rows<H.value>(A0, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 store_at<double>(tv, row[h], y[h]);
                 v[0] += y[h] * y[h];
                 v[1] += y[h] * si[h];
@@ -1668,7 +1715,7 @@ __device__ __forceinline__ void op_prolong(const LevelDev& L, const LevelDev& N,
 template <class T>
 __device__ __forceinline__ void op_coarse_row(const LevelDev& L, int i, int lane, int out) {
     constexpr int G = 8;
-    const unsigned n = static_cast<unsigned>(L.n);
+    const int n = L.n;
     const auto m = gm(L.cinv) + static_cast<long long>(i) * L.n;
     const auto b = gm(static_cast<const T*>(L.b));
     double s = 0.0;
@@ -1754,19 +1801,19 @@ __global__ void __launch_bounds__(k_block) k_l0_residual_x1(const SysDev* __rest
     const auto b = gm(static_cast<const T*>(L.b));
     const auto t = gm(static_cast<T*>(L.v[out]));
     const L0Op<Form, T, GatherX1<T>> M(L.a, {gm(static_cast<const T*>(L.wd)), b, f});
-    const unsigned n = static_cast<unsigned>(L.n);
+    const int n = L.n;
     if (!cycle_runs<Step>(S, first_, report, bk_.x) | (L.coarsest != 0)) {
         return;
     }
     for_group_rows<true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds) {
         T y[2];
         T bi[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) { bi[h] = load_at<T>(b, r); });
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) { bi[h] = load_at<T>(b, r); });
         l0_rows<H.value>(M, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 store_at<T>(t, row[h], bi[h] - y[h]);
             }
         }
@@ -1785,7 +1832,7 @@ __global__ void __launch_bounds__(k_block) k_l0_presmooth2(const SysDev* __restr
     const auto wd = gm(static_cast<const T*>(L.wd));
     const auto x = gm(static_cast<T*>(L.v[out]));
     const L0Op<Form, T, GatherX1<T>> M(L.a, {wd, b, f1});
-    const unsigned n = static_cast<unsigned>(L.n);
+    const int n = L.n;
     if (!cycle_runs<Step>(S, first_, report, bk_.x) | (L.coarsest != 0)) {
         return;
     }
@@ -1793,15 +1840,15 @@ __global__ void __launch_bounds__(k_block) k_l0_presmooth2(const SysDev* __restr
         T y[2];
         T bi[2];
         T wi[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned r) {
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& r) {
             bi[h] = load_at<T>(b, r);
             wi[h] = load_at<T>(wd, r);
         });
         l0_rows<H.value>(M, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 const T x1 = (f1 * wi[h]) * bi[h];
                 store_at<T>(x, row[h], x1 + (f2 * wi[h]) * (bi[h] - y[h]));
             }
@@ -1825,7 +1872,7 @@ __global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict_
     const auto r = gm(static_cast<const double*>(S.r));
     const auto qv = gm(static_cast<const double*>(S.q));
     const L0Op<Form, T, GatherX<T>> M(L.a, {x});
-    const unsigned n = static_cast<unsigned>(L.n);
+    const int n = L.n;
     if ((S.st->status != ST_RUNNING) | (L.coarsest != 0)) {
         return;
     }
@@ -1836,8 +1883,8 @@ __global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict_
         T xi[2];
         double ri[2];
         double qi[2];
-        unsigned row[2];
-        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, unsigned i) {
+        RowOf<Form> row[2];
+        own_rows<H.value>(slice, ds, lane, n, row, [&](int h, const auto& i) {
             bi[h] = load_at<T>(b, i);
             wi[h] = load_at<T>(wd, i);
             xi[h] = load_at<T>(x, i);
@@ -1849,7 +1896,7 @@ __global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict_
         l0_rows<H.value>(M, slice, ds, lane, y);
 #pragma unroll
         for (int h = 0; h < H.value; ++h) {
-            if (row[h] < n) {
+            if (inside(row[h], n)) {
                 const T z = xi[h] + (f * wi[h]) * (bi[h] - y[h]);
                 store_at<T>(o, row[h], z);
                 const double zd = static_cast<double>(z);
