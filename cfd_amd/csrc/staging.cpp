@@ -7,19 +7,16 @@
 // its own. The set-up's copies keep the OpenMP team that runs the loops around them: more threads
 // beside its spinning workers exceed a CPU quota of the team's size, and the process is stopped for
 // the rest of the scheduler's period (set-up 4% slower, the first solve after it up to 5 ms).
+#include "copy_team.hpp"
 #include "hip_util.hpp"
 
 #include <omp.h>
 
 #include <algorithm>
-#include <atomic>
-#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
+#include <memory>
 #include <mutex>
-#include <thread>
-#include <vector>
 
 namespace cfdg {
 
@@ -46,7 +43,6 @@ constexpr std::size_t k_chunk = std::size_t(16) << 20; // bytes per chunk; two c
 constexpr std::size_t k_slot = std::size_t(4) << 20; // d2h_copies' share of a chunk
 constexpr int k_slots_per_chunk = static_cast<int>(k_chunk / k_slot);
 constexpr int k_ring = 2 * k_slots_per_chunk;        // its slots per area
-constexpr int k_helpers = 3;                         // its threads beside the caller: seven gain nothing
 
 // Bytes per piece of d2h_copies: small enough that a copy's first and last pieces, which nothing
 // overlaps, are a small part of it, large enough for the 10 us that each costs. Measured with 1, 2
@@ -61,6 +57,27 @@ struct Area {
     hipEvent_t done[2] = {nullptr, nullptr};
     hipEvent_t slot_done[k_ring] = {};
     int device = -1;
+    Area* next = nullptr; // in the free list
+    Area() = default;
+    Area(const Area&) = delete;
+    Area& operator=(const Area&) = delete;
+    ~Area() {
+        for (char* b : buf) {
+            if (b != nullptr) {
+                (void)hipHostFree(b);
+            }
+        }
+        for (hipEvent_t e : done) {
+            if (e != nullptr) {
+                (void)hipEventDestroy(e);
+            }
+        }
+        for (hipEvent_t e : slot_done) {
+            if (e != nullptr) {
+                (void)hipEventDestroy(e);
+            }
+        }
+    }
     [[nodiscard]] char* slot(int i) const {
         return buf[i / k_slots_per_chunk] + static_cast<std::size_t>(i % k_slots_per_chunk) * k_slot;
     }
@@ -69,20 +86,20 @@ struct Area {
 thread_local bool t_host_parallel = true;
 
 std::mutex g_mutex;
-std::vector<Area*> g_free;
+Area* g_free = nullptr;
 
 Area* acquire(int device) {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        for (std::size_t i = 0; i < g_free.size(); ++i) {
-            if (g_free[i]->device == device) {
-                Area* a = g_free[i];
-                g_free.erase(g_free.begin() + static_cast<std::ptrdiff_t>(i));
+        for (Area** at = &g_free; *at != nullptr; at = &(*at)->next) {
+            if ((*at)->device == device) {
+                Area* a = *at;
+                *at = a->next;
                 return a;
             }
         }
     }
-    auto* a = new Area;
+    auto a = std::make_unique<Area>();
     a->device = device;
     for (int k = 0; k < 2; ++k) {
         hip_check(hipHostMalloc(reinterpret_cast<void**>(&a->buf[k]), k_chunk, hipHostMallocDefault),
@@ -92,12 +109,13 @@ Area* acquire(int device) {
     for (hipEvent_t& e : a->slot_done) {
         hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "staging event");
     }
-    return a;
+    return a.release();
 }
 
-void release(Area* a) {
+void release(Area* a) noexcept {
     std::lock_guard<std::mutex> lock(g_mutex);
-    g_free.push_back(a);
+    a->next = g_free;
+    g_free = a;
 }
 
 // Host memcpy split over the host threads for large blocks.
@@ -114,71 +132,6 @@ void host_copy(char* dst, const char* src, std::size_t n) {
         std::memcpy(dst + o, src + o, n - o < piece ? n - o : piece);
     }
 }
-
-// Helper threads of the copies, started with the first one and asleep between copies; a copy that
-// finds them busy with others goes on alone. (OpenMP teams instead: a team of another size than the
-// last region's is rebuilt, and a call took up to milliseconds longer.) Never destroyed: the threads
-// may outlive static objects.
-class Helpers {
-public:
-    static Helpers& get() {
-        static Helpers* h = new Helpers;
-        return *h;
-    }
-    // Runs work() on the caller and on the helpers that wake in time; returns when every one of them
-    // has returned from it.
-    void run(const std::function<void()>& work) {
-        Job job{&work, 0};
-        {
-            std::lock_guard<std::mutex> lock(m_);
-            jobs_.push_back(&job);
-        }
-        wake_.notify_all();
-        work();
-        std::unique_lock<std::mutex> lock(m_);
-        jobs_.erase(std::find(jobs_.begin(), jobs_.end(), &job));
-        done_.wait(lock, [&] { return job.users == 0; });
-    }
-
-private:
-    struct Job {
-        const std::function<void()>* work;
-        int users;
-        bool taken[k_helpers] = {};
-    };
-    Helpers() {
-        for (int k = 0; k < k_helpers; ++k) {
-            std::thread([this, k] { loop(k); }).detach();
-        }
-    }
-    void loop(int k) {
-        std::unique_lock<std::mutex> lock(m_);
-        for (;;) {
-            Job* job = nullptr;
-            wake_.wait(lock, [&] {
-                for (Job* j : jobs_) {
-                    if (!j->taken[k]) {
-                        job = j;
-                        return true;
-                    }
-                }
-                return false;
-            });
-            job->taken[k] = true;
-            ++job->users;
-            lock.unlock();
-            (*job->work)();
-            lock.lock();
-            if (--job->users == 0) {
-                done_.notify_all();
-            }
-        }
-    }
-    std::mutex m_;
-    std::condition_variable wake_;
-    std::condition_variable done_;
-    std::vector<Job*> jobs_;
-};
 
 } // namespace
 
@@ -268,82 +221,52 @@ void d2h_staged(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
 
 namespace {
 
-// Copies the pieces of a list from the device through the ring of one area, piece i through slot
-// i mod k_ring: queued on s as soon as the slot's previous piece has been copied out, then copied out
-// by the thread that took it when it has arrived. A thread takes pieces in order, so a piece that
-// another one waits for is always already taken; queued[slot] is the number of the piece that was
-// last queued through the slot.
-hipError_t copy_pieces(const HostCopy* list, int n, Area& a, hipStream_t s, std::size_t piece) {
-    struct Piece {
+// The device's side of d2h_copies: the pieces of a list of copies, through the slots of one area.
+struct PieceCopy {
+    const HostCopy* list;
+    int n;
+    std::size_t piece;
+    Area& a;
+    hipStream_t s;
+
+    struct Part {
         const char* dev;
         char* host;
         std::size_t bytes;
     };
-    std::vector<Piece> pieces;
-    for (int k = 0; k < n; ++k) {
-        for (std::size_t o = 0; o < list[k].bytes; o += piece) {
-            pieces.push_back({static_cast<const char*>(list[k].dev) + o, static_cast<char*>(list[k].host) + o,
-                              std::min(piece, list[k].bytes - o)});
+    [[nodiscard]] int count() const {
+        std::size_t c = 0;
+        for (int k = 0; k < n; ++k) {
+            c += pieces(list[k].bytes);
         }
+        return static_cast<int>(c);
     }
-    const int count = static_cast<int>(pieces.size());
-    std::atomic<int> next{0};
-    std::atomic<int> error{static_cast<int>(hipSuccess)};
-    std::atomic<int> queued[k_ring];
-    for (auto& q : queued) {
-        q.store(-1);
+    [[nodiscard]] std::size_t pieces(std::size_t bytes) const { return (bytes + piece - 1) / piece; }
+    [[nodiscard]] Part part(int i) const {
+        std::size_t j = static_cast<std::size_t>(i);
+        const HostCopy* c = list;
+        for (; j >= pieces(c->bytes); ++c) {
+            j -= pieces(c->bytes);
+        }
+        const std::size_t o = j * piece;
+        return {static_cast<const char*>(c->dev) + o, static_cast<char*>(c->host) + o, std::min(piece, c->bytes - o)};
     }
-    auto failed = [&] { return error.load(std::memory_order_relaxed) != static_cast<int>(hipSuccess); };
-    auto check = [&](hipError_t e) {
-        if (e != hipSuccess) {
-            error.store(static_cast<int>(e));
-        }
-        return e == hipSuccess;
-    };
-    auto queue = [&](int i) {
-        const Piece& p = pieces[static_cast<std::size_t>(i)];
-        const int slot = i % k_ring;
-        (void)(check(hipMemcpyAsync(a.slot(slot), p.dev, p.bytes, hipMemcpyDeviceToHost, s)) &&
-               check(hipEventRecord(a.slot_done[slot], s)));
-        queued[slot].store(i, std::memory_order_release);
-    };
-    auto wait = [&](int i) { // until piece i, queued by whichever thread, has arrived
-        const int slot = i % k_ring;
-        while (queued[slot].load(std::memory_order_acquire) < i && !failed()) {
-        }
-        while (!failed()) {
-            const hipError_t e = hipEventQuery(a.slot_done[slot]);
-            if (e == hipSuccess) {
-                return;
-            }
-            if (e != hipErrorNotReady) {
-                check(e);
-            }
-        }
-    };
-    for (int i = 0; i < std::min(count, k_ring) && !failed(); ++i) {
-        queue(i);
+    [[nodiscard]] int enter() const { return hipSetDevice(a.device); }
+    [[nodiscard]] int queue(int i, int slot) const {
+        const Part p = part(i);
+        const hipError_t e = hipMemcpyAsync(a.slot(slot), p.dev, p.bytes, hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipEventRecord(a.slot_done[slot], s);
     }
-    const std::function<void()> work = [&] {
-        check(hipSetDevice(a.device));
-        for (int i = next.fetch_add(1); i < count && !failed(); i = next.fetch_add(1)) {
-            const Piece& p = pieces[static_cast<std::size_t>(i)];
-            wait(i);
-            if (!failed()) {
-                std::memcpy(p.host, a.slot(i % k_ring), p.bytes);
-            }
-            if (i + k_ring < count) {
-                queue(i + k_ring);
-            }
-        }
-    };
-    if (t_host_parallel) {
-        Helpers::get().run(work);
-    } else {
-        work();
+    [[nodiscard]] int arrived(int slot, bool& yes) const {
+        const hipError_t e = hipEventQuery(a.slot_done[slot]);
+        yes = e == hipSuccess;
+        return e == hipErrorNotReady ? hipSuccess : e;
     }
-    return static_cast<hipError_t>(error.load());
-}
+    void copy_out(int i, int slot) const {
+        const Part p = part(i);
+        std::memcpy(p.host, a.slot(slot), p.bytes);
+    }
+};
 
 } // namespace
 
@@ -363,11 +286,13 @@ void d2h_copies(const HostCopy* list, int n, hipStream_t s) {
     }
     int device = 0;
     hip_check(hipGetDevice(&device), "hipGetDevice");
-    Area* a = acquire(device);
-    const hipError_t e = copy_pieces(list, n, *a, s, piece_bytes(total));
+    Area* a = acquire(device); // nothing below throws before it is released
+    PieceCopy pieces{list, n, piece_bytes(total), *a, s};
+    RingCopy<k_ring, PieceCopy> ring(pieces, pieces.count());
+    const int e = ring.run(t_host_parallel ? &CopyTeam::get() : nullptr);
     const hipError_t w = hipStreamSynchronize(s); // the area is free again
     release(a);
-    hip_check(e, "D2H copy");
+    hip_check(static_cast<hipError_t>(e), "D2H copy");
     hip_check(w, "D2H copy sync");
 }
 
