@@ -41,7 +41,7 @@ void h2d_staged(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 void d2h_staged(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 constexpr std::size_t k_staged_min_bytes = std::size_t(4) << 20;
 
-// Results copied to pageable host arrays, several in one call, by a few threads through pinned
+// Results copied to pageable host arrays, several in one call, through pinned
 // staging from k_pieces_min_bytes in all (staging.cpp; below, the runtime's copy is as fast).
 struct HostCopy {
     const void* dev;

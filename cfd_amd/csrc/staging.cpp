@@ -3,10 +3,11 @@
 // (or out of) pinned chunks while the DMA engine moves the previous chunk. Staging areas come
 // from a process-wide free list (one per concurrent caller, kept until the process ends).
 //
-// The results of solves and finite-volume calls (d2h_copies) take a finer pipeline with threads of
-// its own. The set-up's copies keep the OpenMP team that runs the loops around them: more threads
-// beside its spinning workers exceed a CPU quota of the team's size, and the process is stopped for
-// the rest of the scheduler's period (set-up 4% slower, the first solve after it up to 5 ms).
+// The results of solves and finite-volume calls (d2h_copies) take a finer pipeline, by the caller and, if
+// they are large, helper threads of its own (copy_team.hpp). The set-up's copies keep the OpenMP team that
+// runs the loops around them: more threads beside its spinning workers exceed a CPU quota of the team's
+// size, and the process is stopped for the rest of the scheduler's period (set-up 4% slower, the first
+// solve after it up to 5 ms).
 #include "copy_team.hpp"
 #include "hip_util.hpp"
 
@@ -17,6 +18,8 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <new>
+#include <type_traits>
 
 namespace cfdg {
 
@@ -40,14 +43,20 @@ __attribute__((constructor)) void short_omp_blocktime() {
 
 constexpr std::size_t k_chunk = std::size_t(16) << 20; // bytes per chunk; two chunks per area
 
+
+// Helper threads of d2h_copies: one, with which the caller keeps up with the link (16 MiB 0.48 ms, 0.52
+// alone, with three 0.49, through the runtime 0.95); from k_large_copy on, where malloc hands out fresh pages each time and
+// the copy waits for their zeroing, all of them (32 MiB 1.05 ms, with one 1.8, alone 2.0).
+constexpr std::size_t k_large_copy = std::size_t(24) << 20;
+constexpr int helpers_of(std::size_t total) { return total >= k_large_copy ? CopyTeam::k_helpers : 1; }
+
 constexpr std::size_t k_slot = std::size_t(4) << 20; // d2h_copies' share of a chunk
 constexpr int k_slots_per_chunk = static_cast<int>(k_chunk / k_slot);
 constexpr int k_ring = 2 * k_slots_per_chunk;        // its slots per area
 
 // Bytes per piece of d2h_copies: small enough that a copy's first and last pieces, which nothing
-// overlaps, are a small part of it, large enough for the 10 us that each costs. Measured with 1, 2
-// and 4 MiB (us): 4 MiB 221, 201, 259; 17 MiB 642, 555, 565 (1025 through the runtime, whose one
-// thread copies while the link waits); 64 MiB 2610, 2640, 2336 (6773).
+// overlaps, are a small part of it, large enough for the 10 us that each costs. 2 and 4 MiB at 200 MiB: 6.9
+// and 5.6 ms; 1, 2 and 4 MiB at 17 MiB: 642, 555 and 565 us.
 constexpr std::size_t piece_bytes(std::size_t total) {
     return total > (std::size_t(32) << 20) ? k_slot : std::size_t(2) << 20;
 }
@@ -58,6 +67,7 @@ struct Area {
     hipEvent_t slot_done[k_ring] = {};
     int device = -1;
     Area* next = nullptr; // in the free list
+    alignas(64) unsigned char copy[512]; // d2h_copies' state, used by a late helper after the call returned
     Area() = default;
     Area(const Area&) = delete;
     Area& operator=(const Area&) = delete;
@@ -223,10 +233,10 @@ namespace {
 
 // The device's side of d2h_copies: the pieces of a list of copies, through the slots of one area.
 struct PieceCopy {
-    const HostCopy* list;
+    const HostCopy* list; // the caller's
     int n;
     std::size_t piece;
-    Area& a;
+    Area* a;
     hipStream_t s;
 
     struct Part {
@@ -251,22 +261,30 @@ struct PieceCopy {
         const std::size_t o = j * piece;
         return {static_cast<const char*>(c->dev) + o, static_cast<char*>(c->host) + o, std::min(piece, c->bytes - o)};
     }
-    [[nodiscard]] int enter() const { return hipSetDevice(a.device); }
     [[nodiscard]] int queue(int i, int slot) const {
         const Part p = part(i);
-        const hipError_t e = hipMemcpyAsync(a.slot(slot), p.dev, p.bytes, hipMemcpyDeviceToHost, s);
-        return e != hipSuccess ? e : hipEventRecord(a.slot_done[slot], s);
+        const hipError_t e = hipMemcpyAsync(a->slot(slot), p.dev, p.bytes, hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipEventRecord(a->slot_done[slot], s);
     }
     [[nodiscard]] int arrived(int slot, bool& yes) const {
-        const hipError_t e = hipEventQuery(a.slot_done[slot]);
+        const hipError_t e = hipEventQuery(a->slot_done[slot]);
         yes = e == hipSuccess;
         return e == hipErrorNotReady ? hipSuccess : e;
     }
-    void copy_out(int i, int slot) const {
+    [[nodiscard]] bool copy_out(int i, int slot, int k) const {
+        constexpr std::size_t step = std::size_t(256) << 10; // 20 us
         const Part p = part(i);
-        std::memcpy(p.host, a.slot(slot), p.bytes);
+        const std::size_t o = static_cast<std::size_t>(k) * step;
+        std::memcpy(p.host + o, a->slot(slot) + o, std::min(step, p.bytes - o));
+        return o + step < p.bytes;
     }
+    void drain() const { (void)hipStreamSynchronize(s); }
+    void leave() const { release(a); }
 };
+
+using Copy = RingCopy<k_ring, PieceCopy>;
+static_assert(sizeof(Copy) <= sizeof(Area::copy) && alignof(Copy) <= 64 && std::is_trivially_destructible_v<Copy>,
+              "a copy lives in its area until the area is used again");
 
 } // namespace
 
@@ -286,14 +304,11 @@ void d2h_copies(const HostCopy* list, int n, hipStream_t s) {
     }
     int device = 0;
     hip_check(hipGetDevice(&device), "hipGetDevice");
-    Area* a = acquire(device); // nothing below throws before it is released
-    PieceCopy pieces{list, n, piece_bytes(total), *a, s};
-    RingCopy<k_ring, PieceCopy> ring(pieces, pieces.count());
-    const int e = ring.run(t_host_parallel ? &CopyTeam::get() : nullptr);
-    const hipError_t w = hipStreamSynchronize(s); // the area is free again
-    release(a);
+    Area* a = acquire(device);
+    const PieceCopy pieces{list, n, piece_bytes(total), a, s};
+    Copy* copy = new (a->copy) Copy(pieces, pieces.count());
+    const int e = copy->run(t_host_parallel ? &CopyTeam::get() : nullptr, helpers_of(total));
     hip_check(static_cast<hipError_t>(e), "D2H copy");
-    hip_check(w, "D2H copy sync");
 }
 
 } // namespace cfdg

@@ -1,7 +1,8 @@
 """The helper threads and the slot ring of the result copies (copy_team.hpp), on the host with a stand-in
 for the device: every piece arrives once and unchanged with any number of helpers, also with those that
-the system refuses to start, from several callers at once, and a failure in any piece ends the copy with
-its error."""
+the system refuses to start, from several callers at once; a failure in any piece ends the copy with its
+error; the device is only called by the caller, and the caller waits for a helper only while that one
+copies a piece."""
 from __future__ import annotations
 
 import shutil
@@ -19,11 +20,16 @@ PROGRAM = r"""
 #include <dlfcn.h>
 #include <pthread.h>
 
+#include <algorithm>
 #include <cerrno>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <vector>
+
+using cfdg::CopyTeam;
 
 static int allowed = 1 << 30; // threads that may still be started
 
@@ -38,41 +44,85 @@ struct Fake {
     static constexpr int ring = 8;
     std::vector<char> dev, host, slots;
     std::vector<int> copied, asked;
-    int fail_queue = -1, fail_arrive = -1;
+    std::thread::id caller = std::this_thread::get_id();
+    int fail_queue = -1, fail_arrive = -1, strangers = 0, drained = 0;
+    std::atomic<int> left{0};
+    static inline std::atomic<int> helpers{0};
     explicit Fake(int n) : dev(n * bytes), host(n * bytes), slots(ring * bytes), copied(n), asked(ring) {
         for (std::size_t i = 0; i < dev.size(); ++i) {
             dev[i] = static_cast<char>(i * 7 + i / 251);
         }
     }
-    int enter() { return 0; }
-    int queue(int i, int slot) {
-        if (i == fail_queue) {
-            return 11;
-        }
-        std::memcpy(&slots[slot * bytes], &dev[i * bytes], bytes);
-        asked[slot] = 0;
-        return 0;
-    }
-    int arrived(int slot, bool& yes) {
-        yes = ++asked[slot] >= 3;
-        return slot == fail_arrive ? 22 : 0;
-    }
-    void copy_out(int i, int slot) {
-        std::memcpy(&host[i * bytes], &slots[slot * bytes], bytes);
-        ++copied[i];
-    }
 };
 
-static int copy(Fake& f, cfdg::CopyTeam* team) {
-    return cfdg::RingCopy<Fake::ring, Fake>(f, static_cast<int>(f.copied.size())).run(team);
+struct Device {
+    Fake* f;
+    int queue(int i, int slot) const {
+        f->strangers += std::this_thread::get_id() != f->caller;
+        if (i == f->fail_queue) {
+            return 11;
+        }
+        std::memcpy(&f->slots[slot * f->bytes], &f->dev[i * f->bytes], f->bytes);
+        f->asked[slot] = 0;
+        return 0;
+    }
+    int arrived(int slot, bool& yes) const {
+        f->strangers += std::this_thread::get_id() != f->caller;
+        yes = ++f->asked[slot] >= 3;
+        return slot == f->fail_arrive ? 22 : 0;
+    }
+    bool copy_out(int i, int slot, int part) const {
+        const std::size_t o = part * f->bytes / 4;
+        std::memcpy(&f->host[i * f->bytes + o], &f->slots[slot * f->bytes + o], f->bytes / 4);
+        ++f->copied[i];
+        return part < 3;
+    }
+    void drain() const { ++f->drained; }
+    void leave() const { f->left.fetch_add(1); }
+};
+
+// The copy's error, negative if the device was used wrongly.
+static int copy(Fake& f, CopyTeam* team) {
+    auto ring = std::make_unique<cfdg::RingCopy<Fake::ring, Device>>(Device{&f}, static_cast<int>(f.copied.size()));
+    const int e = ring->run(team, 1 + f.helpers++ % CopyTeam::k_helpers);
+    const std::vector<char> host = f.host;
+    while (f.left.load() == 0) {
+    }
+    return f.strangers != 0 || host != f.host || f.left != 1 || f.drained != (e != 0) ? -1 : e;
 }
 
-static int whole(int n, cfdg::CopyTeam* team) {
+static int whole(int n, CopyTeam* team) {
     Fake f(n);
     int bad = copy(f, team) != 0;
     bad += f.host != f.dev;
     for (int c : f.copied) {
-        bad += c != 1;
+        bad += c != 4; // parts
+    }
+    return bad;
+}
+
+// A helper that is kept from leaving a job (as one whose CPU another thread has taken) keeps no caller.
+struct Held : CopyTeam::Job {
+    std::atomic<int> in{0}, go{0}, out{0};
+};
+
+static int late_helper(CopyTeam& team) {
+    Held h;
+    h.help = [](CopyTeam::Job& j) {
+        auto& s = static_cast<Held&>(j);
+        s.in.fetch_add(1);
+        while (s.go.load() == 0) {
+        }
+    };
+    h.leave = [](CopyTeam::Job& j) { static_cast<Held&>(j).out.fetch_add(1); };
+    team.open(h, CopyTeam::k_helpers);
+    while (h.in.load() < team.helpers()) {
+    }
+    team.close(h);
+    int bad = h.out.load() != (team.helpers() == 0);
+    bad += whole(20, &team); // alone: every helper is in the other job
+    h.go.store(1);
+    while (h.out.load() == 0) {
     }
     return bad;
 }
@@ -80,10 +130,11 @@ static int whole(int n, cfdg::CopyTeam* team) {
 int main(int argc, char** argv) {
     const int starts = argc > 1 ? std::atoi(argv[1]) : 1 << 30;
     allowed = starts;
-    cfdg::CopyTeam* team = &cfdg::CopyTeam::get();
-    int bad = team->helpers() != std::min(starts, static_cast<int>(cfdg::CopyTeam::k_helpers));
+    CopyTeam* team = &CopyTeam::get();
+    const int wanted = CopyTeam::k_helpers;
+    int bad = team->helpers() != std::min(starts, wanted);
     allowed = 1 << 30;
-    for (cfdg::CopyTeam* t : {team, static_cast<cfdg::CopyTeam*>(nullptr)}) {
+    for (CopyTeam* t : {team, static_cast<CopyTeam*>(nullptr)}) {
         for (int n : {0, 1, 7, 8, 9, 16, 100}) {
             for (int rep = 0; rep < 5; ++rep) {
                 bad += whole(n, t);
@@ -97,6 +148,7 @@ int main(int argc, char** argv) {
             bad += copy(a, t) != 22;
         }
     }
+    bad += late_helper(*team);
     std::vector<std::thread> callers;
     std::atomic<int> wrong{0};
     for (int k = 0; k < 6; ++k) {
