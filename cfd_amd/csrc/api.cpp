@@ -54,6 +54,7 @@ extern "C" cfdg_status cfdg_device_available(int* available) {
 extern "C" cfdg_status cfdg_release_cached_memory(size_t* freed_bytes, size_t* reserved_bytes) {
     return guarded([&] {
         const std::size_t f = pool_release_cached();
+        release_staging();
         if (freed_bytes != nullptr) {
             *freed_bytes = f;
         }

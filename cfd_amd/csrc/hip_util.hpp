@@ -41,14 +41,16 @@ void h2d_staged(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 void d2h_staged(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 constexpr std::size_t k_staged_min_bytes = std::size_t(4) << 20;
 
-// Results copied to pageable host arrays, several in one call, through pinned
-// staging from k_pieces_min_bytes in all (staging.cpp; below, the runtime's copy is as fast).
+// Results copied to pageable host arrays, several in one call, through pinned staging from
+// k_pieces_min_bytes in all (staging.cpp; below, the runtime's copy is as fast).
 struct HostCopy {
     const void* dev;
     void* host;
     std::size_t bytes;
 };
 void d2h_copies(const HostCopy* list, int n, hipStream_t s);
+// Frees the pinned staging areas that no copy uses.
+void release_staging() noexcept;
 constexpr std::size_t k_pieces_min_bytes = std::size_t(3) << 20;
 
 // Owning device allocation from the pool; the owner must have no device work pending on it

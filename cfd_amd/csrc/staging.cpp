@@ -1,7 +1,8 @@
 // Large host <-> device copies through pinned staging memory. A copy from or to pageable memory
 // runs at a fraction of the PCIe rate; here the pageable side is copied by the host threads into
 // (or out of) pinned chunks while the DMA engine moves the previous chunk. Staging areas come
-// from a process-wide free list (one per concurrent caller, kept until the process ends).
+// from a process-wide free list: at most k_kept_areas are kept, until cfdg_release_cached_memory, and
+// result copies that would need more go through the runtime.
 //
 // The results of solves and finite-volume calls (d2h_copies) take a finer pipeline, by the caller and, if
 // they are large, helper threads of its own (copy_team.hpp). The set-up's copies keep the OpenMP team that
@@ -95,18 +96,29 @@ struct Area {
 
 thread_local bool t_host_parallel = true;
 
+constexpr int k_kept_areas = 8; // 32 MiB each
+
 std::mutex g_mutex;
 Area* g_free = nullptr;
+int g_areas = 0; // in use or free
+
+// An idle area of the device, or null.
+Area* take_free(int device) {
+    for (Area** at = &g_free; *at != nullptr; at = &(*at)->next) {
+        if ((*at)->device == device) {
+            Area* a = *at;
+            *at = a->next;
+            return a;
+        }
+    }
+    return nullptr;
+}
 
 Area* acquire(int device) {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        for (Area** at = &g_free; *at != nullptr; at = &(*at)->next) {
-            if ((*at)->device == device) {
-                Area* a = *at;
-                *at = a->next;
-                return a;
-            }
+        if (Area* a = take_free(device)) {
+            return a;
         }
     }
     auto a = std::make_unique<Area>();
@@ -119,13 +131,41 @@ Area* acquire(int device) {
     for (hipEvent_t& e : a->slot_done) {
         hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "staging event");
     }
+    std::lock_guard<std::mutex> lock(g_mutex);
+    ++g_areas;
     return a.release();
 }
 
+// As acquire; null where the area would be one too many or cannot be had.
+Area* try_acquire(int device) noexcept {
+    try {
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            if (Area* a = take_free(device)) {
+                return a;
+            }
+            if (g_areas >= k_kept_areas) {
+                return nullptr;
+            }
+        }
+        return acquire(device);
+    } catch (...) { // no pinned memory to be had
+        (void)hipGetLastError();
+        return nullptr;
+    }
+}
+
 void release(Area* a) noexcept {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    a->next = g_free;
-    g_free = a;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if (g_areas <= k_kept_areas) {
+            a->next = g_free;
+            g_free = a;
+            return;
+        }
+        --g_areas;
+    }
+    delete a;
 }
 
 // Host memcpy split over the host threads for large blocks.
@@ -148,6 +188,22 @@ void host_copy(char* dst, const char* src, std::size_t n) {
 bool host_parallel() { return t_host_parallel; }
 
 void set_host_parallel(bool on) { t_host_parallel = on; }
+
+void release_staging() noexcept {
+    for (;;) {
+        Area* a = nullptr;
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            a = g_free;
+            if (a == nullptr) {
+                return;
+            }
+            g_free = a->next;
+            --g_areas;
+        }
+        delete a;
+    }
+}
 
 void parallel_copy(void* dst, const void* src, std::size_t bytes) {
     host_copy(static_cast<char*>(dst), static_cast<const char*>(src), bytes);
@@ -293,7 +349,10 @@ void d2h_copies(const HostCopy* list, int n, hipStream_t s) {
     for (int k = 0; k < n; ++k) {
         total += list[k].bytes;
     }
-    if (total < k_pieces_min_bytes) {
+    int device = 0;
+    hip_check(hipGetDevice(&device), "hipGetDevice");
+    Area* a = total < k_pieces_min_bytes ? nullptr : try_acquire(device);
+    if (a == nullptr) { // small, or the runtime's way
         for (int k = 0; k < n; ++k) {
             if (list[k].bytes > 0) {
                 hip_check(hipMemcpyAsync(list[k].host, list[k].dev, list[k].bytes, hipMemcpyDeviceToHost, s), "D2H copy");
@@ -302,9 +361,6 @@ void d2h_copies(const HostCopy* list, int n, hipStream_t s) {
         hip_check(hipStreamSynchronize(s), "D2H copy sync");
         return;
     }
-    int device = 0;
-    hip_check(hipGetDevice(&device), "hipGetDevice");
-    Area* a = acquire(device);
     const PieceCopy pieces{list, n, piece_bytes(total), a, s};
     Copy* copy = new (a->copy) Copy(pieces, pieces.count());
     const int e = copy->run(t_host_parallel ? &CopyTeam::get() : nullptr, helpers_of(total));

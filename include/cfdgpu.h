@@ -124,7 +124,8 @@ cfdg_status cfdg_last_error(char* buf, size_t len);
 int cfdg_version(void);
 /* No counterpart in the reference. Device buffers come from a pool of large slabs that keeps
  * released memory for reuse; this returns the slabs no buffer uses to the device and reports
- * the bytes freed (may be NULL) and the bytes the pool still holds (may be NULL). */
+ * the bytes freed (may be NULL) and the bytes the pool still holds (may be NULL). The pinned host
+ * memory kept for copies (32 MiB for each of up to 8 callers at once) is freed too, not counted. */
 cfdg_status cfdg_release_cached_memory(size_t* freed_bytes, size_t* reserved_bytes);
 
 /* ------------------------------------------------------------------------------------------

@@ -4,12 +4,14 @@ one thread and from several at once, and together in one call (DeviceSolver.asse
 """
 from __future__ import annotations
 
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
 import cfd_amd
+from cfd_amd import _lib as L
 from cfd_amd import LduPattern, Method, SolveControl, cases
 
 pytestmark = pytest.mark.gpu
@@ -56,6 +58,45 @@ def test_round_trips_from_several_threads():
     for d in devs:
         d.close()
     assert not failed
+
+
+def _mapped_mib():
+    with open("/proc/self/status") as f:
+        return next(int(line.split()[1]) for line in f if line.startswith("VmSize:")) / 1024
+
+
+def test_staging_memory_is_bounded_and_given_back():
+    """More callers at once than staging areas are kept: all results whole, and the areas go with the
+    cached memory (a copy needs 32 MiB of pinned memory; 8 callers' areas are kept)."""
+    devs = [_diagonal(4 * MIB + 11 * k) for k in range(12)]
+    xs = [np.random.default_rng(k).standard_normal(d.n) for k, d in enumerate(devs)]
+    for d, x in zip(devs, xs):
+        d.set_x(x)
+    gate = threading.Barrier(len(devs))
+    same = [False] * len(devs)
+
+    def work(k):
+        ok = True
+        for _ in range(10):
+            gate.wait()
+            ok = np.array_equal(devs[k].get_x(), xs[k]) and ok
+        same[k] = ok
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(devs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(same)
+    before = _mapped_mib()
+    slabs = C.c_size_t()
+    L.call("cfdg_release_cached_memory", C.byref(slabs), None)
+    freed = before - _mapped_mib() - slabs.value / 2 ** 20  # device memory is mapped, too
+    assert 32 <= freed <= 8 * 32 + 16
+    for seed in range(2):  # and anew
+        _round_trip(devs[0], seed)
+    for d in devs:
+        d.close()
 
 
 @pytest.mark.parametrize("shape", [(40, 40, 40), (75, 70, 66)])  # 3.5 and 19 MiB of coefficients
