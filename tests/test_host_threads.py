@@ -41,3 +41,20 @@ def test_load_sets_a_short_block_time():
 def test_process_settings_take_precedence():
     assert _blocktime({"KMP_BLOCKTIME": "50"}) == 50
     assert _blocktime({"OMP_WAIT_POLICY": "PASSIVE"}) == 0
+
+
+UNLOAD = """
+import ctypes, sys
+import _ctypes
+lib = ctypes.CDLL(sys.argv[1])
+_ctypes.dlclose(lib._handle)
+print(sum(sys.argv[1].rsplit("/", 1)[1] in line for line in open("/proc/self/maps")))
+"""
+
+
+@pytest.mark.skipif(not L.LIB_PATH.exists(), reason="library not present")
+def test_library_stays_mapped_when_closed():
+    """Its copy helpers sleep in the library's code for the life of the process."""
+    out = subprocess.run([sys.executable, "-c", UNLOAD, str(L.LIB_PATH)], capture_output=True, text=True, timeout=120,
+                         check=True)
+    assert int(out.stdout.strip().splitlines()[-1]) > 0
