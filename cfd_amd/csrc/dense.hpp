@@ -12,13 +12,11 @@ namespace cfdg {
 // 6 ms), and the largest inverted on the device at all (two launches per 16-row block step).
 constexpr int kDenseMaxOrder = 256;
 constexpr int kDenseWideMaxOrder = 2048;
-// Dense tails of the FP32 cycle up to these orders are taken whatever the finest level's size:
-// kTailOrderKept where the hierarchy is kept for many solves, kTailOrder where it serves one or a few
-// (an inverse of order 560 takes 1.2 ms and saves 0.1 ms a solve). Measured with 512, 768 and 1024:
-// 4420 cells (560 rows on level 1) 482, 375, 369 us a solve, 16-system batch 2528, 2588, 2673, 64-system
-// batch 13.11, 13.18, 13.27 ms (every member reads its own inverse and an extra launch may come in).
+// Dense tails of the FP32 cycle up to this order are taken whatever the finest level's size. With 768 a
+// solve of 4420 cells (560 rows on level 1) takes 375 instead of 482 us, but set_amg 1.1 ms longer, also where
+// it is called for every few solves, and a batch of 16 systems 2588 instead of 2528 us (every member reads
+// its own inverse).
 constexpr int kTailOrder = 512;
-constexpr int kTailOrderKept = 768;
 
 // Inverts the row-major order[i] x order[i] host matrices mats[i] into out[i] on the device
 // (block Gauss-Jordan without pivoting, FP64 MFMA): one workgroup per matrix up to kDenseMaxOrder,

@@ -1116,12 +1116,11 @@ void System::set_amg(const cfdg_amg_view& v, bool fuse_wanted) {
     // Dense tail of the FP32 cycle: a level below the finest that is not the coarsest is solved
     // exactly with its dense inverse (computed on the matrix cores) instead of being smoothed and
     // restricted further: the levels under it are launch-bound, and one dense product replaces
-    // their launches. The first level with at most tail_order rows takes it, or one with at most
+    // their launches. The first level with at most kTailOrder rows takes it, or one with at most
     // kDenseWideMaxOrder rows whose inverse holds at most a tenth as many entries as the finest
     // operator: in a batch the launches are shared by all members while every member reads its
     // own inverse, so the larger tails pay off only against a large finest level (CFDG_DENSE_TAIL=0:
     // off).
-    const int tail_order = fuse_wanted ? kTailOrderKept : kTailOrder;
     int tail = 0;
     const char* tenv = std::getenv("CFDG_DENSE_TAIL");
     if (!(tenv != nullptr && std::string(tenv) == "0")) {
@@ -1131,7 +1130,7 @@ void System::set_amg(const cfdg_amg_view& v, bool fuse_wanted) {
         for (int l = 1; l + 1 < L; ++l) {
             const int nl = rows[static_cast<std::size_t>(l)];
             const long long cells = static_cast<long long>(nl) * nl;
-            if (nl > kDenseWideMaxOrder || (nl > tail_order && 10 * cells > nnz0)) {
+            if (nl > kDenseWideMaxOrder || (nl > kTailOrder && 10 * cells > nnz0)) {
                 continue;
             }
             const cfdg_csr& a = v.levels[l].a;
