@@ -1172,26 +1172,27 @@ __global__ void __launch_bounds__(k_block) k_start(const SysDev* __restrict__ sy
     (void)first_;                                                                                 \
     (void)lane;
 
-// Runs rows(H, slice, ds) over the slices of group g that the wavefront serves: slice and, where the
-// constant H is 2, slice + ds (its slice of the group's next chunk). Rows past the end are included.
-// Pair: two chunks at a time, so that two rows' loads are in flight in each lane (a system of more
-// than one chunk a group has about four wavefronts on a SIMD).
-template <bool Pair, class R>
-__device__ __forceinline__ void group_rows(const SysDev& S, int g, int wave, R rows) {
+// The chunks of a workgroup's groups in the order in which its wavefronts serve them: a group at a time,
+// or, where groups are single chunks and the kernel takes two chunks at a time (Pair: two rows' loads in
+// flight in each lane), two groups at a time. slice: the wavefront's in the first chunk, ds slices before
+// the next one's.
+struct Chunks {
+    int groups; // served together, 1 or 2
+    int count;
+    int slice;
+    int ds;
+};
+
+template <bool Pair>
+__device__ __forceinline__ Chunks chunks_of(const SysDev& S, int g, int end, int wave) {
     const int chunks = S.chunks;
+    if (Pair && chunks == 1 && g + 1 < end) {
+        return {2, 2, g * k_slices_per_block + wave, k_slices_per_block};
+    }
     const int seg = S.segment;
     const int s = g / seg;
     const int ds = min(seg, S.n_groups - s * seg) * k_slices_per_block; // a group's chunks are this far apart
-    int slice = (s * seg * chunks + (g - s * seg)) * k_slices_per_block + wave;
-    int c = 0;
-    if constexpr (Pair) {
-        for (; c + 1 < chunks; c += 2, slice += 2 * ds) {
-            rows(std::integral_constant<int, 2>{}, slice, ds);
-        }
-    }
-    for (; c < chunks; ++c, slice += ds) {
-        rows(std::integral_constant<int, 1>{}, slice, ds);
-    }
+    return {1, chunks, (s * seg * chunks + (g - s * seg)) * k_slices_per_block + wave, ds};
 }
 
 // How a level-0 kernel names a lane's row. Symmetric storage has fewer than 2^29 rows (System builds
@@ -1234,35 +1235,88 @@ __host__ __device__ __forceinline__ void own_rows(int slice, int ds, int lane, i
     }
 }
 
-// Runs rows(H, slice, ds, v) over the workgroup's groups (v[q] += the rows' terms, first row first)
-// and stores the sums of each group in partials slots slot(0) .. slot(N - 1).
+// Runs rows(H, slice, ds, t) over the workgroup's groups: slice and, where the constant H is 2, slice +
+// ds; rows past the end are included. The rows' terms t[h][q] are added, first row first, and the sums of
+// each group go to partials slots slot(0) .. slot(N - 1). The wavefronts meet once, after the last group:
+// with two barriers a group and single chunks one at a time a batch of 256 systems (14 groups a workgroup)
+// took 43.7 ms in mixed and 48.5 in BF16, so 43.5 and 47.4.
 template <int N, bool Pair, class R, class Slot>
 __device__ __forceinline__ void for_groups(const SysDev& S, int first, int gpb, int wave, R rows, Slot slot) {
+    __shared__ double red[k_max_gpb][N][k_slices_per_block];
     const int n = S.n_groups;
     const int end = min(first + gpb, n);
-    for (int g = first; g < end; ++g) {
-        double v[N] = {};
-        group_rows<Pair>(S, g, wave, [&](auto H, int slice, int ds) { rows(H, slice, ds, v); });
-        double o[N];
-        block_sums<N>(v, o);
-        if (threadIdx.x == 0) {
+    for (int g = first; g < end;) {
+        const Chunks ch = chunks_of<Pair>(S, g, end, wave);
+        double v[2][N] = {};
+        int slice = ch.slice;
+        int c = 0;
+        if constexpr (Pair) {
+            for (; c + 1 < ch.count; c += 2, slice += 2 * ch.ds) {
+                double t[2][N] = {};
+                rows(std::integral_constant<int, 2>{}, slice, ch.ds, t);
 #pragma unroll
-            for (int q = 0; q < N; ++q) {
-                S.partials[slot(q) * n + g] = o[q];
+                for (int q = 0; q < N; ++q) {
+                    v[0][q] += t[0][q];
+                    if (ch.groups == 2) {
+                        v[1][q] += t[1][q];
+                    } else {
+                        v[0][q] += t[1][q];
+                    }
+                }
             }
         }
-        if (g + 1 < end) {
-            __syncthreads(); // block_sums' buffer is read by thread 0
+        for (; c < ch.count; ++c, slice += ch.ds) {
+            double t[2][N] = {};
+            rows(std::integral_constant<int, 1>{}, slice, ch.ds, t);
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                v[0][q] += t[0][q];
+            }
         }
+#pragma unroll
+        for (int h = 0; h < (Pair ? 2 : 1); ++h) {
+            if (h < ch.groups) {
+#pragma unroll
+                for (int q = 0; q < N; ++q) {
+                    const double w = wave_sum(v[h][q]);
+                    if (threadIdx.x % k_wave == 0) {
+                        red[g + h - first][q][wave] = w;
+                    }
+                }
+            }
+        }
+        g += ch.groups;
+    }
+    __syncthreads();
+    const int i = static_cast<int>(threadIdx.x) / N; // group and slot of this thread
+    const int q = static_cast<int>(threadIdx.x) % N;
+    if (i < end - first) {
+        double s = red[i][q][0];
+#pragma unroll
+        for (int w = 1; w < k_slices_per_block; ++w) {
+            s += red[i][q][w];
+        }
+        S.partials[slot(q) * n + first + i] = s;
     }
 }
 
-// The same without dot products.
+// The same without dot products: rows(H, slice, ds).
 template <bool Pair, class R>
 __device__ __forceinline__ void for_group_rows(const SysDev& S, int first, int gpb, int wave, R rows) {
     const int end = min(first + gpb, S.n_groups);
-    for (int g = first; g < end; ++g) {
-        group_rows<Pair>(S, g, wave, rows);
+    for (int g = first; g < end;) {
+        const Chunks ch = chunks_of<Pair>(S, g, end, wave);
+        int slice = ch.slice;
+        int c = 0;
+        if constexpr (Pair) {
+            for (; c + 1 < ch.count; c += 2, slice += 2 * ch.ds) {
+                rows(std::integral_constant<int, 2>{}, slice, ch.ds);
+            }
+        }
+        for (; c < ch.count; ++c, slice += ch.ds) {
+            rows(std::integral_constant<int, 1>{}, slice, ch.ds);
+        }
+        g += ch.groups;
     }
 }
 
@@ -1275,7 +1329,7 @@ template <bool Mixed, int Form>
 __global__ void __launch_bounds__(k_block) k_residual0(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
     CFDG_L0_PROLOGUE(sys, blocks)
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
-    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2]) {
+    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][2]) {
         const int row = slice * k_wave + lane;
         double y[2];
         l0_rows<1>(A0, slice, 0, lane, y);
@@ -1288,8 +1342,8 @@ __global__ void __launch_bounds__(k_block) k_residual0(const SysDev* __restrict_
             if (Mixed) {
                 gm(S.r32)[row] = static_cast<float>(ri);
             }
-            v[0] += ri * ri;
-            v[1] += bi * bi;
+            v[0][0] = ri * ri;
+            v[0][1] = bi * bi;
         }
     }, [](int q) { return q == 0 ? SLOT_RR : SLOT_BB; });
 }
@@ -1299,7 +1353,7 @@ template <int Form>
 __global__ void __launch_bounds__(k_block) k_cg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
     CFDG_L0_PROLOGUE(sys, blocks)
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
-    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[3]) {
+    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][3]) {
         const int row = slice * k_wave + lane;
         double y[2];
         l0_rows<1>(A0, slice, 0, lane, y);
@@ -1310,9 +1364,9 @@ __global__ void __launch_bounds__(k_block) k_cg_init(const SysDev* __restrict__ 
             gm(S.r)[row] = ri;
             gm(S.z)[row] = zi;
             gm(S.p)[row] = 0.0;
-            v[0] += ri * ri;
-            v[1] += ri * zi;
-            v[2] += bi * bi;
+            v[0][0] = ri * ri;
+            v[0][1] = ri * zi;
+            v[0][2] = bi * bi;
         }
     }, [](int q) { return q == 0 ? SLOT_RR : q == 1 ? SLOT_RZ : SLOT_BB; });
 }
@@ -1348,7 +1402,7 @@ __global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ 
         return;
     }
     A0.load.beta = st.beta;
-    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2][1]) {
         double y[2];
         double pi[2];
         RowOf<Form> row[2];
@@ -1359,7 +1413,7 @@ __global__ void __launch_bounds__(k_block) k_spmv_pz(const SysDev* __restrict__ 
             if (inside(row[h], n)) {
                 store_at<double>(pn, row[h], pi[h]);
                 store_at<double>(qv, row[h], y[h]);
-                v[0] += pi[h] * y[h];
+                v[h][0] = pi[h] * y[h];
             }
         }
     }, [](int) { return SLOT_PQ; });
@@ -1395,17 +1449,17 @@ __global__ void __launch_bounds__(k_block) k_update_xr(const SysDev* __restrict_
     }
     const double alpha = st.alpha;
     constexpr int n_dots = Mode == 1 ? 2 : 1;
-    for_groups<n_dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[n_dots]) {
+    for_groups<n_dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][n_dots]) {
         const int row = slice * k_wave + lane;
         if (row < n) {
             x[row] = x[row] + alpha * p[row];
             const double ri = r[row] - alpha * qv[row];
             r[row] = ri;
-            v[0] += ri * ri;
+            v[0][0] = ri * ri;
             if constexpr (Mode == 1) {
                 const double zi = ri * dinv[row];
                 z[row] = zi;
-                v[1] += ri * zi;
+                v[0][1] = ri * zi;
             }
             if (Mode == 2) {
                 r32[row] = static_cast<float>(ri);
@@ -1421,7 +1475,7 @@ __global__ void __launch_bounds__(k_block) k_true_residual(const SysDev* __restr
     const auto b = gm(S.b);
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
     const int n = S.n;
-    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2][1]) {
         double y[2];
         double bi[2];
         RowOf<Form> row[2];
@@ -1431,7 +1485,7 @@ __global__ void __launch_bounds__(k_block) k_true_residual(const SysDev* __restr
         for (int h = 0; h < H.value; ++h) {
             if (inside(row[h], n)) {
                 const double ri = bi[h] - y[h];
-                v[0] += ri * ri;
+                v[h][0] = ri * ri;
             }
         }
     }, [](int) { return SLOT_TRUE; });
@@ -1446,7 +1500,7 @@ template <int Form>
 __global__ void __launch_bounds__(k_block) k_bicg_init(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int gpb) {
     CFDG_L0_PROLOGUE(sys, blocks)
     const L0Op<Form, double, GatherX<double>> A0(S.a64, {gm(static_cast<const double*>(S.x))});
-    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[3]) {
+    for_groups<3, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][3]) {
         const int row = slice * k_wave + lane;
         double y[2];
         l0_rows<1>(A0, slice, 0, lane, y);
@@ -1457,9 +1511,9 @@ __global__ void __launch_bounds__(k_block) k_bicg_init(const SysDev* __restrict_
             gm(S.r0)[row] = ri;
             gm(S.p)[row] = 0.0;
             gm(S.v)[row] = 0.0;
-            v[0] += ri * ri;
-            v[1] += ri * ri;
-            v[2] += bi * bi;
+            v[0][0] = ri * ri;
+            v[0][1] = ri * ri;
+            v[0][2] = bi * bi;
         }
     }, [](int q) { return q == 0 ? SLOT_RR : q == 1 ? SLOT_R0R : SLOT_BB; });
 }
@@ -1501,7 +1555,7 @@ __global__ void __launch_bounds__(k_block) k_bicg_v(const SysDev* __restrict__ s
     if (S.st->status != ST_RUNNING) {
         return;
     }
-    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[1]) {
+    for_groups<1, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2][1]) {
         double y[2];
         double ri[2];
         RowOf<Form> row[2];
@@ -1511,7 +1565,7 @@ __global__ void __launch_bounds__(k_block) k_bicg_v(const SysDev* __restrict__ s
         for (int h = 0; h < H.value; ++h) {
             if (inside(row[h], n)) {
                 store_at<double>(vv, row[h], y[h]);
-                v[0] += ri[h] * y[h];
+                v[h][0] = ri[h] * y[h];
             }
         }
     }, [](int) { return SLOT_R0V; });
@@ -1531,13 +1585,13 @@ __global__ void __launch_bounds__(k_block) k_bicg_s(const SysDev* __restrict__ s
         return;
     }
     const double alpha = st.alpha;
-    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[1]) {
+    for_groups<1, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][1]) {
         const int row = slice * k_wave + lane;
         if (row < n) {
             const double si = r[row] - alpha * vv[row];
             sv[row] = si;
             sh[row] = si * dinv[row];
-            v[0] += si * si;
+            v[0][0] = si * si;
         }
     }, [](int) { return SLOT_SS; });
 }
@@ -1565,7 +1619,7 @@ __global__ void __launch_bounds__(k_block) k_bicg_t(const SysDev* __restrict__ s
     if (st.status != ST_RUNNING) {
         return;
     }
-    for_groups<2, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2]) {
+    for_groups<2, true>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2][2]) {
         double y[2];
         double si[2];
         RowOf<Form> row[2];
@@ -1575,8 +1629,8 @@ __global__ void __launch_bounds__(k_block) k_bicg_t(const SysDev* __restrict__ s
         for (int h = 0; h < H.value; ++h) {
             if (inside(row[h], n)) {
                 store_at<double>(tv, row[h], y[h]);
-                v[0] += y[h] * y[h];
-                v[1] += y[h] * si[h];
+                v[h][0] = y[h] * y[h];
+                v[h][1] = y[h] * si[h];
             }
         }
     }, [](int q) { return q == 0 ? SLOT_TT : SLOT_TS; });
@@ -1599,14 +1653,14 @@ __global__ void __launch_bounds__(k_block) k_bicg_xr(const SysDev* __restrict__ 
     }
     const double alpha = st.alpha;
     const double omega = st.omega;
-    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2]) {
+    for_groups<2, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][2]) {
         const int row = slice * k_wave + lane;
         if (row < n) {
             x[row] = x[row] + (alpha * ph[row] + omega * sh[row]);
             const double ri = sv[row] - omega * tv[row];
             r[row] = ri;
-            v[0] += ri * ri;
-            v[1] += r0[row] * ri;
+            v[0][0] = ri * ri;
+            v[0][1] = r0[row] * ri;
         }
     }, [](int q) { return q == 0 ? SLOT_RR : SLOT_R0R; });
 }
@@ -1876,7 +1930,7 @@ __global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict_
     if ((S.st->status != ST_RUNNING) | (L.coarsest != 0)) {
         return;
     }
-    for_groups<Dots, Pair>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[Dots]) {
+    for_groups<Dots, Pair>(S, bk_.y, gpb, wave_, [&](auto H, int slice, int ds, double (&v)[2][Dots]) {
         T y[2];
         T bi[2];
         T wi[2];
@@ -1901,10 +1955,10 @@ __global__ void __launch_bounds__(k_block) k_l0_jacobi(const SysDev* __restrict_
                 store_at<T>(o, row[h], z);
                 const double zd = static_cast<double>(z);
                 if constexpr (Dots == 1) {
-                    v[0] += static_cast<double>(bi[h]) * zd;
+                    v[h][0] = static_cast<double>(bi[h]) * zd;
                 } else {
-                    v[0] += ri[h] * zd;
-                    v[1] += zd * qi[h];
+                    v[h][0] = ri[h] * zd;
+                    v[h][1] = zd * qi[h];
                 }
             }
         }
@@ -1920,15 +1974,15 @@ __global__ void __launch_bounds__(k_block) k_level0_dots(const SysDev* __restric
         return;
     }
     const LevelDev& L = S.lv[0];
-    for_groups<Dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[Dots]) {
+    for_groups<Dots, false>(S, bk_.y, gpb, wave_, [&](auto, int slice, int, double (&v)[2][Dots]) {
         const int row = slice * k_wave + lane;
         if (row < S.n) {
             const double z = static_cast<double>(static_cast<const T*>(L.v[buf])[row]);
             if constexpr (Dots == 1) {
-                v[0] += static_cast<double>(static_cast<const T*>(L.b)[row]) * z;
+                v[0][0] = static_cast<double>(static_cast<const T*>(L.b)[row]) * z;
             } else {
-                v[0] += S.r[row] * z;
-                v[1] += z * S.q[row];
+                v[0][0] = S.r[row] * z;
+                v[0][1] = z * S.q[row];
             }
         }
     }, [](int q) { return q == 0 ? SLOT_RZ : SLOT_ZQ; });

@@ -42,6 +42,8 @@ constexpr unsigned k_report_none = 15; // status of a word that no step has writ
 constexpr int k_states = 4;        // copies of a system's state (kernels.hpp, take_step)
 constexpr int k_max_groups = 1024; // row groups (partial sums per dot product) of a system
 
+constexpr int k_max_gpb = 16;      // row groups of a workgroup
+
 // 256-row chunks of a system's row groups, and the number of groups.
 constexpr int group_chunks(int n) { return ((n + k_block - 1) / k_block + k_max_groups - 1) / k_max_groups; }
 constexpr int group_count(int n) {

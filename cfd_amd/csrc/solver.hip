@@ -1366,7 +1366,7 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
         groups += group_count(x->n());
         tb.sym7 = tb.sym7 && x->symmetric_offsets() == 7;
     }
-    tb.gpb = static_cast<int>(std::min(16LL, std::max(1LL, (groups + 8191) / 8192)));
+    tb.gpb = static_cast<int>(std::min<long long>(k_max_gpb, std::max(1LL, (groups + 8191) / 8192)));
     const std::size_t L = static_cast<std::size_t>(tb.l_max);
     // Host image: ids (two per int2), then the tables; offsets recorded per table.
     std::vector<int2> img((ids.size() + 1) / 2, make_int2(0, 0));

@@ -111,3 +111,50 @@ def test_batch_zero_x_matches_per_member_set_x(prec):
     finally:
         for d in devs:
             d.close()
+
+
+# Rows that leave the last slice and the last chunk incomplete; more than 8192 row groups together, so that a
+# workgroup serves two groups. Groups of one chunk (odd and even numbers of them), of two and of three.
+LARGE = [(61, 59, 57)] * 5 + [(60, 58, 61)] * 5 + [(67, 65, 63), (83, 81, 79), (13, 11, 9)]
+
+
+@pytest.fixture(scope="module")
+def large_members():
+    # A launch takes the fused restriction of a level only if all its systems have it, and they are made up to
+    # a number of rows: without them the arithmetic of a member is the same alone and in any batch.
+    env = pytest.MonkeyPatch()
+    env.setenv("CFDG_FUSED_RESTRICTION", "0")
+    members = []
+    for i, shape in enumerate(LARGE):
+        s = cases.pressure_system(cases.box_mesh(*shape, jitter=0.2, seed=90 + i), rhs_seed=20 + i)
+        pat = cases.csr_pattern(s.n, s.owner, s.neighbour)
+        dev = cfd_amd.DeviceSolver(pat)
+        dev.assemble(s.diag, s.upper, s.lower)
+        a = cases.ldu_to_csr(pat, s.diag, s.upper, s.lower)
+        dev.set_amg(AmgHierarchy(a, AmgSettings(strength_decay=0.5), device=s.n > 40000).view())
+        dev.set_rhs(s.source)
+        members.append((dev, SolveControl(1e-8 * float(np.linalg.norm(s.source)), 25)))
+    env.undo()
+    yield members
+    for dev, _ in members:
+        dev.close()
+
+
+@pytest.mark.parametrize("method,amg,prec", [(Method.Cg, True, Precision.FP64), (Method.Cg, True, Precision.MIXED_FP32),
+                                             (Method.Cg, True, Precision.MIXED_BF16), (Method.Cg, False, Precision.FP64),
+                                             (Method.BiCgStab, False, Precision.FP64)])
+def test_several_groups_a_workgroup_match_members_alone(large_members, method, amg, prec):
+    """A member's iterations, residual and solution do not depend on the launch that it shares, bit for bit."""
+    devs = [d for d, _ in large_members]
+    alone = []
+    for d, c in large_members:
+        d.set_x(None)
+        st = d.solve_resident(method, amg, prec, c)
+        alone.append((st.iterations, st.residual, st.true_residual, d.get_x()))
+    with cfd_amd.Batch(devs, method, amg, prec) as batch:
+        for _ in range(2):  # kernel by kernel, then graphs
+            batch.zero_x()
+            stats = batch.solve([c for _, c in large_members])
+            for d, st, want in zip(devs, stats, alone):
+                assert (st.iterations, st.residual, st.true_residual) == want[:3]
+                assert np.array_equal(d.get_x(), want[3])
