@@ -1,7 +1,7 @@
-"""Level-0 FP32 post-sweep with two slices per wavefront against the one-slice kernel
-(CFDG_NO_PAIR_SWEEPS): mixed FP32 and BF16 solves, alone and in a batch, with the stencil and
-the per-slot column layouts (equal and unequal slice widths), are bit-identical. The members'
-sizes leave a block's last slice pair incomplete or empty.
+"""FP32 level-0 kernels with two rows a lane against one (CFDG_NO_PAIR_SWEEPS): mixed FP32 and BF16
+solves, alone and in a batch, with the stencil and the per-slot column layouts, are bit-identical. The
+prolongation pairs slices at every size (the small members leave a block's last pair incomplete or
+empty); the post-sweep pairs the chunks of a row group, of which there are several above 262,144 rows.
 """
 from __future__ import annotations
 
@@ -114,3 +114,65 @@ def test_pair_prolongation_with_other_transfer_layouts(monkeypatch, lanes, csr):
     finally:
         path = Path(cfd_amd.__file__).resolve().parent / "tuning.json"
         autotune.apply(json.loads(path.read_text()) if path.exists() else {"layout_rules": []})
+
+
+# Two chunks a row group, three, and two with column offsets that need 32 bits; the last slice and the
+# last chunk are incomplete.
+LARGE = [(67, 65, 63), (83, 81, 79), (190, 190, 8)]
+LAYOUTS = {"symmetric": (), "stencil": ("CFDG_NO_SYM",), "explicit": ("CFDG_NO_SYM", "CFDG_NO_STENCIL")}
+
+
+@pytest.fixture(scope="module")
+def large_systems():
+    out = []
+    for i, shape in enumerate(LARGE):
+        s = cases.pressure_system(cases.box_mesh(*shape, jitter=0.2, seed=80 + i), rhs_seed=80 + i)
+        pat = cases.csr_pattern(s.n, s.owner, s.neighbour)
+        a = cases.ldu_to_csr(pat, s.diag, s.upper, s.lower)
+        out.append((s, pat, AmgHierarchy(a, AmgSettings(strength_decay=0.5), device=True).view()))
+    return out
+
+
+def _results(systems, runs):
+    devs = [_build(*t) for t in systems]
+    try:
+        ctls = [SolveControl(1e-8 * np.linalg.norm(t[0].source), 20) for t in systems]
+        out = {}
+        for run in runs:
+            res = []
+            for d, c in zip(devs, ctls):
+                d.set_x(None)
+                st = d.solve_resident(*run, c)
+                res.append((st.iterations, st.residual, st.true_residual, d.get_x()))
+            with cfd_amd.Batch(devs, *run) as batch:
+                batch.zero_x()
+                for d, st in zip(devs, batch.solve(ctls)):
+                    res.append((st.iterations, st.residual, st.true_residual, d.get_x()))
+            out[run] = res
+        return out
+    finally:
+        for d in devs:
+            d.close()
+
+
+def _same(a, b):
+    for run in a:
+        for x, y in zip(a[run], b[run]):
+            assert x[:3] == y[:3] and np.array_equal(x[3], y[3]), run
+
+
+def test_pairs_of_chunks(monkeypatch, large_systems):
+    """Groups of two and three chunks: one row a lane and two give the same bits in every layout, and the
+    layouts of one matrix give the same bits as each other (BF16 rows have one layout)."""
+    cycles = [(Method.Cg, True, Precision.MIXED_FP32), (Method.Cg, True, Precision.MIXED_BF16)]
+    krylov = [(Method.Cg, True, Precision.FP64), (Method.Cg, False, Precision.FP64), (Method.BiCgStab, False, Precision.FP64)]
+    first = None
+    for layout, switches in LAYOUTS.items():
+        with monkeypatch.context() as env:
+            for name in switches:
+                env.setenv(name, "1")
+            here = _results(large_systems, cycles + krylov)
+            env.setenv("CFDG_NO_PAIR_SWEEPS", "1")
+            _same(_results(large_systems, cycles), here)
+        first = first or here
+        _same(here, first)
