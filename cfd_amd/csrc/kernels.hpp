@@ -1910,6 +1910,52 @@ __global__ void __launch_bounds__(k_block) k_l0_presmooth2(const SysDev* __restr
     });
 }
 
+// k_residual and k_jacobi of level 0 for launches whose systems all have the operator in L0_SYM7 form: 256
+// rows a workgroup, the stencil in scalar registers and the row as the only vector address. FP64 at 128^3
+// 24.0 -> 21.4 us and 35.3 -> 34.3 (as row groups 23.5 and 35.2: neither has a step or a dot product to
+// share among a group's rows).
+#define CFDG_SYM7_PROLOGUE(sysarr, blocks, in)                                                    \
+    const int2 bk_ = block_entry(blocks);                                                         \
+    const SysDev& S = (sysarr)[bk_.x];                                                            \
+    const LevelDev& L = S.lv[0];                                                                  \
+    const int wave_ = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / k_wave);     \
+    const int lane = static_cast<int>(threadIdx.x) % k_wave;                                      \
+    const int slice = bk_.y * k_slices_per_block + wave_;                                         \
+    const unsigned row = static_cast<unsigned>(slice * k_wave + lane);                            \
+    const unsigned r = in_matrix(row, L.n);                                                       \
+    const auto x = gm(static_cast<const T*>(L.v[in]));                                            \
+    const T bi = load_at<T>(gm(static_cast<const T*>(L.b)), r);
+
+template <class T>
+__global__ void __launch_bounds__(k_block) k_sym7_residual(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int in, int out) {
+    CFDG_SYM7_PROLOGUE(sys, blocks, in)
+    const L0Op<L0_SYM7, T, GatherX<T>> M(L.a, {x});
+    if ((S.st->status != ST_RUNNING) | (L.coarsest != 0)) {
+        return;
+    }
+    T y[2];
+    l0_rows<1>(M, slice, 0, lane, y);
+    if (inside(row, L.n)) {
+        store_at<T>(gm(static_cast<T*>(L.v[out])), row, bi - y[0]);
+    }
+}
+
+template <class T>
+__global__ void __launch_bounds__(k_block) k_sym7_jacobi(const SysDev* __restrict__ sys, const int2* __restrict__ blocks, int in, int out, T f) {
+    CFDG_SYM7_PROLOGUE(sys, blocks, in)
+    const T wi = load_at<T>(gm(static_cast<const T*>(L.wd)), r);
+    const T xi = load_at<T>(x, r);
+    const L0Op<L0_SYM7, T, GatherX<T>> M(L.a, {x});
+    if ((S.st->status != ST_RUNNING) | (L.coarsest != 0)) {
+        return;
+    }
+    T y[2];
+    l0_rows<1>(M, slice, 0, lane, y);
+    if (inside(row, L.n)) {
+        store_at<T>(gm(static_cast<T*>(L.v[out])), row, xi + (f * wi) * (bi - y[0]));
+    }
+}
+
 // The last post-sweep v[out] = v[in] + (f wd) (b - A v[in]) with the dot products of its result:
 // Dots 1 partial r.z with r = b (FP64 level 0, where b aliases r); 2 partials r.z and z.q with r, q
 // the FP64 outer vectors (mixed level 0). Pair: two chunks' rows at a time (the same results bit

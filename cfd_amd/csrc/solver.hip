@@ -1634,6 +1634,23 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
     if (!step) {
         run_step<FIN_RES>(d, tb, s, report);
     }
+    // Plain sweep and residual of level l.
+    const auto sweep = [&](int l, int in, int out, T f) {
+        const std::size_t li = static_cast<std::size_t>(l);
+        if (l == 0 && sym7) {
+            CFDG_LAUNCH(k_sym7_jacobi<T>, tb.tmn[0][li], s, d, tb.tm[0][li].get(), in, out, f);
+        } else {
+            CFDG_LAUNCH(k_jacobi<T>, tb.tmn[0][li], s, d, tb.tm[0][li].get(), l, in, out, f);
+        }
+    };
+    const auto residual = [&](int l, int in, int out) {
+        const std::size_t li = static_cast<std::size_t>(l);
+        if (l == 0 && sym7) {
+            CFDG_LAUNCH(k_sym7_residual<T>, tb.tmn[0][li], s, d, tb.tm[0][li].get(), in, out);
+        } else {
+            CFDG_LAUNCH(k_residual<T>, tb.tmn[0][li], s, d, tb.tm[0][li].get(), l, in, out);
+        }
+    };
     CFDG_LAUNCH(k_coarse<T>, tb.cn[0], s, d, tb.c[0].get(), 0, fin);
     std::vector<int> cur(static_cast<std::size_t>(L), 0);
     // Where the first sweep from zero of level l is stored as v[x1_slot(l)] = wd b (-1: not
@@ -1685,7 +1702,7 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
                 if (l == 0) {
                     CFDG_LAUNCH(k_jacobi_zero<T>, ga, s, d, ba, l, 0, f1);
                 }
-                CFDG_LAUNCH(k_residual<T>, ga, s, d, ba, l, 0, 1);
+                residual(l, 0, 1);
             }
             CFDG_LAUNCH(k_restrict<T>, tb.tmn[2][li], s, d, tb.tm[2][li].get(), l, 1, x1_next, f1);
             CFDG_LAUNCH(k_coarse<T>, tb.cn[li + 1], s, d, tb.c[li + 1].get(), l + 1, fin);
@@ -1702,23 +1719,21 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
                 if (l == 0) {
                     CFDG_LAUNCH(k_jacobi_zero<T>, ga, s, d, ba, l, 2, f1);
                 }
-                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, 2, 0, f2);
+                sweep(l, 2, 0, f2);
             }
             for (int k = 2; k < sweeps; ++k) {
                 const int o = c == 0 ? 2 : 0;
-                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, c, o, static_cast<T>(sf.pre[k]));
+                sweep(l, c, o, static_cast<T>(sf.pre[k]));
                 c = o;
             }
         }
         cur[li] = c;
-        CFDG_LAUNCH(k_residual<T>, ga, s, d, ba, l, c, 1);
+        residual(l, c, 1);
         CFDG_LAUNCH(k_restrict<T>, tb.tmn[2][li], s, d, tb.tm[2][li].get(), l, 1, x1_next, f1);
         CFDG_LAUNCH(k_coarse<T>, tb.cn[li + 1], s, d, tb.c[li + 1].get(), l + 1, fin);
     }
     for (int l = L - 2; l >= 0; --l) {
         const std::size_t li = static_cast<std::size_t>(l);
-        const int ga = tb.tmn[0][li];
-        const int2* ba = tb.tm[0][li].get();
         const int c0 = cur[li];
         if (sweeps == 1) {
             CFDG_LAUNCH_EITHER(pair && l == 0, (k_prolong_pair<T, true>), (k_prolong<T, true>), tb.tmn[1][li], s, d,
@@ -1745,7 +1760,7 @@ void enqueue_vcycle(const SysDev* d, const Tables& tb, int sweeps, hipStream_t s
                 }
                 probe_end(PROBE_L0_SWEEP, s);
             } else {
-                CFDG_LAUNCH(k_jacobi<T>, ga, s, d, ba, l, c, o, fk);
+                sweep(l, c, o, fk);
             }
             c = o;
         }
