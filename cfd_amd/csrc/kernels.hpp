@@ -1155,7 +1155,7 @@ __global__ void __launch_bounds__(k_block) k_start(const SysDev* __restrict__ sy
 // that a step adds at most k_max_groups partials whatever the system's size (one chunk up to
 // 262,144 rows, 8 at 128^3); the grouping depends on the system's size only, so its sums do not
 // depend on which systems share the launch. gpb > 1 in large batches keeps the number of
-// workgroups, each of which makes the step, near 8192.
+// workgroups, each of which makes the step, near 16384.
 //
 // A group's chunks are not neighbours: the groups fall into k_xcds segments (one XCD's workgroups of
 // a single system), a segment owns a contiguous range of chunks, and its groups take the chunks of
@@ -1238,8 +1238,8 @@ __host__ __device__ __forceinline__ void own_rows(int slice, int ds, int lane, i
 // Runs rows(H, slice, ds, t) over the workgroup's groups: slice and, where the constant H is 2, slice +
 // ds; rows past the end are included. The rows' terms t[h][q] are added, first row first, and the sums of
 // each group go to partials slots slot(0) .. slot(N - 1). The wavefronts meet once, after the last group:
-// with two barriers a group and single chunks one at a time a batch of 256 systems (14 groups a workgroup)
-// took 43.7 ms in mixed and 48.5 in BF16, so 43.5 and 47.4.
+// with two barriers a group and single chunks one at a time a batch of 256 systems at 14 groups a
+// workgroup took 43.7 ms in mixed and 48.5 in BF16, so 43.5 and 47.4.
 template <int N, bool Pair, class R, class Slot>
 __device__ __forceinline__ void for_groups(const SysDev& S, int first, int gpb, int wave, R rows, Slot slot) {
     __shared__ double red[k_max_gpb][N][k_slices_per_block];

@@ -1355,18 +1355,18 @@ void build_tables(Tables& tb, const std::vector<System*>& sys, bool use_amg, boo
             tb.l_max = std::max(tb.l_max, x->n_levels(fp32));
         }
     }
-    // Row groups per workgroup: one up to 8192 groups in all, so that a single system's few groups
-    // spread over the chip; above, the workgroups of a large batch stay near 8192, each making its
-    // kernel's step once for several groups. The line at 2048: 16 systems of 4 k to 300 k cells 2.53
-    // instead of 2.60 ms, 64 of 4 k to 500 k (8.0 M cells) 13.86 instead of 13.13 ms; at 4096: 2.58 and
-    // 13.39 ms; at 16384 both as here.
+    // Row groups per workgroup: one up to 16384 groups in all, so that a single system's few groups
+    // spread over the chip; above, the workgroups of a large batch stay near 16384, each making its
+    // kernel's step once for several groups. 256 systems of 4 k to 500 k cells (114 k groups), line at
+    // 4096 / 8192 / 16384 / 32768: FP64 89.9, 88.9, 88.1, 87.9 ms, mixed 44.1, 43.5, 42.8, 42.5, BF16 48.4,
+    // 47.4, 46.9, 47.0; 64 systems (8.0 M cells) at 8192 / 16384 / 32768: mixed 13.05, 13.02, 13.58.
     long long groups = 0;
     tb.sym7 = true;
     for (System* x : sys) {
         groups += group_count(x->n());
         tb.sym7 = tb.sym7 && x->symmetric_offsets() == 7;
     }
-    tb.gpb = static_cast<int>(std::min<long long>(k_max_gpb, std::max(1LL, (groups + 8191) / 8192)));
+    tb.gpb = static_cast<int>(std::min<long long>(k_max_gpb, std::max(1LL, (groups + 16383) / 16384)));
     const std::size_t L = static_cast<std::size_t>(tb.l_max);
     // Host image: ids (two per int2), then the tables; offsets recorded per table.
     std::vector<int2> img((ids.size() + 1) / 2, make_int2(0, 0));

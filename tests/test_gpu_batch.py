@@ -113,9 +113,9 @@ def test_batch_zero_x_matches_per_member_set_x(prec):
             d.close()
 
 
-# Rows that leave the last slice and the last chunk incomplete; more than 8192 row groups together, so that a
+# Rows that leave the last slice and the last chunk incomplete; more than 16384 row groups together, so that a
 # workgroup serves two groups. Groups of one chunk (odd and even numbers of them), of two and of three.
-LARGE = [(61, 59, 57)] * 5 + [(60, 58, 61)] * 5 + [(67, 65, 63), (83, 81, 79), (13, 11, 9)]
+LARGE = [(61, 59, 57)] * 10 + [(60, 58, 61)] * 10 + [(67, 65, 63), (83, 81, 79), (13, 11, 9)]
 
 
 @pytest.fixture(scope="module")
