@@ -172,7 +172,7 @@ constexpr int ell_group() {
 }
 
 // Storage-order row sum of sliced-ELL slots with values val (type V) converted to T. Loads are
-// issued ell_group entries at a time, the tail (w mod k_ell_group, uniform over the slice's
+// issued ell_group entries at a time, the tail (w mod ell_group, uniform over the slice's
 // wavefront) as one more group with its unused loads repeating a valid slot; only real entries
 // are summed.
 template <class T, class V, class C, class F>

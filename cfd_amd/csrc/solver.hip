@@ -3,8 +3,8 @@
 // Reference counterparts: DeviceSolver (src/gpu/src/device_solver.cpp), the CUDA system
 // (src/gpu/src/krylov_cuda.cu:566-677) and the solver loops of
 // src/gpu/src/krylov_kernels.inc. The host here only enqueues kernels; every scalar of the
-// Krylov recurrences lives on the device, and the host reads back one integer per iteration
-// (the number of systems still running) one iteration behind the launches.
+// Krylov recurrences lives on the device, and the host polls one report word a system (status,
+// finished iterations, residual) while the iterations that it expects to need are queued.
 #include "solver.hpp"
 #include "fv.hpp"
 #include "kernels.hpp"
@@ -1926,11 +1926,11 @@ private:
 
 // Everything a set of systems needs to be solved together, built once and reused: launch
 // tables, device descriptors, and (unless kernels are being probed) HIP graphs of the solver's
-// start-up sequence and of one, two and four iterations. Every iteration ends by writing each
-// system's report word into pinned host memory; the host polls the words and queues, one
-// iteration ahead of them, as many iterations as the residuals let it expect (Forecast): a graph
-// launch costs 8 us beyond its kernels, and an iteration queued past the end of the solve all its
-// launches.
+// start-up sequence and of one, two and four iterations. Every residual test, which is part of the
+// next iteration's first kernel or a launch of its own at the end of a graph, writes the system's
+// report word into pinned host memory; the host polls the words and queues, one iteration ahead of
+// them, as many iterations as the residuals let it expect (Forecast): a graph launch costs 8 us
+// beyond its kernels, and an iteration queued past the end of the solve all its launches.
 class Runner {
 public:
     Runner(const std::vector<System*>& systems, const BatchOptions& opt, hipStream_t s)
@@ -2104,12 +2104,11 @@ public:
             o.solve_ms = ms;
         }
         if (probe != nullptr) {
-            // Launches that did work: the initial V-cycle plus one per iteration that
-            // preconditioned (level-0 sweep), or one per iteration (outer SpMV).
-            const int its = stats[0].iterations;
-            std::size_t useful = static_cast<std::size_t>(its);
-            if (probe->kind == PROBE_L0_SWEEP && stats[0].exit_reason != ST_CONVERGED) {
-                useful = static_cast<std::size_t>(its) + 1;
+            // Launches that did work: one an iteration, and the cycle after which the iteration
+            // limit was found exceeded.
+            std::size_t useful = static_cast<std::size_t>(stats[0].iterations);
+            if (probe->kind == PROBE_L0_SWEEP && stats[0].exit_reason == ST_MAXIT) {
+                ++useful;
             }
             useful = std::min(useful, probe->used);
             for (std::size_t i = 0; i < useful; ++i) {
