@@ -44,10 +44,9 @@ __attribute__((constructor)) void short_omp_blocktime() {
 
 constexpr std::size_t k_chunk = std::size_t(16) << 20; // bytes per chunk; two chunks per area
 
-
-// Helper threads of d2h_copies: one, with which the caller keeps up with the link (16 MiB 0.48 ms, 0.52
-// alone, with three 0.49, through the runtime 0.95); from k_large_copy on, where malloc hands out fresh pages each time and
-// the copy waits for their zeroing, all of them (32 MiB 1.05 ms, with one 1.8, alone 2.0).
+// Helper threads of d2h_copies: one, with which the caller keeps up with the link (16 MiB 0.48 ms, alone
+// 0.52, with three 0.49, through the runtime 0.95); from k_large_copy on, where malloc hands out fresh pages
+// each time and the copy waits for their zeroing, all of them (32 MiB 1.05 ms, with one 1.8, alone 2.0).
 constexpr std::size_t k_large_copy = std::size_t(24) << 20;
 constexpr int helpers_of(std::size_t total) { return total >= k_large_copy ? CopyTeam::k_helpers : 1; }
 
