@@ -1893,19 +1893,14 @@ public:
     void reset(double tol) {
         tol_ = tol;
         res_.clear();
-        last_ = estimate();
     }
     void add(const Report& r) {
         if (!r.none() && r.done >= static_cast<int>(res_.size())) {
             res_.resize(static_cast<std::size_t>(r.done) + 1, r.res); // iterations the poll missed take this one's
-            last_ = estimate();
         }
     }
     // Number of the iteration at which the residual is expected to reach the tolerance.
-    [[nodiscard]] int last() const { return last_; }
-
-private:
-    [[nodiscard]] int estimate() const {
+    [[nodiscard]] int last() const {
         const int k = static_cast<int>(res_.size()) - 1;
         if (k < 1) {
             return k + k_unknown;
@@ -1920,10 +1915,10 @@ private:
         return k + static_cast<int>(std::min(1000.0, std::max(1.0, std::floor(need / rate + 0.7))));
     }
 
+private:
     static constexpr int k_span = 3;
     static constexpr int k_unknown = 4;
     double tol_ = 0.0;
-    int last_ = 0;
     std::vector<float> res_;
 };
 
